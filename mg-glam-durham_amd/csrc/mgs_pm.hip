@@ -8,14 +8,14 @@
 //
 // Deposit into the solver's level-0 density (colour-split FP64, the array
 // mgs_set_density fills), so a solve can follow without a host trip.  The
-// particles are binned by the 16^3-cell tile of their CIC base cell, in runs
-// of consecutive particles of one tile (a counting sort of the runs: per-tile
-// counts whose atomics also rank the runs, an exclusive scan, a scatter of
-// (first particle, length) into tile order); one workgroup per tile then
-// accumulates its particles' 8 weights in a 17^3 fixed-point buffer in LDS
-// and adds each touched cell to the grid once, instead of eight global
-// atomics per particle.  Integer accumulation makes the sum independent of
-// the order of the additions (the reference adds into REAL*4 FI).
+// particles are binned by the 32 x 16 x 8-cell tile of their CIC base cell and
+// by the tile faces their +1 nodes cross, in runs of consecutive particles of
+// one bin (a counting sort: counts gathered per block in LDS, an exclusive
+// scan, a scatter of the particles' indices into bin order); one
+// workgroup per tile then accumulates every weight that falls into its cells
+// in a fixed-point buffer in LDS and writes each cell's density once.  Integer
+// accumulation makes the sum independent of the order of the additions (the
+// reference adds into REAL*4 FI).
 //
 // Move: one thread per particle gathers the 32 potential values of its 2x2x2
 // node block and their outer neighbours (PMP2main.f90:496-558), forms the
@@ -40,19 +40,20 @@ namespace mgs {
 
 struct PmState {
     int64_t np = 0;
-    float* buf = nullptr;  // x, y, z, vx, vy, vz: 6 * np floats
+    int64_t ld = 0;        // floats from one array to the next: np rounded up to 64, so each starts 256-byte aligned
+    float* buf = nullptr;  // x, y, z, vx, vy, vz: 6 * ld floats
     float* phi = nullptr;  // N^3 potential, x fastest, REAL*4 like the reference's FI
     double* part = nullptr;
     int* bad = nullptr;    // particles outside [1, N+1) seen by the last kernel
     int npart_blocks = 0;
-    // deposit binning (runs of particles, see k_bin_count): per particle its
-    // key and rank, the run descriptors in tile order; per tile its count of
-    // runs and first run
+    // deposit binning (runs of particles, see k_bin_count): the run records
+    // and their number per wave, the particles in bin order; per bin its count
+    // and first particle
     int64_t nbin = 0;
-    int* key = nullptr;
-    int* rank = nullptr;
-    int64_t* runs = nullptr;  // nbin (at most one run per particle)
-    int ntiles = 0;
+    unsigned long long* recs = nullptr;
+    int* nrec = nullptr;
+    unsigned* order = nullptr;  // nbin particle indices
+    int nbins = 0;
     int* count = nullptr;
     int64_t* first = nullptr;
     void* scan_tmp = nullptr;
@@ -78,7 +79,7 @@ void pm_release(mgs_handle* h)
     if (p->phi) (void)hipFree(p->phi);
     if (p->part) (void)hipFree(p->part);
     if (p->bad) (void)hipFree(p->bad);
-    for (void* q : {(void*)p->key, (void*)p->rank, (void*)p->runs, (void*)p->count, (void*)p->first, p->scan_tmp})
+    for (void* q : {(void*)p->recs, (void*)p->nrec, (void*)p->order, (void*)p->count, (void*)p->first, p->scan_tmp})
         if (q) (void)hipFree(q);
     delete p;
     h->pm = nullptr;
@@ -101,137 +102,202 @@ float* pm_potential(mgs_handle* h)
     return p->phi;
 }
 
-// INT(X) of the reference for X in [1, N+1): the 1-based cell; -1 outside
-__device__ __forceinline__ int cell_of(double X, int N)
+// INT(X) of the reference for X in [1, N+1): the 1-based cell; -1 outside (or
+// NaN).  N + 1 <= 1025 is exact in REAL*4.
+__device__ __forceinline__ int cell_of(float X, int N)
 {
-    if (!(X >= 1.0 && X < (double)N + 1.0)) return -1;
+    if (!(X >= 1.0f && X < (float)(N + 1))) return -1;
     return (int)X;
 }
 
 // DENSIT's CIC loop, PMP2mod_density.f90:235-281 (0-based cells here), over
-// the particles binned by tile.
-constexpr int PM_TILE = 16;                                            // cells per tile side
-constexpr int PM_TBUF = PM_TILE + 1;                                   // with the +1 CIC reach
-constexpr int PM_TCELLS = PM_TBUF * PM_TBUF * PM_TBUF;                 // 4913 (38.4 KiB of LDS)
+// the particles binned by tile.  A tile is 32 x 16 x 8 cells: long in x, so
+// that consecutive particles of a lattice-ordered array stay in one tile and
+// a tile's rows are whole 128-byte lines of each colour half.
+constexpr int PM_TX = 32, PM_TY = 16, PM_TZ = 8;
+constexpr int PM_LX = PM_TX + 1;                  // LDS row stride: rows start in different banks
+constexpr int PM_TCELLS = PM_LX * PM_TY * PM_TZ;  // 4224 (33 KiB of LDS)
 
-// tile of 0-based base cell (i0, j0, k0); TT tiles per side
-__device__ __forceinline__ int tile_of(int i0, int j0, int k0, int TT)
+// tiles per side
+struct PmTiles {
+    int x, y, z;
+};
+
+static PmTiles pm_tiles(int N)
 {
-    return ((k0 / PM_TILE) * TT + j0 / PM_TILE) * TT + i0 / PM_TILE;
+    return PmTiles{(N + PM_TX - 1) / PM_TX, (N + PM_TY - 1) / PM_TY, (N + PM_TZ - 1) / PM_TZ};
+}
+
+// Bin of a particle with 0-based base cell (i0, j0, k0): 8 bins per tile, by
+// whether the particle's +1 nodes lie beyond the tile in x (1), y (2), z (4).
+__device__ __forceinline__ int bin_of(int i0, int j0, int k0, int N, const PmTiles& T)
+{
+    const int t = ((k0 / PM_TZ) * T.y + j0 / PM_TY) * T.x + i0 / PM_TX;
+    const int fx = (i0 % PM_TX == PM_TX - 1 || i0 == N - 1) ? 1 : 0;
+    const int fy = (j0 % PM_TY == PM_TY - 1 || j0 == N - 1) ? 2 : 0;
+    const int fz = (k0 % PM_TZ == PM_TZ - 1 || k0 == N - 1) ? 4 : 0;
+    return t * 8 + (fx | fy | fz);
 }
 
 // The binning passes take PM_RUN consecutive particles per thread (particles
 // in array order are usually neighbours in space, so consecutive ones usually
-// share a tile) and bin *runs*: maximal sequences of a thread's particles in
-// one tile, described by (first particle, length).
+// share a bin) and bin *runs*: maximal sequences of a thread's particles in
+// one bin, described by (first particle, length).
 constexpr int PM_RUN = 8;
-constexpr int KEY_OUTSIDE = -1;  // particle outside [1, N+1)
-constexpr int KEY_CONT = -2;     // particle continuing the run before it
+constexpr int PM_WCHUNK = 64 * PM_RUN;  // particles of one wave, whose run records are stored together
+constexpr int KEY_OUTSIDE = -1;         // particle outside [1, N+1)
 
-// per run: its tile (in key[] at the run's first particle; the others KEY_CONT)
-// and its rank among the runs of that tile (in rank[] there); per tile: the
-// count of runs
+// A run's record between the two binning passes: its rank (the particles of
+// the bin before it), the bin (21 bits: 2^21 bins at N = 1024), the first
+// particle's place in the wave's 512 and the length - 1.
+__device__ __forceinline__ unsigned long long run_record(unsigned rank, int bin, int local, int len)
+{
+    return (unsigned long long)rank << 33 | (unsigned long long)(unsigned)bin << 12 | (unsigned)local << 3 |
+           (unsigned)(len - 1);
+}
+
+// per run: its record; per bin: the count of particles.  A block first counts
+// its particles per bin in an LDS hash table (a lattice-ordered block of 2048
+// meets some tens of bins), then adds each bin's count to the global counter
+// once; the global counter's old value plus the run's rank in the block is
+// its rank.  Before, one returning global atomic per run bound this pass:
+// 2.13 ms for 512^3 particles in lattice order, now 0.49 ms (1.6 GB of
+// positions read, 0.4 GB of records written).  A run whose bin finds no slot
+// within PM_PROBES (blocks of unordered particles) takes the global atomic
+// itself.
+constexpr int PM_SLOTS = 1024, PM_PROBES = 8;
+
 __global__ __launch_bounds__(PM_BLOCK) void k_bin_count(const float* __restrict__ xs, const float* __restrict__ ys,
-                                                        const float* __restrict__ zs, int64_t np, int N, int TT,
-                                                        int* __restrict__ key, int* __restrict__ rank,
+                                                        const float* __restrict__ zs, int64_t np, int N, PmTiles T,
+                                                        unsigned long long* __restrict__ recs, int* __restrict__ nrec,
                                                         int* __restrict__ count, int* __restrict__ bad)
 {
-    const int64_t nchunk = (np + PM_RUN - 1) / PM_RUN;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t ch = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; ch < nchunk; ch += stride) {
-        const int64_t p0 = ch * PM_RUN;
-        // a whole chunk with 16-byte aligned rows: two 16-byte loads per array
-        const bool vec = (np & 3) == 0 && p0 + PM_RUN <= np;
-        float x[PM_RUN], y[PM_RUN], z[PM_RUN];
-        if (vec) {
+    __shared__ int keys[PM_SLOTS];
+    __shared__ int cnt[PM_SLOTS];
+    for (int i = threadIdx.x; i < PM_SLOTS; i += PM_BLOCK) {
+        keys[i] = -1;
+        cnt[i] = 0;
+    }
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = (int64_t)blockIdx.x * (PM_BLOCK / 64) + (threadIdx.x >> 6);
+    const int64_t p0 = wave * PM_WCHUNK + lane * PM_RUN;
+    float x[PM_RUN], y[PM_RUN], z[PM_RUN];
+    if (p0 + PM_RUN <= np) {  // the arrays start 256-byte aligned: 16-byte loads
 #pragma unroll
-            for (int v = 0; v < PM_RUN / 4; v++) {
-                const float4 a = ((const float4*)(xs + p0))[v], b = ((const float4*)(ys + p0))[v],
-                             c = ((const float4*)(zs + p0))[v];
-                x[4 * v] = a.x, x[4 * v + 1] = a.y, x[4 * v + 2] = a.z, x[4 * v + 3] = a.w;
-                y[4 * v] = b.x, y[4 * v + 1] = b.y, y[4 * v + 2] = b.z, y[4 * v + 3] = b.w;
-                z[4 * v] = c.x, z[4 * v + 1] = c.y, z[4 * v + 2] = c.z, z[4 * v + 3] = c.w;
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < PM_RUN; r++) {
-                const int64_t p = p0 + r < np ? p0 + r : np - 1;
-                x[r] = xs[p];
-                y[r] = ys[p];
-                z[r] = zs[p];
-            }
+        for (int v = 0; v < PM_RUN / 4; v++) {
+            const float4 a = ((const float4*)(xs + p0))[v], b = ((const float4*)(ys + p0))[v],
+                         c = ((const float4*)(zs + p0))[v];
+            x[4 * v] = a.x, x[4 * v + 1] = a.y, x[4 * v + 2] = a.z, x[4 * v + 3] = a.w;
+            y[4 * v] = b.x, y[4 * v + 1] = b.y, y[4 * v + 2] = b.z, y[4 * v + 3] = b.w;
+            z[4 * v] = c.x, z[4 * v + 1] = c.y, z[4 * v + 2] = c.z, z[4 * v + 3] = c.w;
         }
-        int t[PM_RUN];
+    } else {
 #pragma unroll
         for (int r = 0; r < PM_RUN; r++) {
-            t[r] = KEY_OUTSIDE;
-            if (p0 + r < np) {
-                const int I = cell_of(x[r], N), J = cell_of(y[r], N), K = cell_of(z[r], N);
-                if (I < 0 || J < 0 || K < 0)
-                    atomicAdd(bad, 1);
-                else
-                    t[r] = tile_of(I - 1, J - 1, K - 1, TT);
+            const int64_t p = p0 + r < np ? p0 + r : np - 1;
+            x[r] = xs[p];
+            y[r] = ys[p];
+            z[r] = zs[p];
+        }
+    }
+    int t[PM_RUN];
+    int nbad = 0;
+#pragma unroll
+    for (int r = 0; r < PM_RUN; r++) {
+        t[r] = KEY_OUTSIDE;
+        if (p0 + r < np) {
+            const int I = cell_of(x[r], N), J = cell_of(y[r], N), K = cell_of(z[r], N);
+            if (I < 0 || J < 0 || K < 0)
+                nbad++;
+            else
+                t[r] = bin_of(I - 1, J - 1, K - 1, N, T);
+        }
+    }
+    if (nbad) atomicAdd(bad, nbad);
+    __syncthreads();  // the table is clear
+    // the run starting at particle r: its length, its slot (-1: none) and its
+    // rank in the block's count of the slot, or its global rank without a slot
+    int slot[PM_RUN], rk[PM_RUN], len[PM_RUN], ns = 0;
+#pragma unroll
+    for (int r = 0; r < PM_RUN; r++) {
+        slot[r] = -1;
+        rk[r] = 0;
+        len[r] = 0;
+        const bool start = t[r] >= 0 && (r == 0 || t[r] != t[r - 1]);
+        if (!start) continue;
+        ns++;
+        len[r] = 1;
+        bool same = true;
+#pragma unroll
+        for (int q = r + 1; q < PM_RUN; q++) {
+            same = same && t[q] == t[r];
+            len[r] += same ? 1 : 0;
+        }
+        unsigned s = ((unsigned)t[r] * 2654435761u) >> 22;
+        for (int q = 0; q < PM_PROBES; q++) {
+            int k = *(volatile int*)&keys[s];
+            if (k == -1) k = atomicCAS(&keys[s], -1, t[r]);
+            if (k == -1 || k == t[r]) {
+                slot[r] = (int)s;
+                break;
             }
+            s = (s + 1) & (PM_SLOTS - 1);
         }
-        int k[PM_RUN], rk[PM_RUN];
+        rk[r] = slot[r] >= 0 ? atomicAdd(&cnt[slot[r]], len[r]) : atomicAdd(&count[t[r]], len[r]);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < PM_SLOTS; i += PM_BLOCK)
+        if (keys[i] >= 0) cnt[i] = atomicAdd(&count[keys[i]], cnt[i]);
+    // the wave's records, one after the other
+    int pre = ns;
 #pragma unroll
-        for (int r = 0; r < PM_RUN; r++) {
-            const bool start = t[r] >= 0 && (r == 0 || t[r] != t[r - 1]);
-            k[r] = start || t[r] < 0 ? t[r] : KEY_CONT;
-            rk[r] = 0;
-            if (start) rk[r] = atomicAdd(&count[t[r]], 1);
-        }
-        if (p0 + PM_RUN <= np) {  // key + p0 is 32-byte aligned (p0 a multiple of 8)
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(pre, off, 64);
+        if (lane >= off) pre += v;
+    }
+    if (lane == 63 && wave * PM_WCHUNK < np) nrec[wave] = pre;
+    __syncthreads();
+    unsigned long long* out = recs + wave * PM_WCHUNK + (pre - ns);
 #pragma unroll
-            for (int v = 0; v < PM_RUN / 4; v++) {
-                ((int4*)(key + p0))[v] = make_int4(k[4 * v], k[4 * v + 1], k[4 * v + 2], k[4 * v + 3]);
-                ((int4*)(rank + p0))[v] = make_int4(rk[4 * v], rk[4 * v + 1], rk[4 * v + 2], rk[4 * v + 3]);
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < PM_RUN; r++)
-                if (p0 + r < np) {
-                    key[p0 + r] = k[r];
-                    rank[p0 + r] = rk[r];
-                }
-        }
+    for (int r = 0; r < PM_RUN; r++) {
+        if (!len[r]) continue;
+        const unsigned rank = (unsigned)(slot[r] >= 0 ? cnt[slot[r]] + rk[r] : rk[r]);
+        *out++ = run_record(rank, t[r], lane * PM_RUN + r, len[r]);
     }
 }
 
-// run descriptors into tile order: (first particle) * PM_RUN + (length - 1)
-__global__ __launch_bounds__(PM_BLOCK) void k_bin_scatter(int64_t np, const int* __restrict__ key,
-                                                          const int* __restrict__ rank,
+// 2 and 4 words stored (loaded) at 4-byte alignment by one instruction
+struct __attribute__((packed, aligned(4))) Words2 {
+    unsigned v[2];
+};
+struct __attribute__((packed, aligned(4))) Words4 {
+    unsigned v[4];
+};
+
+// the particles' indices in bin order (the deposit takes fewer than 2^31
+// particles); one wave per PM_WCHUNK particles.  Bound by the number of
+// scattered stores: a run's words go out in stores of 4, 2 and 1 (512^3
+// particles of a clustered lattice: 0.52 ms, 0.68 with one store per word)
+__global__ __launch_bounds__(PM_BLOCK) void k_bin_scatter(int64_t nwaves, const unsigned long long* __restrict__ recs,
+                                                          const int* __restrict__ nrec,
                                                           const int64_t* __restrict__ first,
-                                                          int64_t* __restrict__ runs)
+                                                          unsigned* __restrict__ order)
 {
-    const int64_t nchunk = (np + PM_RUN - 1) / PM_RUN;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t ch = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; ch < nchunk; ch += stride) {
-        const int64_t p0 = ch * PM_RUN;
-        int k[PM_RUN];
-        if (p0 + PM_RUN <= np) {
-#pragma unroll
-            for (int v = 0; v < PM_RUN / 4; v++) {
-                const int4 a = ((const int4*)(key + p0))[v];
-                k[4 * v] = a.x, k[4 * v + 1] = a.y, k[4 * v + 2] = a.z, k[4 * v + 3] = a.w;
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < PM_RUN; r++) k[r] = p0 + r < np ? key[p0 + r] : KEY_OUTSIDE;
+    const int64_t wave = (int64_t)blockIdx.x * (PM_BLOCK / 64) + (threadIdx.x >> 6);
+    if (wave >= nwaves) return;
+    const int n = nrec[wave];
+    for (int i = threadIdx.x & 63; i < n; i += 64) {
+        const unsigned long long r = recs[wave * PM_WCHUNK + i];
+        unsigned* o = order + first[(unsigned)(r >> 12) & 0x1fffffu] + (int64_t)(r >> 33);
+        const unsigned p = (unsigned)(wave * PM_WCHUNK) + ((unsigned)(r >> 3) & 511u);
+        const unsigned len = ((unsigned)r & 7u) + 1u;
+        unsigned u = 0;
+        for (; u + 4 <= len; u += 4) *(Words4*)(o + u) = Words4{{p + u, p + u + 1, p + u + 2, p + u + 3}};
+        if (len & 2) {
+            *(Words2*)(o + u) = Words2{{p + u, p + u + 1}};
+            u += 2;
         }
-#pragma unroll
-        for (int r = 0; r < PM_RUN; r++) {
-            if (k[r] < 0) continue;
-            int len = 1;
-#pragma unroll
-            for (int q = r + 1; q < PM_RUN; q++) {
-                bool cont = true;
-#pragma unroll
-                for (int u = r + 1; u <= q; u++) cont = cont && k[u] == KEY_CONT;
-                len += cont ? 1 : 0;
-            }
-            runs[first[k[r]] + rank[p0 + r]] = (p0 + r) * PM_RUN + (len - 1);
-        }
+        if (len & 1) o[u] = p + u;
     }
 }
 
@@ -246,89 +312,156 @@ __global__ __launch_bounds__(PM_BLOCK) void k_bin_scatter(int64_t np, const int*
 constexpr double PM_FIX = 1099511627776.0;          // 2^40
 constexpr double PM_UNFIX = 1.0 / 1099511627776.0;  // 2^-40
 
-__device__ __forceinline__ unsigned long long pm_fix(double v) { return __double2ull_rn(v * PM_FIX); }
-
-// one workgroup per tile: the CIC weights of the particles of its runs
-// accumulated in LDS over the tile's cells and their +1 reach, then added
-// per touched cell into the level's density storage, which holds the
-// fixed-point sums until k_deposit_finish converts them.
-//
-// PHASED: the launch covers the tiles of one parity class (tile coordinates
-// (2a + px, 2b + py, 2c + pz), phase = px + 2 py + 4 pz) and adds with plain
-// loads and stores.  Two tiles of a class are at least two tiles apart, so
-// their 17^3 boxes are disjoint (with TT even also across the periodic wrap,
-// whose reach lands in tile 0's box only), and the eight classes run as
-// eight launches in order.  Otherwise every tile in one launch adds with
-// device-scope 64-bit atomics.  Integer sums make both bitwise the same.
-template <bool PHASED>
-__global__ __launch_bounds__(PM_BLOCK) void k_tile_deposit(const float* __restrict__ xs, const float* __restrict__ ys,
-                                                           const float* __restrict__ zs,
-                                                           const int64_t* __restrict__ runs,
-                                                           const int* __restrict__ count,
-                                                           const int64_t* __restrict__ first, int nlaunch, int TT,
-                                                           int phase, unsigned long long* __restrict__ sums, Geo g,
-                                                           double wpar)
+// SMALL: v < 2^11.  v + 1.5 * 2^12 then lies in [2^12, 2^13), where a double's
+// last place is 2^-40: the addition itself rounds v to nearest (ties to even,
+// as the conversion does), and the sum's bits less those of 1.5 * 2^12 (whose
+// low word is zero) are the integer.  Two instructions instead of the dozen of
+// the 64-bit conversion.
+template <bool SMALL>
+__device__ __forceinline__ unsigned long long pm_fix(double v)
 {
-    __shared__ unsigned long long acc[PM_TCELLS];
-    const int N = g.n;
-    for (int bt = blockIdx.x; bt < nlaunch; bt += gridDim.x) {
-        int t = bt;
-        if constexpr (PHASED) {
-            const int H = TT >> 1;
-            const int a = bt % H, b2 = (bt / H) % H, c2 = bt / (H * H);
-            t = ((2 * c2 + ((phase >> 2) & 1)) * TT + 2 * b2 + ((phase >> 1) & 1)) * TT + 2 * a + (phase & 1);
-        }
-        const int c = count[t];
-        if (c == 0) continue;  // uniform over the block
-        for (int i = threadIdx.x; i < PM_TCELLS; i += blockDim.x) acc[i] = 0ull;
-        __syncthreads();
-        const int i00 = (t % TT) * PM_TILE, j00 = ((t / TT) % TT) * PM_TILE, k00 = (t / (TT * TT)) * PM_TILE;
-        const int64_t o = first[t];
-        // thread q: particle q % PM_RUN of run q / PM_RUN (idle past its length)
-        for (int64_t q = threadIdx.x; q < (int64_t)c * PM_RUN; q += blockDim.x) {
-            const int64_t d = runs[o + q / PM_RUN];
-            const int u = (int)(q % PM_RUN);
-            if (u > (int)(d % PM_RUN)) continue;
-            const int64_t pr = d / PM_RUN;
-            const double X = xs[pr + u], Y = ys[pr + u], Z = zs[pr + u];
-            const int I = (int)X, J = (int)Y, K = (int)Z;  // in [1, N]: checked when binned
-            const double D1 = X - (double)I, D2 = Y - (double)J, D3 = Z - (double)K;
-            const double T1 = 1.0 - D1, T2 = 1.0 - D2, T3 = 1.0 - D3;
-            const double T2W = T2 * wpar, D2W = D2 * wpar;
-            const int b = ((K - 1 - k00) * PM_TBUF + (J - 1 - j00)) * PM_TBUF + (I - 1 - i00);
-            atomicAdd(&acc[b], pm_fix(T3 * T1 * T2W));
-            atomicAdd(&acc[b + 1], pm_fix(T3 * D1 * T2W));
-            atomicAdd(&acc[b + PM_TBUF], pm_fix(T3 * T1 * D2W));
-            atomicAdd(&acc[b + PM_TBUF + 1], pm_fix(T3 * D1 * D2W));
-            atomicAdd(&acc[b + PM_TBUF * PM_TBUF], pm_fix(D3 * T1 * T2W));
-            atomicAdd(&acc[b + PM_TBUF * PM_TBUF + 1], pm_fix(D3 * D1 * T2W));
-            atomicAdd(&acc[b + PM_TBUF * PM_TBUF + PM_TBUF], pm_fix(D3 * T1 * D2W));
-            atomicAdd(&acc[b + PM_TBUF * PM_TBUF + PM_TBUF + 1], pm_fix(D3 * D1 * D2W));
-        }
-        __syncthreads();
-        for (int i = threadIdx.x; i < PM_TCELLS; i += blockDim.x) {
-            const unsigned long long v = acc[i];
-            if (v == 0ull) continue;
-            int gi = i00 + i % PM_TBUF, gj = j00 + (i / PM_TBUF) % PM_TBUF, gk = k00 + i / (PM_TBUF * PM_TBUF);
-            gi = gi >= N ? gi - N : gi;
-            gj = gj >= N ? gj - N : gj;
-            gk = gk >= N ? gk - N : gk;
-            if constexpr (PHASED)
-                sums[split_index(g, gi, gj, gk)] += v;
-            else
-                atomicAdd(&sums[split_index(g, gi, gj, gk)], v);
-        }
-        __syncthreads();
-    }
+    if constexpr (SMALL)
+        return (unsigned long long)__double_as_longlong(v + 6144.0) - 0x40B8000000000000ull;
+    else
+        return __double2ull_rn(v * PM_FIX);
+}
+constexpr double PM_FIX_SMALL = 2048.0;
+
+// the eight weights of a particle with fractions D1, D2, D3 (DENSIT's products
+// in its order) added at LDS cell b and its +1 neighbours, where KEEP says that
+// the node is the tile's
+template <bool SMALL, typename KEEP>
+__device__ __forceinline__ void pm_add8(unsigned long long* acc, int b, double D1, double D2, double D3, double wpar,
+                                        KEEP keep)
+{
+    const double T1 = 1.0 - D1, T2 = 1.0 - D2, T3 = 1.0 - D3;
+    const double T2W = T2 * wpar, D2W = D2 * wpar;
+    const double TT = T3 * T1, TD = T3 * D1, DT = D3 * T1, DD = D3 * D1;
+    constexpr int SY = PM_LX, SZ = PM_TY * PM_LX;
+    if (keep(0, 0, 0)) atomicAdd(&acc[b], pm_fix<SMALL>(TT * T2W));
+    if (keep(1, 0, 0)) atomicAdd(&acc[b + 1], pm_fix<SMALL>(TD * T2W));
+    if (keep(0, 1, 0)) atomicAdd(&acc[b + SY], pm_fix<SMALL>(TT * D2W));
+    if (keep(1, 1, 0)) atomicAdd(&acc[b + SY + 1], pm_fix<SMALL>(TD * D2W));
+    if (keep(0, 0, 1)) atomicAdd(&acc[b + SZ], pm_fix<SMALL>(DT * T2W));
+    if (keep(1, 0, 1)) atomicAdd(&acc[b + SZ + 1], pm_fix<SMALL>(DD * T2W));
+    if (keep(0, 1, 1)) atomicAdd(&acc[b + SZ + SY], pm_fix<SMALL>(DT * D2W));
+    if (keep(1, 1, 1)) atomicAdd(&acc[b + SZ + SY + 1], pm_fix<SMALL>(DD * D2W));
 }
 
-// the fixed-point sums (in place) -> delta = -1 + sum * 2^-40
-__global__ __launch_bounds__(256) void k_deposit_finish(double* __restrict__ rho, size_t n)
+// One workgroup per tile: the CIC weights that fall into the tile's cells
+// accumulated in LDS, then written once as delta.  The particles are those of
+// the tile's own 8 bins and, for each of the 7 tiles one step back in x, y
+// and/or z, those of its bins whose +1 nodes reach this tile; of a particle
+// only the nodes inside the tile are added.  Every cell is written by exactly
+// one block, so the density needs no clearing, no atomics and no conversion
+// pass, at the price of the reach's particles being read twice (1.25 times
+// the particles).  One thread per particle: a thread per (run, position) left
+// two lanes in three idle, as runs of a clustered lattice are short.
+//
+// 512^3 cells, 512^3 particles (lattice displaced by 2 cells rms): this kernel
+// 1.35 ms (2.75 with a thread per run and position), the whole deposit with
+// its reading back 6.5 -> 2.85 ms.  Before, 16^3-cell tiles added into the
+// grid in eight launches by parity class (2.65 ms) between a clearing and a
+// conversion pass (0.55 ms).  What bounds it now is the gather of positions
+// in bin order and the LDS additions (a third of the time each).
+constexpr int PM_SEGS = 21;  // own inner bin; own bins 1..7; 4 + 4 + 2 + 4 + 2 + 2 + 1 bins of the others
+constexpr int PM_DBLOCK = 512;
+
+template <bool SMALL>
+__global__ __launch_bounds__(PM_DBLOCK) void k_tile_deposit(const float* __restrict__ xs,
+                                                            const float* __restrict__ ys,
+                                                            const float* __restrict__ zs,
+                                                            const unsigned* __restrict__ order,
+                                                            const int* __restrict__ count,
+                                                            const int64_t* __restrict__ first, unsigned ntiles,
+                                                            PmTiles T, double* __restrict__ rho, Geo g, double wpar)
 {
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const unsigned long long v = reinterpret_cast<const unsigned long long*>(rho)[i];
-        rho[i] = -1.0 + (double)v * PM_UNFIX;
+    __shared__ unsigned long long acc[PM_TCELLS];
+    __shared__ int64_t seg_off[PM_SEGS];  // item q of segment s is order[seg_off[s] + q]
+    __shared__ int64_t seg_end[PM_SEGS];  // running count of particles
+    __shared__ int seg_dir[PM_SEGS];
+    unsigned t;
+    if (!map_block(ntiles, t)) return;
+    const int N = g.n;
+    const int tx = (int)(t % (unsigned)T.x), ty = (int)((t / (unsigned)T.x) % (unsigned)T.y),
+              tz = (int)(t / (unsigned)(T.x * T.y));
+    if (threadIdx.x < 64) {
+        // segment s > 1: the tile one step back in the directions of d, one of
+        // its bins with all of d set
+        const int s = (int)threadIdx.x;
+        int64_t items = 0, start = 0;
+        if (s < PM_SEGS) {
+            const int dir[PM_SEGS] = {0, 0, 1, 1, 1, 1, 2, 2, 2, 2, 3, 3, 4, 4, 4, 4, 5, 5, 6, 6, 7};
+            const int flag[PM_SEGS] = {0, 1, 1, 3, 5, 7, 2, 3, 6, 7, 3, 7, 4, 5, 6, 7, 5, 7, 6, 7, 7};
+            const int d = dir[s];
+            const int bx = (d & 1) ? wrap_dec(tx, T.x) : tx, by = (d & 2) ? wrap_dec(ty, T.y) : ty,
+                      bz = (d & 4) ? wrap_dec(tz, T.z) : tz;
+            const int b = ((bz * T.y + by) * T.x + bx) * 8 + flag[s];
+            start = first[b];
+            items = s == 1 ? first[b + 6] + count[b + 6] - start : (int64_t)count[b];
+            seg_dir[s] = d;
+        }
+        int64_t end = items;
+#pragma unroll
+        for (int off = 1; off < 32; off <<= 1) {
+            const int64_t v = __shfl_up(end, off, 64);
+            if (s >= off) end += v;
+        }
+        if (s < PM_SEGS) {
+            seg_end[s] = end;
+            seg_off[s] = start - (end - items);
+        }
+    }
+    for (int i = threadIdx.x; i < PM_TCELLS; i += PM_DBLOCK) acc[i] = 0ull;
+    __syncthreads();
+    const int i00 = tx * PM_TX, j00 = ty * PM_TY, k00 = tz * PM_TZ;
+    const int ex = N - i00 < PM_TX ? N - i00 : PM_TX, ey = N - j00 < PM_TY ? N - j00 : PM_TY,
+              ez = N - k00 < PM_TZ ? N - k00 : PM_TZ;
+    // INT(X) >= 1 (checked when binned) and the fraction X - INT(X), both exact
+    // in REAL*4; the next particle is loaded before this one is added
+    const int64_t total = seg_end[PM_SEGS - 1];
+    int s = 0, sn = 0;
+    float x = 0.0f, y = 0.0f, z = 0.0f;
+    auto fetch = [&](int64_t q, int& seg, float& fx, float& fy, float& fz) {
+        if (q >= total) return;
+        while (q >= seg_end[seg]) seg++;
+        const unsigned p = order[seg_off[seg] + q];
+        fx = xs[p];
+        fy = ys[p];
+        fz = zs[p];
+    };
+    fetch(threadIdx.x, s, x, y, z);
+    for (int64_t q = threadIdx.x; q < total; q += PM_DBLOCK) {
+        float xn = 0.0f, yn = 0.0f, zn = 0.0f;
+        sn = s;
+        fetch(q + PM_DBLOCK, sn, xn, yn, zn);
+        const float fi = truncf(x), fj = truncf(y), fk = truncf(z);
+        const double D1 = (double)(x - fi), D2 = (double)(y - fj), D3 = (double)(z - fk);
+        const int I = (int)fi - 1 - i00, J = (int)fj - 1 - j00, K = (int)fk - 1 - k00;
+        if (__all(s == 0)) {  // all eight nodes are the tile's
+            pm_add8<SMALL>(acc, (K * PM_TY + J) * PM_LX + I, D1, D2, D3, wpar, [](int, int, int) { return true; });
+        } else {
+            // base cell in the tile's frame: -1 in a direction the particle comes from
+            const int d = seg_dir[s];
+            const int bi = (d & 1) ? -1 : I, bj = (d & 2) ? -1 : J, bk = (d & 4) ? -1 : K;
+            pm_add8<SMALL>(acc, (bk * PM_TY + bj) * PM_LX + bi, D1, D2, D3, wpar, [&](int a, int b, int c) {
+                return (a ? bi + 1 < ex : bi >= 0) && (b ? bj + 1 < ey : bj >= 0) && (c ? bk + 1 < ez : bk >= 0);
+            });
+        }
+        s = sn;
+        x = xn;
+        y = yn;
+        z = zn;
+    }
+    __syncthreads();
+    // delta = -1 + sum * 2^-40, 16 values of one colour at a time (the tile's
+    // first cell has even coordinates, so local parity is global parity)
+    for (int i = threadIdx.x; i < PM_TX * PM_TY * PM_TZ; i += PM_DBLOCK) {
+        const int m = i & 15, c = (i >> 4) & 1, j = (i >> 5) & (PM_TY - 1), k = i >> 9;
+        if (2 * m >= ex || j >= ey || k >= ez) continue;
+        const int xc = 2 * m + ((c + j + k) & 1);
+        const unsigned long long v = acc[(k * PM_TY + j) * PM_LX + xc];
+        rho[(size_t)c * g.half + row_base(g, j00 + j, k00 + k) + (unsigned)(i00 / 2 + m)] = -1.0 + (double)v * PM_UNFIX;
     }
 }
 
@@ -350,9 +483,10 @@ __global__ __launch_bounds__(PM_BLOCK) void k_move(float* __restrict__ xs, float
     double svel = 0.0;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < np; p += stride) {
-        double X = xs[p], Y = ys[p], Z = zs[p];
+        const float xf0 = xs[p], yf0 = ys[p], zf0 = zs[p];
+        double X = xf0, Y = yf0, Z = zf0;
         double VVX = vxs[p], VVY = vys[p], VVZ = vzs[p];
-        const int I = cell_of(X, N), J = cell_of(Y, N), K = cell_of(Z, N);
+        const int I = cell_of(xf0, N), J = cell_of(yf0, N), K = cell_of(zf0, N);
         if (I < 0 || J < 0 || K < 0) {
             atomicAdd(bad, 1);
             continue;
@@ -452,11 +586,13 @@ static int pm_ensure_particles(mgs_handle* h, int64_t np)
     if (p->buf) (void)hipFree(p->buf);
     p->buf = nullptr;
     p->np = 0;
-    if (hipMalloc((void**)&p->buf, (size_t)np * 6 * sizeof(float)) != hipSuccess) {
+    const int64_t ld = (np + 63) / 64 * 64;
+    if (hipMalloc((void**)&p->buf, (size_t)ld * 6 * sizeof(float)) != hipSuccess) {
         p->buf = nullptr;
         return set_err(h, MGS_E_NOMEM, "particle arrays (" + std::to_string(np) + " particles)");
     }
     p->np = np;
+    p->ld = ld;
     return 0;
 }
 
@@ -493,7 +629,7 @@ int mgs_particles_set(mgs_handle* h, const float* x, const float* y, const float
     const hipMemcpyKind kind = where == MGS_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
     const float* src[6] = {x, y, z, vx, vy, vz};
     for (int a = 0; a < 6; a++) {
-        float* dst = p->buf + (size_t)a * npart;
+        float* dst = p->buf + (size_t)a * p->ld;
         const hipError_t e = src[a] ? hipMemcpyAsync(dst, src[a], bytes, kind, h->s) : hipMemsetAsync(dst, 0, bytes, h->s);
         if (e != hipSuccess) return set_err(h, MGS_E_HIP, "particle upload");
     }
@@ -511,43 +647,44 @@ int mgs_particles_get(mgs_handle* h, float* x, float* y, float* z, float* vx, fl
     const hipMemcpyKind kind = where == MGS_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
     float* dst[6] = {x, y, z, vx, vy, vz};
     for (int a = 0; a < 6; a++)
-        if (dst[a] && hipMemcpyAsync(dst[a], p->buf + (size_t)a * p->np, bytes, kind, h->s) != hipSuccess)
+        if (dst[a] && hipMemcpyAsync(dst[a], p->buf + (size_t)a * p->ld, bytes, kind, h->s) != hipSuccess)
             return set_err(h, MGS_E_HIP, "particle download");
     if (hipStreamSynchronize(h->s) != hipSuccess) return set_err(h, MGS_E_HIP, "particle download");
     return 0;
 }
 
-// the deposit's binning buffers for the current particle count and ntiles
-static int pm_ensure_bins(mgs_handle* h, PmState* p, int ntiles)
+// the deposit's binning buffers for the current particle count and nbins
+static int pm_ensure_bins(mgs_handle* h, PmState* p, int nbins)
 {
     if (p->nbin != p->np) {
-        for (void* q : {(void*)p->key, (void*)p->rank, (void*)p->runs})
+        for (void* q : {(void*)p->recs, (void*)p->nrec, (void*)p->order})
             if (q) (void)hipFree(q);
-        p->key = p->rank = nullptr;
-        p->runs = nullptr;
+        p->recs = nullptr;
+        p->nrec = nullptr;
+        p->order = nullptr;
         p->nbin = 0;
-        const size_t n = (size_t)p->np;
-        if (hipMalloc((void**)&p->key, n * sizeof(int)) != hipSuccess ||
-            hipMalloc((void**)&p->rank, n * sizeof(int)) != hipSuccess ||
-            hipMalloc((void**)&p->runs, n * sizeof(int64_t)) != hipSuccess)
+        const size_t waves = ((size_t)p->np + PM_WCHUNK - 1) / PM_WCHUNK;
+        if (hipMalloc((void**)&p->recs, waves * PM_WCHUNK * sizeof(unsigned long long)) != hipSuccess ||
+            hipMalloc((void**)&p->nrec, waves * sizeof(int)) != hipSuccess ||
+            hipMalloc((void**)&p->order, (size_t)p->np * sizeof(int64_t)) != hipSuccess)
             return set_err(h, MGS_E_NOMEM, "deposit binning arrays");
         p->nbin = p->np;
     }
-    if (p->ntiles != ntiles) {
+    if (p->nbins != nbins) {
         for (void* q : {(void*)p->count, (void*)p->first, p->scan_tmp})
             if (q) (void)hipFree(q);
         p->count = nullptr;
         p->first = nullptr;
         p->scan_tmp = nullptr;
-        p->ntiles = 0;
+        p->nbins = 0;
         size_t bytes = 0;
-        if (hipMalloc((void**)&p->count, (size_t)ntiles * sizeof(int)) != hipSuccess ||
-            hipMalloc((void**)&p->first, (size_t)ntiles * sizeof(int64_t)) != hipSuccess ||
-            hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, p->count, p->first, ntiles, h->s) != hipSuccess ||
+        if (hipMalloc((void**)&p->count, (size_t)nbins * sizeof(int)) != hipSuccess ||
+            hipMalloc((void**)&p->first, (size_t)nbins * sizeof(int64_t)) != hipSuccess ||
+            hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, p->count, p->first, nbins, h->s) != hipSuccess ||
             hipMalloc(&p->scan_tmp, bytes + 256) != hipSuccess)
             return set_err(h, MGS_E_NOMEM, "deposit tile arrays");
         p->scan_bytes = bytes + 256;
-        p->ntiles = ntiles;
+        p->nbins = nbins;
     }
     return 0;
 }
@@ -560,39 +697,33 @@ int mgs_cic_deposit(mgs_handle* h)
     if (p->np >= ((int64_t)1 << 31)) return set_err(h, MGS_E_ARG, "the deposit takes fewer than 2^31 particles");
     const int N = h->p.ngrid;
     const Geo g = make_geo(N);
-    const int TT = (N + PM_TILE - 1) / PM_TILE;
-    int rc = pm_ensure_bins(h, p, TT * TT * TT);
+    const PmTiles T = pm_tiles(N);
+    const int ntiles = T.x * T.y * T.z;
+    int rc = pm_ensure_bins(h, p, 8 * ntiles);
     if (rc) return rc;
-    const int64_t np = p->np;
+    const int64_t np = p->np, ld = p->ld;
     const float* b = p->buf;
     prof_begin(h, MGS_KC_PM, (double)np * 56.0 + 32.0 * (double)N * N * N);
-    // the density storage holds the fixed-point sums (zero) until k_deposit_finish
-    launch_fill_f64(h->L[0].rho, (size_t)N * N * N, 0.0, h->s);
     if (hipMemsetAsync(p->bad, 0, sizeof(int), h->s) != hipSuccess ||
-        hipMemsetAsync(p->count, 0, (size_t)p->ntiles * sizeof(int), h->s) != hipSuccess)
+        hipMemsetAsync(p->count, 0, (size_t)p->nbins * sizeof(int), h->s) != hipSuccess)
         return set_err(h, MGS_E_HIP, "deposit");
-    const int gbin = pm_grid((np + PM_RUN - 1) / PM_RUN);
-    hipLaunchKernelGGL(k_bin_count, dim3(gbin), dim3(PM_BLOCK), 0, h->s, b, b + np, b + 2 * np, np, N, TT,
-                       p->key, p->rank, p->count, p->bad);
-    if (hipcub::DeviceScan::ExclusiveSum(p->scan_tmp, p->scan_bytes, p->count, p->first, p->ntiles, h->s) !=
+    const int64_t nwaves = (np + PM_WCHUNK - 1) / PM_WCHUNK;
+    const unsigned gbin = (unsigned)((nwaves + PM_BLOCK / 64 - 1) / (PM_BLOCK / 64));
+    hipLaunchKernelGGL(k_bin_count, dim3(gbin), dim3(PM_BLOCK), 0, h->s, b, b + ld, b + 2 * ld, np, N, T, p->recs,
+                       p->nrec, p->count, p->bad);
+    if (hipcub::DeviceScan::ExclusiveSum(p->scan_tmp, p->scan_bytes, p->count, p->first, p->nbins, h->s) !=
         hipSuccess)
         return set_err(h, MGS_E_HIP, "deposit scan");
-    hipLaunchKernelGGL(k_bin_scatter, dim3(gbin), dim3(PM_BLOCK), 0, h->s, np, p->key, p->rank, p->first, p->runs);
-    unsigned long long* sums = reinterpret_cast<unsigned long long*>(h->L[0].rho);
-    if (TT % 2 == 0) {
-        const int per = p->ntiles / 8;  // tiles of one parity class
-        for (int ph = 0; ph < 8; ph++)
-            hipLaunchKernelGGL(k_tile_deposit<true>, dim3((unsigned)per), dim3(PM_BLOCK), 0, h->s, b, b + np,
-                               b + 2 * np, p->runs, p->count, p->first, per, TT, ph, sums, g, wpar_of(N, np));
-    } else {
-        hipLaunchKernelGGL(k_tile_deposit<false>, dim3((unsigned)p->ntiles), dim3(PM_BLOCK), 0, h->s, b, b + np,
-                           b + 2 * np, p->runs, p->count, p->first, p->ntiles, TT, 0, sums, g, wpar_of(N, np));
-    }
-    {
-        const size_t n3 = (size_t)N * N * N;
-        const unsigned gfin = (unsigned)std::min<size_t>((n3 + 255) / 256, 65536);
-        hipLaunchKernelGGL(k_deposit_finish, dim3(gfin), dim3(256), 0, h->s, h->L[0].rho, n3);
-    }
+    hipLaunchKernelGGL(k_bin_scatter, dim3(gbin), dim3(PM_BLOCK), 0, h->s, nwaves, p->recs, p->nrec, p->first,
+                       p->order);
+    const double wpar = wpar_of(N, np);
+    const unsigned gt = ((unsigned)ntiles + 7) / 8 * 8;  // map_block
+    if (wpar < PM_FIX_SMALL)
+        hipLaunchKernelGGL(k_tile_deposit<true>, dim3(gt), dim3(PM_DBLOCK), 0, h->s, b, b + ld, b + 2 * ld, p->order,
+                           p->count, p->first, (unsigned)ntiles, T, h->L[0].rho, g, wpar);
+    else
+        hipLaunchKernelGGL(k_tile_deposit<false>, dim3(gt), dim3(PM_DBLOCK), 0, h->s, b, b + ld, b + 2 * ld, p->order,
+                           p->count, p->first, (unsigned)ntiles, T, h->L[0].rho, g, wpar);
     prof_end(h);
     rc = pm_check_bad(h, "CIC deposit");
     h->has_density = true;
@@ -611,10 +742,10 @@ int mgs_move(mgs_handle* h, double pconst, double xconst, double* svel)
     const int grid = pm_grid(p->np);
     prof_begin(h, MGS_KC_PM, (double)p->np * 48.0);
     if (hipMemsetAsync(p->bad, 0, sizeof(int), h->s) != hipSuccess) return set_err(h, MGS_E_HIP, "move");
-    const int64_t np = p->np;
+    const int64_t np = p->np, ld = p->ld;
     float* b = p->buf;
-    hipLaunchKernelGGL(k_move, dim3(grid), dim3(PM_BLOCK), 0, h->s, b, b + np, b + 2 * np, b + 3 * np, b + 4 * np,
-                       b + 5 * np, np, p->phi, N, pconst, xconst, wpar_of(N, np), p->part, p->bad);
+    hipLaunchKernelGGL(k_move, dim3(grid), dim3(PM_BLOCK), 0, h->s, b, b + ld, b + 2 * ld, b + 3 * ld, b + 4 * ld,
+                       b + 5 * ld, np, p->phi, N, pconst, xconst, wpar_of(N, np), p->part, p->bad);
     launch_sum_partials(p->part, grid, h->dsum, h->s);
     prof_end(h);
     double s = 0.0;

@@ -1,0 +1,49 @@
+"""The deposit's tiles (32 x 16 x 8 cells) and run binning at their edges,
+against the numpy restatement in oracle/pm.py."""
+import numpy as np
+import pytest
+
+import mgsolve as M
+import pm as P
+
+
+def _cfg(N):
+    return M.Config(N=N, model=M.MODEL_FR, fr_n=1, box=2.0 * N, fr0=-1e-5, precision=M.PREC_FP64)
+
+
+# one partial tile; a last tile two cells wide in x and y; whole tiles; a
+# weight of 2^11 and more (the 64-bit conversion); more bins in a block of
+# unordered particles than its table has slots; a single particle
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,n,edge", [(8, 4001, True), (34, 30007, True), (64, 50000, False), (64, 100, True),
+                                      (192, 40000, False), (16, 1, False)])
+def test_deposit_at_tile_edges(N, n, edge):
+    rng = np.random.default_rng(N + n)
+    pos = [rng.uniform(1.0, N + 1.0, n).astype(np.float32) for _ in range(3)]
+    last = np.nextafter(np.float32(N + 1), np.float32(0))
+    if edge:  # a third of the coordinates on or beside tile faces and the wrap
+        for a, t in zip(pos, (32, 16, 8)):
+            faces = np.arange(0, N + 1, t)
+            v = rng.choice(faces, n // 3) + rng.choice([0.5, 1.0, 1.5, 0.99999994], n // 3)
+            a[:n // 3] = np.clip(v, 1.0, last)
+    pos = [np.clip(a, np.float32(1.0), last) for a in pos]
+    print(f"[pm tiles] N={N} np={n}", flush=True)
+    with M.Solver(_cfg(N)) as S:
+        S.set_particles(*pos)
+        S.cic_deposit()
+        d = S.get_density(np.float64)
+        perm = rng.permutation(n)
+        S.set_particles(*[a[perm] for a in pos])
+        S.cic_deposit()
+        d2 = S.get_density(np.float64)
+    ref = P.cic_deposit(*pos, N)
+    # contributions per cell: each is rounded to a multiple of 2^-40, and the
+    # oracle's FP64 sum rounds once per addition
+    cnt = np.zeros((N, N, N))
+    idx = [a.astype(np.int64) - 1 for a in pos]
+    for o in range(8):
+        i, j, k = ((v + ((o >> b) & 1)) % N for b, v in enumerate(idx))
+        np.add.at(cnt, (k, j, i), 1.0)
+    tol = cnt.max() * (2.0 ** -41 + 2.0 ** -52 * (ref.max() + 2.0)) + 2.0 ** -52 * (ref.max() + 2.0)
+    assert np.max(np.abs(d - ref)) <= tol, (np.max(np.abs(d - ref)), tol)
+    assert np.array_equal(d, d2)
