@@ -362,8 +362,8 @@ __device__ __forceinline__ void pm_add8(unsigned long long* acc, int b, double D
 // 1.35 ms (2.75 with a thread per run and position), the whole deposit with
 // its reading back 6.5 -> 2.85 ms.  Before, 16^3-cell tiles added into the
 // grid in eight launches by parity class (2.65 ms) between a clearing and a
-// conversion pass (0.55 ms).  What bounds it now is the gather of positions
-// in bin order and the LDS additions (a third of the time each).
+// conversion pass (0.55 ms).  What is left is the gather of
+// positions in bin order and the LDS additions.
 constexpr int PM_SEGS = 21;  // own inner bin; own bins 1..7; 4 + 4 + 2 + 4 + 2 + 2 + 1 bins of the others
 constexpr int PM_DBLOCK = 512;
 
@@ -465,6 +465,28 @@ __global__ __launch_bounds__(PM_DBLOCK) void k_tile_deposit(const float* __restr
     }
 }
 
+// M adjacent floats from element i of a (4-byte aligned)
+template <int M>
+__device__ __forceinline__ void row_load(const float* a, unsigned i, float (&v)[M])
+{
+    const char* p = reinterpret_cast<const char*>(a) + i * (unsigned)sizeof(float);
+    if constexpr (M == 4) {
+        const Words4 w = *reinterpret_cast<const Words4*>(p);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = __uint_as_float(w.v[e]);
+    } else {
+        const Words2 w = *reinterpret_cast<const Words2*>(p);
+#pragma unroll
+        for (int e = 0; e < 2; e++) v[e] = __uint_as_float(w.v[e]);
+    }
+}
+
+// Bound by the texture addressers (93 % busy): the lanes of a wave meet
+// different rows, so each load costs an address cycle per line it touches.  A
+// row's values in one 16- or 8-byte load make 12 loads of the 32; 15.6 M
+// particles on 250^3 cells: 633 -> 435 us.  Prefetching the next particle, or
+// five waves per SIMD (28 bytes of spills: 527 us), did not help.
+//
 // MOVE's particle loop for the f(R) and nDGP models (no friction or mass
 // terms, PMP2main.f90:488-684): kick with the CIC-interpolated gradient of
 // the potential, drift, periodic wrap, SVEL partial per block
@@ -479,7 +501,7 @@ __global__ __launch_bounds__(PM_BLOCK) void k_move(float* __restrict__ xs, float
     // reference does (default REAL: the 1e-8 is below float resolution)
     const double XN = (double)((float)N + 1.0f - 1.0e-8f);
     const double YN = (double)N;
-    const size_t n = (size_t)N;
+    const unsigned n = (unsigned)N;
     double svel = 0.0;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < np; p += stride) {
@@ -498,16 +520,49 @@ __global__ __launch_bounds__(PM_BLOCK) void k_move(float* __restrict__ xs, float
         const int x1 = I - 1, x2 = I == N ? 0 : I, x3 = I + 1 >= N ? I + 1 - N : I + 1, x0 = I == 1 ? N - 1 : I - 2;
         const int y1 = J - 1, y2 = J == N ? 0 : J, y3 = J + 1 >= N ? J + 1 - N : J + 1, y0 = J == 1 ? N - 1 : J - 2;
         const int z1 = K - 1, z2 = K == N ? 0 : K, z3 = K + 1 >= N ? K + 1 - N : K + 1, z0 = K == 1 ? N - 1 : K - 2;
-#define PHI(a, b, c) phi[(size_t)(a) + n * ((size_t)(b) + n * (size_t)(c))]
-        const float F111 = PHI(x1, y1, z1), F211 = PHI(x2, y1, z1), F121 = PHI(x1, y2, z1), F221 = PHI(x2, y2, z1);
-        const float F112 = PHI(x1, y1, z2), F212 = PHI(x2, y1, z2), F122 = PHI(x1, y2, z2), F222 = PHI(x2, y2, z2);
-        const float F113 = PHI(x1, y1, z3), F213 = PHI(x2, y1, z3), F123 = PHI(x1, y2, z3), F223 = PHI(x2, y2, z3);
-        const float F110 = PHI(x1, y1, z0), F210 = PHI(x2, y1, z0), F120 = PHI(x1, y2, z0), F220 = PHI(x2, y2, z0);
-        const float F311 = PHI(x3, y1, z1), F321 = PHI(x3, y2, z1), F131 = PHI(x1, y3, z1), F231 = PHI(x2, y3, z1);
-        const float F312 = PHI(x3, y1, z2), F322 = PHI(x3, y2, z2), F132 = PHI(x1, y3, z2), F232 = PHI(x2, y3, z2);
-        const float F011 = PHI(x0, y1, z1), F021 = PHI(x0, y2, z1), F101 = PHI(x1, y0, z1), F201 = PHI(x2, y0, z1);
-        const float F012 = PHI(x0, y1, z2), F022 = PHI(x0, y2, z2), F102 = PHI(x1, y0, z2), F202 = PHI(x2, y0, z2);
-#undef PHI
+        // rows of the 4 x 4 x 4 block: x0 .. x3 in the four centre rows, x1 and x2
+        // in the eight rows beside them.  Away from the wrap in x a row's values
+        // are adjacent: one 16-byte and one 8-byte load (4-byte aligned) per row
+        // instead of 32 loads
+        float c11[4], c21[4], c12[4], c22[4];        // (y, z)
+        float a01[2], a31[2], a02[2], a32[2];        // y0, y3 at z1, z2
+        float b10[2], b13[2], b20[2], b23[2];        // z0, z3 at y1, y2
+        // rows as 32-bit element offsets from the uniform base (N^3 <= 2^30)
+        const unsigned r11 = n * ((unsigned)y1 + n * (unsigned)z1), r21 = n * ((unsigned)y2 + n * (unsigned)z1);
+        const unsigned r12 = n * ((unsigned)y1 + n * (unsigned)z2), r22 = n * ((unsigned)y2 + n * (unsigned)z2);
+        const unsigned q01 = n * ((unsigned)y0 + n * (unsigned)z1), q31 = n * ((unsigned)y3 + n * (unsigned)z1);
+        const unsigned q02 = n * ((unsigned)y0 + n * (unsigned)z2), q32 = n * ((unsigned)y3 + n * (unsigned)z2);
+        const unsigned p10 = n * ((unsigned)y1 + n * (unsigned)z0), p13 = n * ((unsigned)y1 + n * (unsigned)z3);
+        const unsigned p20 = n * ((unsigned)y2 + n * (unsigned)z0), p23 = n * ((unsigned)y2 + n * (unsigned)z3);
+        if (I > 1 && I < N - 1) {
+            const unsigned e0 = (unsigned)x0, e1 = (unsigned)x1;
+            row_load(phi, r11 + e0, c11), row_load(phi, r21 + e0, c21), row_load(phi, r12 + e0, c12);
+            row_load(phi, r22 + e0, c22), row_load(phi, q01 + e1, a01), row_load(phi, q31 + e1, a31);
+            row_load(phi, q02 + e1, a02), row_load(phi, q32 + e1, a32), row_load(phi, p10 + e1, b10);
+            row_load(phi, p13 + e1, b13), row_load(phi, p20 + e1, b20), row_load(phi, p23 + e1, b23);
+        } else {
+            const unsigned xi[4] = {(unsigned)x0, (unsigned)x1, (unsigned)x2, (unsigned)x3};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                c11[e] = elem(phi, r11 + xi[e]), c21[e] = elem(phi, r21 + xi[e]);
+                c12[e] = elem(phi, r12 + xi[e]), c22[e] = elem(phi, r22 + xi[e]);
+            }
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const unsigned x = xi[e + 1];
+                a01[e] = elem(phi, q01 + x), a31[e] = elem(phi, q31 + x), a02[e] = elem(phi, q02 + x);
+                a32[e] = elem(phi, q32 + x), b10[e] = elem(phi, p10 + x), b13[e] = elem(phi, p13 + x);
+                b20[e] = elem(phi, p20 + x), b23[e] = elem(phi, p23 + x);
+            }
+        }
+        const float F011 = c11[0], F111 = c11[1], F211 = c11[2], F311 = c11[3];
+        const float F021 = c21[0], F121 = c21[1], F221 = c21[2], F321 = c21[3];
+        const float F012 = c12[0], F112 = c12[1], F212 = c12[2], F312 = c12[3];
+        const float F022 = c22[0], F122 = c22[1], F222 = c22[2], F322 = c22[3];
+        const float F101 = a01[0], F201 = a01[1], F131 = a31[0], F231 = a31[1];
+        const float F102 = a02[0], F202 = a02[1], F132 = a32[0], F232 = a32[1];
+        const float F110 = b10[0], F210 = b10[1], F113 = b13[0], F213 = b13[1];
+        const float F120 = b20[0], F220 = b20[1], F123 = b23[0], F223 = b23[1];
         // doubled gradients at the 8 nodes (the 1/2 is in pconst); the
         // reference's F's are default REAL, so each difference is a REAL*4
         // subtraction (PMP2main.f90:580-602), widened afterwards

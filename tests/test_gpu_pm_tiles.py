@@ -47,3 +47,25 @@ def test_deposit_at_tile_edges(N, n, edge):
     tol = cnt.max() * (2.0 ** -41 + 2.0 ** -52 * (ref.max() + 2.0)) + 2.0 ** -52 * (ref.max() + 2.0)
     assert np.max(np.abs(d - ref)) <= tol, (np.max(np.abs(d - ref)), tol)
     assert np.array_equal(d, d2)
+
+
+# every row of the potential's block wraps (N = 4); an odd particle count;
+# cells 1, N-1 and N in x, whose rows are gathered value by value
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,n", [(4, 777), (6, 64), (34, 20001)])
+def test_move_rows_at_the_wrap(N, n):
+    rng = np.random.default_rng(N)
+    pos = [rng.uniform(1.0, N + 1.0, n).astype(np.float32) for _ in range(3)]
+    last = np.nextafter(np.float32(N + 1), np.float32(0))
+    pos = [np.clip(a, np.float32(1.0), last) for a in pos]
+    vel = [rng.normal(0.0, 0.3, n).astype(np.float32) for _ in range(3)]
+    phi = rng.standard_normal((N, N, N)).astype(np.float32)
+    print(f"[pm move] N={N} np={n}", flush=True)
+    with M.Solver(_cfg(N)) as S:
+        S.set_potential(phi)
+        S.set_particles(*pos, *vel)
+        S.move(-0.07, 0.9)
+        got = S.get_particles()
+    ref = P.move(phi.astype(np.float64), *pos, *vel, -0.07, 0.9)
+    for a, b, name in zip(got, ref[:6], ("x", "y", "z", "vx", "vy", "vz")):
+        assert np.array_equal(a, b), (name, int(np.sum(a != b)))
