@@ -137,6 +137,24 @@ __device__ __forceinline__ T& lvl(T* a, unsigned i)
     else
         return a[i];
 }
+
+// the cells x = 2m, 2m+1 of a row of a lexicographic array, loaded or stored
+// by one instruction; aligned as an element, since a caller's array need be
+template <typename T>
+struct __attribute__((packed, aligned(sizeof(T)))) Pair {
+    T a, b;
+};
+
+// offsets in a colour-split array of the cells x = 2m and 2m+1 of row (j, k):
+// the same place in the half of parity (j + k) & 1 and in the other
+__device__ __forceinline__ void pair_split(const Geo& g, int m, int j, int k, size_t& e, size_t& o)
+{
+    const size_t r = row_base(g, j, k) + (unsigned)m;
+    const bool odd = (j + k) & 1;
+    e = r + (odd ? g.half : 0);
+    o = r + (odd ? 0 : g.half);
+}
+
 template <int FRN, typename T>
 __device__ __forceinline__ T wpow(T x)
 {

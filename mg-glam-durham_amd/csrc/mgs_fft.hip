@@ -19,6 +19,7 @@
 #include "mgs_device.h"
 #include "mgs_internal.h"
 #include "mgs_kernels.h"
+#include "mgs_stencil.h"
 
 namespace mgs {
 
@@ -163,39 +164,65 @@ __global__ __launch_bounds__(256) void k_lognormal(const double* __restrict__ g,
     }
 }
 
-// fifth-force potential at one cell from the split field
-__device__ __forceinline__ double psi_at(const double* __restrict__ u, const Geo& g, int i, int j, int k, int model,
-                                         int frn, double fct, double inv_ubg)
+// fifth-force potential of a cell with field value v
+__device__ __forceinline__ double psi_of(double v, int model, int frn, double fct, double inv_ubg)
 {
-    const double v = u[split_index(g, i, j, k)];
     if (model == MGS_MODEL_DGP) return 0.5 * v;
     const double x = v * inv_ubg;
     const double w = frn == 0 ? x : (frn == 1 ? x * x : x * x * x);
     return -fct * w;
 }
 
+// psi and its central differences, one thread per pair of cells (2m, 2m+1) of
+// a row, marching over a run of planes with psi of the planes k-1, k, k+1 in
+// registers: every access is a unit-stride run (the pairs of the rows beside
+// it lie at the same m), and the outputs are written once, past the caches.
+// A stream of 8 bytes in and 16 out per cell; 256^3, all four outputs in
+// REAL*4: 115 us = 3.5 TB/s (one thread per cell with 64-bit divisions 187,
+// pairs without the march 139, with cached stores 156).
 template <typename T>
 __global__ __launch_bounds__(256) void k_fifth_force(const double* __restrict__ u, T* __restrict__ psi,
                                                      T* __restrict__ gx, T* __restrict__ gy, T* __restrict__ gz, Geo g,
-                                                     int model, int frn, double fct, double inv_ubg)
+                                                     int model, int frn, double fct, double inv_ubg, int TX, int TY,
+                                                     int XB, int JB, int KC, unsigned NB)
 {
-    const size_t n3 = 2 * g.half;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n3; q += stride) {
-        const int i = (int)(q % g.n);
-        const size_t r = q / g.n;
-        const int j = (int)(r % g.n), k = (int)(r / g.n);
-        const int n = g.n;
-        if (psi) psi[q] = (T)psi_at(u, g, i, j, k, model, frn, fct, inv_ubg);
-        if (gx)
-            gx[q] = (T)(0.5 * (psi_at(u, g, wrap_inc(i, n), j, k, model, frn, fct, inv_ubg) -
-                               psi_at(u, g, wrap_dec(i, n), j, k, model, frn, fct, inv_ubg)));
-        if (gy)
-            gy[q] = (T)(0.5 * (psi_at(u, g, i, wrap_inc(j, n), k, model, frn, fct, inv_ubg) -
-                               psi_at(u, g, i, wrap_dec(j, n), k, model, frn, fct, inv_ubg)));
-        if (gz)
-            gz[q] = (T)(0.5 * (psi_at(u, g, i, j, wrap_inc(k, n), model, frn, fct, inv_ubg) -
-                               psi_at(u, g, i, j, wrap_dec(k, n), model, frn, fct, inv_ubg)));
+    ZCol c;
+    if (!zcol(g, TX, TY, XB, JB, KC, NB, c)) return;
+    const int n = g.n, j = c.j, m = c.m;
+    auto at = [&](size_t q) { return psi_of(u[q], model, frn, fct, inv_ubg); };
+    typedef T V2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));  // a caller's array: aligned as its elements
+    double pe, po, me = 0.0, mo = 0.0;  // planes k and k-1
+    size_t e, o;
+    if (gz) {
+        pair_split(g, m, j, wrap_dec(c.k0, n), e, o);
+        me = at(e), mo = at(o);
+    }
+    pair_split(g, m, j, c.k0, e, o);
+    pe = at(e), po = at(o);
+    for (int k = c.k0; k < c.k1; k++) {
+        const size_t q = ((size_t)k * n + j) * n + 2 * (unsigned)m;
+        auto store = [&](T* out, double a, double b) {
+            const V2 v = {(T)a, (T)b};
+            __builtin_nontemporal_store(v, reinterpret_cast<V2*>(out + q));
+        };
+        size_t en, on;
+        pair_split(g, m, j, wrap_inc(k, n), en, on);
+        double ne = 0.0, no = 0.0;
+        if (gz || k + 1 < c.k1) ne = at(en), no = at(on);
+        if (psi) store(psi, pe, po);
+        if (gx) {
+            const int ml = wrap_dec(m, g.h), mr = wrap_inc(m, g.h);
+            store(gx, 0.5 * (po - at(o - (unsigned)m + (unsigned)ml)), 0.5 * (at(e - (unsigned)m + (unsigned)mr) - pe));
+        }
+        if (gy) {
+            size_t ep, op, em, om;
+            pair_split(g, m, wrap_inc(j, n), k, ep, op);
+            pair_split(g, m, wrap_dec(j, n), k, em, om);
+            store(gy, 0.5 * (at(ep) - at(em)), 0.5 * (at(op) - at(om)));
+        }
+        if (gz) store(gz, 0.5 * (ne - me), 0.5 * (no - mo));
+        me = pe, mo = po, pe = ne, po = no;
+        e = en, o = on;
     }
 }
 
@@ -273,15 +300,25 @@ __global__ __launch_bounds__(256) void k_bin_power(const hipfftDoubleComplex* __
     for (int t = threadIdx.x; t < 6 * nb; t += blockDim.x) out[t] = hist[t];
 }
 
-// bins[t] = sum over blocks of part[block][t], in block order
+// bins[t] = sum over blocks of part[block][t] (nblk = 512 of them): 16 bins of
+// 16 threads each per workgroup, a thread adding every 16th block's value, then
+// the 16 partial sums in order.  One thread per bin walked 512 dependent
+// additions in four workgroups (256^3: 127 us).
 __global__ __launch_bounds__(256) void k_bin_reduce(const double* __restrict__ part, int nblk, int len,
                                                     double* __restrict__ bins)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= len) return;
-    double s = 0.0;
-    for (int b = 0; b < nblk; b++) s += part[(size_t)b * len + t];
-    bins[t] = s;
+    __shared__ double s[16][17];
+    const int c = threadIdx.x & 15, q = threadIdx.x >> 4, t = blockIdx.x * 16 + c;
+    double v = 0.0;
+    if (t < len)
+        for (int b = q; b < nblk; b += 16) v += part[(size_t)b * len + t];
+    s[q][c] = v;
+    __syncthreads();
+    if (q == 0 && t < len) {
+        double r = s[0][c];
+        for (int i = 1; i < 16; i++) r += s[i][c];
+        bins[t] = r;
+    }
 }
 
 // POTENTfft5's Green's function, PMP2main.f90:736-742, 805-816: the discrete
@@ -339,17 +376,22 @@ __global__ __launch_bounds__(256) void k_to_f64(const float* __restrict__ a, dou
 // POTENT_FOR_MG, PMP2main.f90:869-935: the REAL*4 potential (x fastest) plus
 // the scalar field's contribution at each cell, summed in FP64 and rounded
 // once, as FI = FI + sf does there
+// (one thread per pair of cells; 512^3: 387 us = 5.5 TB/s, one per cell 505)
 __global__ __launch_bounds__(256) void k_add_psi(float* __restrict__ phi, const double* __restrict__ u, Geo g,
-                                                 int model, int frn, double fct, double inv_ubg)
+                                                 int model, int frn, double fct, double inv_ubg, int TX, int TY,
+                                                 int XB, unsigned NB)
 {
-    const size_t n3 = 2 * g.half;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n3; q += stride) {
-        const int i = (int)(q % g.n);
-        const size_t r = q / g.n;
-        const int j = (int)(r % g.n), k = (int)(r / g.n);
-        phi[q] = (float)((double)phi[q] + psi_at(u, g, i, j, k, model, frn, fct, inv_ubg));
-    }
+    int m;
+    unsigned row;
+    if (!map_xy(g.h, (long)g.n * g.n, TX, TY, XB, NB, m, row)) return;
+    const int j = (int)(row % (unsigned)g.n), k = (int)(row / (unsigned)g.n);
+    size_t e, o;
+    pair_split(g, m, j, k, e, o);
+    Pair<float>* q = reinterpret_cast<Pair<float>*>(phi + ((size_t)row * g.n + 2 * (unsigned)m));
+    Pair<float> v = *q;
+    v.a = (float)((double)v.a + psi_of(u[e], model, frn, fct, inv_ubg));
+    v.b = (float)((double)v.b + psi_of(u[o], model, frn, fct, inv_ubg));
+    *q = v;
 }
 
 static dim3 grid_for(size_t count)
@@ -458,14 +500,15 @@ int mgs_fifth_force(mgs_handle* h, void* psi, void* gx, void* gy, void* gz, int3
     const double ctilde = 2.99792458e3 * (double)N / h->p.box;
     const double fct = ctilde * ctilde * 0.5 * fbg;
     prof_begin(h, MGS_KC_UPDATE, 0.0);
+    const ZLaunch L = make_zlaunch(make_geo(N));
     if (dtype == MGS_F32)
-        hipLaunchKernelGGL((k_fifth_force<float>), grid_for(n3), dim3(256), 0, h->s, h->L[0].u, (float*)dev[0],
+        hipLaunchKernelGGL((k_fifth_force<float>), L.grid, L.block, 0, h->s, h->L[0].u, (float*)dev[0],
                            (float*)dev[1], (float*)dev[2], (float*)dev[3], make_geo(N), h->p.model, h->p.fr_n, fct,
-                           1.0 / ubg);
+                           1.0 / ubg, L.TX, L.TY, L.XB, L.JB, L.KC, L.NB);
     else
-        hipLaunchKernelGGL((k_fifth_force<double>), grid_for(n3), dim3(256), 0, h->s, h->L[0].u, (double*)dev[0],
+        hipLaunchKernelGGL((k_fifth_force<double>), L.grid, L.block, 0, h->s, h->L[0].u, (double*)dev[0],
                            (double*)dev[1], (double*)dev[2], (double*)dev[3], make_geo(N), h->p.model, h->p.fr_n,
-                           fct, 1.0 / ubg);
+                           fct, 1.0 / ubg, L.TX, L.TY, L.XB, L.JB, L.KC, L.NB);
     prof_end(h);
     int rc = 0;
     if (where == MGS_HOST)
@@ -525,9 +568,10 @@ int mgs_power_spectrum_ex(mgs_handle* h, int32_t which, int32_t ipol, int32_t ic
         double ubg = 1.0;
         const double fbg = fr_background(h->p, &ubg);
         const double ctilde = 2.99792458e3 * (double)N / h->p.box;
-        hipLaunchKernelGGL((k_fifth_force<double>), grid_for(n3), dim3(256), 0, h->s, h->L[0].u, f->real,
+        const ZLaunch L = make_zlaunch(g);
+        hipLaunchKernelGGL((k_fifth_force<double>), L.grid, L.block, 0, h->s, h->L[0].u, f->real,
                            (double*)nullptr, (double*)nullptr, (double*)nullptr, g, h->p.model, h->p.fr_n,
-                           ctilde * ctilde * 0.5 * fbg, 1.0 / ubg);
+                           ctilde * ctilde * 0.5 * fbg, 1.0 / ubg, L.TX, L.TY, L.XB, L.JB, L.KC, L.NB);
     }
     if (hipfftExecD2Z(f->fwd, f->real, f->cplx) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecD2Z");
     const int nb = N / 2 + 1;  // bins 1..N/2 are returned
@@ -543,7 +587,7 @@ int mgs_power_spectrum_ex(mgs_handle* h, int32_t which, int32_t ipol, int32_t ic
     else
         hipLaunchKernelGGL((ipol ? k_bin_power<1, 0, false> : k_bin_power<0, 0, false>), G, B, lds, h->s, f->cplx, N,
                            norm, (const int*)f->logbin, f->binpart, nb);
-    hipLaunchKernelGGL(k_bin_reduce, dim3((6 * nb + 255) / 256), dim3(256), 0, h->s, (const double*)f->binpart,
+    hipLaunchKernelGGL(k_bin_reduce, dim3((6 * nb + 15) / 16), dim3(256), 0, h->s, (const double*)f->binpart,
                        BIN_BLOCKS, 6 * nb, f->bins);
     std::vector<double> hb(6 * (size_t)nb);
     if (hipMemcpyAsync(hb.data(), f->bins, hb.size() * sizeof(double), hipMemcpyDeviceToHost, h->s) != hipSuccess ||
@@ -617,8 +661,9 @@ int mgs_potential_add_fifth_force(mgs_handle* h)
     const double fbg = fr_background(h->p, &ubg);
     const double ctilde = 2.99792458e3 * (double)N / h->p.box;
     prof_begin(h, MGS_KC_PM, 16.0 * (double)n3);
-    hipLaunchKernelGGL(k_add_psi, grid_for(n3), dim3(256), 0, h->s, phi, h->L[0].u, make_geo(N), h->p.model,
-                       h->p.fr_n, ctilde * ctilde * 0.5 * fbg, 1.0 / ubg);
+    const Launch L = make_launch(N / 2, (long)N * N);
+    hipLaunchKernelGGL(k_add_psi, L.grid, L.block, 0, h->s, phi, h->L[0].u, make_geo(N), h->p.model, h->p.fr_n,
+                       ctilde * ctilde * 0.5 * fbg, 1.0 / ubg, L.TX, L.TY, L.XB, L.NB);
     prof_end(h);
     if (hipStreamSynchronize(h->s) != hipSuccess) return set_err(h, MGS_E_HIP, "fifth-force potential");
     return 0;
