@@ -554,12 +554,57 @@ static int cycle_plain(mgs_handle* h, int l, int kind)
 // ---------------------------------------------------------------------------
 // mixed precision: FP32 delta-form FAS V-cycle (inner) and FP64 outer loop
 // ---------------------------------------------------------------------------
+static int vcycle_inner(mgs_handle* h, int l, bool first = false, bool last = false);
+
+// The inner V-cycle on level l >= 1 from what the restriction left there (R d
+// in rd and d, R r in rres): the right-hand side f = D(R d) - R r and the
+// cycle.  *dH: the array that then holds the level's increment.  Small levels
+// run in one launch (the tail), the ones above them in one launch per half,
+// the others operation by operation; the values are the same.
+static int cycle_from_restricted(mgs_handle* h, int l, const float** dH)
+{
+    const int frn = h->p.fr_n;
+    LevelF& v = h->M[l];
+    const DfCoef dc = df_coefs(h->p, l);
+    *dH = v.d;
+    if (l < h->lc && v.n <= h->tail_n && h->use_tail) {
+        TailLevelIn lv[16];
+        const int nlev = h->lc - l + 1;
+        for (int i = 0; i < nlev && i < 16; i++) {
+            const LevelF& m = h->M[l + i];
+            lv[i] = TailLevelIn{m.n, m.d, m.xb, m.f, m.rres, m.rd, df_coefs(h->p, l + i)};
+        }
+        prof_begin(h, MGS_KC_COARSE, 13.0 * n3d(v.n) * 4.0);
+        const bool ok = launch_df_tail(frn, nlev, lv, h->s);
+        prof_end(h);
+        if (ok) return 0;
+    }
+    if (l < h->lc && df_block_level(v.n) && h->sweeps1[0] == 2 && h->sweeps1[1] == 2) {
+        LevelF& c = h->M[l + 1];
+        prof_begin(h, MGS_KC_COARSE, (5.0 * n3d(v.n) + 3.0 * n3d(c.n)) * 4.0);
+        launch_df_block_down(frn, v.rd, v.rres, v.xb, v.d, v.f, c.rres, c.rd, c.d, v.n, dc, h->s);
+        prof_end(h);
+        const float* cH = nullptr;
+        const int rc = cycle_from_restricted(h, l + 1, &cH);
+        if (rc) return rc;
+        prof_begin(h, MGS_KC_COARSE, (4.0 * n3d(v.n) + 2.0 * n3d(c.n)) * 4.0);
+        launch_df_block_up(frn, cH, c.rd, v.d, v.xb, v.f, v.res, v.n, dc, h->s);
+        prof_end(h);
+        *dH = v.res;
+        return 0;
+    }
+    prof_begin(h, MGS_KC_COARSE, 4.0 * n3d(v.n) * 4.0);
+    launch_df_rhs(frn, v.rd, v.xb, v.rres, v.f, v.n, dc, h->s);
+    prof_end(h);
+    return vcycle_inner(h, l);
+}
+
 // One inner V-cycle at level l: V(sweeps0) on level 0, V(sweeps1) below.  On
 // level 0, `first` means colour 0 of d was set by the fused outer residual
 // (relaxed once from zero: that pass is skipped, and colour 1, not written
 // there, is set by the colour-1 pass that follows) and `last` fuses the final
 // colour-1 pass with the outer update of u.
-static int vcycle_inner(mgs_handle* h, int l, bool first = false, bool last = false)
+static int vcycle_inner(mgs_handle* h, int l, bool first, bool last)
 {
     const int frn = h->p.fr_n;
     LevelF& v = h->M[l];
@@ -570,19 +615,6 @@ static int vcycle_inner(mgs_handle* h, int l, bool first = false, bool last = fa
         launch_df_coarsest(frn, v.d, v.xb, v.f, v.n, 8, dc, h->s);
         prof_end(h);
         return 0;
-    }
-    if (l > 0 && v.n <= h->tail_n && h->use_tail) {
-        // the small levels in one launch
-        TailLevelIn lv[16];
-        const int nlev = h->lc - l + 1;
-        for (int i = 0; i < nlev && i < 16; i++) {
-            const LevelF& m = h->M[l + i];
-            lv[i] = TailLevelIn{m.n, m.d, m.xb, m.f, m.rres, m.rd, df_coefs(h->p, l + i)};
-        }
-        prof_begin(h, MGS_KC_COARSE, 12.0 * n3d(v.n) * 4.0);
-        const bool ok = launch_df_tail(frn, nlev, lv, h->s);
-        prof_end(h);
-        if (ok) return 0;
     }
     const double s = 4.0;
     const int npre = l == 0 ? h->sweeps0[0] : h->sweeps1[0];
@@ -595,20 +627,18 @@ static int vcycle_inner(mgs_handle* h, int l, bool first = false, bool last = fa
     prof_begin(h, l == 0 ? MGS_KC_RESTRICT : MGS_KC_COARSE, (3.0 * n3d(v.n) + 3.0 * n3d(c.n)) * s);
     launch_df_restrict_residual(frn, v.d, v.xb, v.f, c.rres, c.rd, c.d, v.n, dc, h->s);
     prof_end(h);
-    auto coarse = [h, l, frn, &c]() {
-        prof_begin(h, MGS_KC_COARSE, 4.0 * n3d(c.n) * 4.0);
-        launch_df_rhs(frn, c.rd, c.xb, c.rres, c.f, c.n, df_coefs(h->p, l + 1), h->s);
-        prof_end(h);
-        return vcycle_inner(h, l + 1);
-    };
+    const float* cH = c.d;
     if (l == 0) {
-        int rc = run_captured(h, &h->g_inner, coarse);
+        // (a replayed graph leaves the increment where its capture said)
+        int rc = run_captured(h, &h->g_inner, [h]() { return cycle_from_restricted(h, 1, &h->inner_dH); });
         if (rc) return rc;
+        cH = h->inner_dH;
     } else {
-        coarse();
+        int rc = cycle_from_restricted(h, l + 1, &cH);
+        if (rc) return rc;
     }
     prof_begin(h, l == 0 ? MGS_KC_CORRECT : MGS_KC_COARSE, (3.0 * n3d(v.n) + 2.0 * n3d(c.n)) * s);
-    launch_df_correct(frn, c.d, c.rd, v.d, v.xb, c.n, h->s);
+    launch_df_correct(frn, cH, c.rd, v.d, v.xb, c.n, h->s);
     prof_end(h);
     const int nps = l == 0 ? h->sweeps0[1] : h->sweeps1[1];
     const int npost = (l == 0 && last) ? 2 * nps - 1 : 2 * nps;
@@ -857,13 +887,19 @@ static int df_cgc(mgs_handle* h, int l, int kind)
     prof_begin(h, cls, (3.0 * n3d(v.n) + 3.0 * n3d(c.n)) * 4.0);
     launch_df_restrict_residual(frn, v.d, v.xb, v.f, c.rres, c.rd, c.d, v.n, df_coefs(h->p, l), h->s);
     prof_end(h);
-    prof_begin(h, MGS_KC_COARSE, 4.0 * n3d(c.n) * 4.0);
-    launch_df_rhs(frn, c.rd, c.xb, c.rres, c.f, c.n, df_coefs(h->p, l + 1), h->s);
-    prof_end(h);
-    const int rc = kind == 0 ? vcycle_inner(h, l + 1) : fw_inner(h, l + 1, kind, false, false);
+    const float* cH = c.d;
+    int rc;
+    if (kind == 0) {
+        rc = cycle_from_restricted(h, l + 1, &cH);
+    } else {
+        prof_begin(h, MGS_KC_COARSE, 4.0 * n3d(c.n) * 4.0);
+        launch_df_rhs(frn, c.rd, c.xb, c.rres, c.f, c.n, df_coefs(h->p, l + 1), h->s);
+        prof_end(h);
+        rc = fw_inner(h, l + 1, kind, false, false);
+    }
     if (rc) return rc;
     prof_begin(h, l == 0 ? MGS_KC_CORRECT : MGS_KC_COARSE, (3.0 * n3d(v.n) + 2.0 * n3d(c.n)) * 4.0);
-    launch_df_correct(frn, c.d, c.rd, v.d, v.xb, c.n, h->s);
+    launch_df_correct(frn, cH, c.rd, v.d, v.xb, c.n, h->s);
     prof_end(h);
     return 0;
 }

@@ -220,6 +220,19 @@ __device__ inline double block_sum(double v)
     return t;
 }
 
+// barrier of the workgroup, or (WAVE) of the calling wave alone: its LDS
+// accesses execute in order, so only the compiler has to keep theirs
+template <bool WAVE>
+__device__ __forceinline__ void group_sync()
+{
+    if constexpr (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
 // sum of p[lo, hi) by one block: thread t adds p[lo + t], p[lo + t + B], ...
 // (B = blockDim.x, a power of two <= 1024), then a tree over the block in
 // s[0..B); the result is s[0].  The order depends only on (lo, hi, B).

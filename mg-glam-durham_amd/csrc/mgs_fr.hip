@@ -300,9 +300,28 @@ __global__ __launch_bounds__(1024) void k_df_coarsest(float* __restrict__ d, con
 }
 
 template <int FRN>
-__global__ __launch_bounds__(1024) void k_df_tail(TailDesc T)
+__global__ __launch_bounds__(TAIL_THREADS) void k_df_tail(TailDesc T)
 {
     df_tail_vcycle<FRN>(T);
+}
+
+template <int FRN, int BX, int BY, int BZ, int NTHR>
+__global__ __launch_bounds__(NTHR) void k_df_block_down(const float* __restrict__ rd, const float* __restrict__ rres,
+                                                        const float* __restrict__ xb, float* __restrict__ d,
+                                                        float* __restrict__ f, float* __restrict__ rres1,
+                                                        float* __restrict__ rd1, float* __restrict__ d1, Geo g, Geo gc,
+                                                        DfCoef c)
+{
+    df_block_down<FRN, BX, BY, BZ, NTHR>(rd, rres, xb, d, f, rres1, rd1, d1, g, gc, c);
+}
+
+template <int FRN, int BX, int BY, int BZ, int NTHR>
+__global__ __launch_bounds__(NTHR) void k_df_block_up(const float* __restrict__ dH, const float* __restrict__ rdc,
+                                                      const float* __restrict__ d, const float* __restrict__ xb,
+                                                      const float* __restrict__ f, float* __restrict__ dout, Geo g,
+                                                      Geo gc, DfCoef c)
+{
+    df_block_up<FRN, BX, BY, BZ, NTHR>(dH, rdc, d, xb, f, dout, g, gc, c);
 }
 
 // ===========================================================================
@@ -660,6 +679,7 @@ bool launch_df_tail(int frn, int nlev, const TailLevelIn* lv, hipStream_t s)
     long lds = 0;  // the LDS copies: d, xb, g of the first level, d, xb, g, rres, rd below
     for (int i = 0; i < nlev; i++) lds += (i == 0 ? 3L : 5L) * lv[i].n * lv[i].n * lv[i].n;
     if (lds > TAIL_LDS_FLOATS) return false;
+    if ((long)lv[0].n * lv[0].n * lv[0].n > 2L * TAIL_CELLS * TAIL_THREADS) return false;
     TailDesc T;
     T.nl = nlev - 1;
     for (int i = 0; i < nlev; i++) {
@@ -671,10 +691,43 @@ bool launch_df_tail(int frn, int nlev, const TailLevelIn* lv, hipStream_t s)
         T.L[i].rd = lv[i].rd;
         T.L[i].dc = lv[i].dc;
     }
-    if (frn == 0) hipLaunchKernelGGL((k_df_tail<0>), dim3(1), dim3(1024), 0, s, T);
-    else if (frn == 1) hipLaunchKernelGGL((k_df_tail<1>), dim3(1), dim3(1024), 0, s, T);
-    else hipLaunchKernelGGL((k_df_tail<2>), dim3(1), dim3(1024), 0, s, T);
+    if (frn == 0) hipLaunchKernelGGL((k_df_tail<0>), dim3(1), dim3(TAIL_THREADS), 0, s, T);
+    else if (frn == 1) hipLaunchKernelGGL((k_df_tail<1>), dim3(1), dim3(TAIL_THREADS), 0, s, T);
+    else hipLaunchKernelGGL((k_df_tail<2>), dim3(1), dim3(TAIL_THREADS), 0, s, T);
     return true;
+}
+
+// (BX, BY, BZ, threads) tiles that cover a level of n cells a side
+#define DF_BLOCK_DISPATCH(KERNEL, n, ...)                                                                          \
+    do {                                                                                                           \
+        const unsigned nn = (unsigned)(n);                                                                         \
+        if (df_block_large(n)) {                                                                                   \
+            const dim3 G(nn / 16 * (nn / 8) * (nn / 8)), T(1024);                                                  \
+            if (frn == 0) hipLaunchKernelGGL((KERNEL<0, 16, 8, 8, 1024>), G, T, 0, s, __VA_ARGS__);                \
+            else if (frn == 1) hipLaunchKernelGGL((KERNEL<1, 16, 8, 8, 1024>), G, T, 0, s, __VA_ARGS__);           \
+            else hipLaunchKernelGGL((KERNEL<2, 16, 8, 8, 1024>), G, T, 0, s, __VA_ARGS__);                         \
+        } else {                                                                                                   \
+            const dim3 G(nn / 8 * (nn / 8) * (nn / 4)), T(512);                                                    \
+            if (frn == 0) hipLaunchKernelGGL((KERNEL<0, 8, 8, 4, 512>), G, T, 0, s, __VA_ARGS__);                  \
+            else if (frn == 1) hipLaunchKernelGGL((KERNEL<1, 8, 8, 4, 512>), G, T, 0, s, __VA_ARGS__);             \
+            else hipLaunchKernelGGL((KERNEL<2, 8, 8, 4, 512>), G, T, 0, s, __VA_ARGS__);                           \
+        }                                                                                                          \
+    } while (0)
+
+static bool df_block_large(int n) { return n > 40 && n % 16 == 0; }
+
+void launch_df_block_down(int frn, const float* rd, const float* rres, const float* xb, float* d, float* f,
+                          float* rres1, float* rd1, float* d1, int n, const DfCoef& c, hipStream_t s)
+{
+    const Geo g = make_geo(n), gc = make_geo(n / 2);
+    DF_BLOCK_DISPATCH(k_df_block_down, n, rd, rres, xb, d, f, rres1, rd1, d1, g, gc, c);
+}
+
+void launch_df_block_up(int frn, const float* dH, const float* rdc, const float* d, const float* xb, const float* f,
+                        float* dout, int n, const DfCoef& c, hipStream_t s)
+{
+    const Geo g = make_geo(n), gc = make_geo(n / 2);
+    DF_BLOCK_DISPATCH(k_df_block_up, n, dH, rdc, d, xb, f, dout, g, gc, c);
 }
 
 void launch_df_coarsest(int frn, float* d, const float* xb, const float* rhs, int n, int sweeps, const DfCoef& c,

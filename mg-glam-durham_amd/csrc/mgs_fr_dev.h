@@ -824,39 +824,116 @@ __device__ __forceinline__ void df_correct_col(const float* __restrict__ dH, con
     }
 }
 
-// coarsest level: red-black sweeps of the delta-form smoother in FP64 by one
-// workgroup (the level holds at most a few thousand cells)
+// x = w^{1/(n+1)} and 1/x in FP64, w > 0, to a few times 1e-16: for n = 1 both
+// from the hardware's reciprocal square root refined once
 template <int FRN>
+__device__ __forceinline__ void xroot_rcp64(double w, double& x, double& rx)
+{
+    if constexpr (FRN == 1) {
+        double y = __builtin_amdgcn_rsq(w);
+        y = __builtin_fma(0.5 * y, __builtin_fma(-w * y, y, 1.0), y);
+        rx = y;
+        x = w * y;
+    } else {
+        x = xroot<FRN>(w);
+        rx = rcp64(x);
+    }
+}
+
+// Newton's method in FP64 on D(d) = r at one cell from d = dl, with neighbour
+// sum S.  A step of relative length s leaves a relative error of order s^2
+// d / xb^{n+1}, so a step below 1e-6 d leaves one far below the FP32 rounding
+// the result is stored with.  Reciprocals are the hardware's refined once
+// (relative error about 1e-15).  The coarsest level is a chain of such
+// solves: with four divisions and a square root per step, iterated to
+// 1e-15, the 2^3 level took 10 us of each V-cycle.
+template <int FRN>
+__device__ __forceinline__ double df_newton64(double dl, double S, double xbc, double wb, double rxb, double r,
+                                              const DfCoef& c)
+{
+    for (int it = 0; it < 30; it++) {
+        double x, rx;
+        xroot_rcp64<FRN>(fmax(wb + dl, 1.0e-300), x, rx);
+        const double F = c.A64 * (S - 6.0 * dl) + c.C64 * dl * rcp64(dden<FRN>(x, xbc)) * (rx * rxb) - r;
+        const double Fp = -6.0 * c.A64 + c.C64 * (1.0 / (double)(FRN + 1)) * rx * wpow<FRN>(rx);
+        double dn = dl - F * rcp64(Fp);
+        if (!(wb + dn > 0.0)) dn = 0.5 * (dl - wb);  // halve the distance to x = 0
+        const bool done = fabs(dn - dl) <= 1.0e-6 * fabs(dn);
+        dl = dn;
+        if (done) break;
+    }
+    return dl;
+}
+
+// (m, j, k) of entry t of a colour half.  The side of a level is a power of
+// two times a small odd number, mostly 1: shifts then, instead of four
+// divisions by a number unknown at compile time, whose chain is as long as a
+// cell update on the levels one workgroup runs.
+__device__ __forceinline__ void half_mjk(const Geo& g, int t, int& m, int& j, int& k)
+{
+    if ((g.n & (g.n - 1)) == 0) {
+        const int lg = 31 - __builtin_clz((unsigned)g.n);
+        m = t & (g.h - 1);
+        j = (t >> (lg - 1)) & (g.n - 1);
+        k = t >> (2 * lg - 1);
+    } else {
+        m = t % g.h;
+        const int row = t / g.h;
+        j = row % g.n;
+        k = row / g.n;
+    }
+}
+
+// the six neighbours' offsets and its own of entry t of a colour half
+__device__ __forceinline__ Nb half_cell(const Geo& g, int colour, int t)
+{
+    int m, j, k;
+    half_mjk(g, t, m, j, k);
+    return neighbours(g, colour, m, j, k);
+}
+
+template <int FRN>
+__device__ __forceinline__ float df_coarsest_cell(const float* d, const Nb& q, double xbc, double rhs, const DfCoef& c)
+{
+    const double S = (((double)d[q.xp] + d[q.xm]) + ((double)d[q.yp] + d[q.ym])) + ((double)d[q.zp] + d[q.zm]);
+    return (float)df_newton64<FRN>(d[q.me], S, xbc, wpow<FRN>(xbc), rcp64(xbc), rhs, c);
+}
+
+// coarsest level: red-black sweeps of the delta-form smoother in FP64 by one
+// workgroup (the level holds at most a few thousand cells), or, with WAVE,
+// by its first wave alone (the others do not call it)
+template <int FRN, bool WAVE = false>
 __device__ __forceinline__ void df_coarsest_block(float* __restrict__ d, const float* __restrict__ xb,
                                                   const float* __restrict__ rhs, const Geo& g, int sweeps,
                                                   const DfCoef& c)
 {
+    const int nthr = WAVE ? 64 : (int)blockDim.x, tid = threadIdx.x, half = (int)g.half;
+    if (half <= nthr) {  // a thread's cell of each colour is the same in every sweep
+        Nb q[2];
+        double xbc[2] = {1.0, 1.0}, r[2] = {0.0, 0.0};
+        if (tid < half)
+#pragma unroll
+            for (int colour = 0; colour < 2; colour++) {
+                q[colour] = half_cell(g, colour, tid);
+                xbc[colour] = xb[q[colour].me];
+                r[colour] = rhs[q[colour].me];
+            }
+        for (int sw = 0; sw < sweeps; sw++) {
+#pragma unroll
+            for (int colour = 0; colour < 2; colour++) {
+                if (tid < half) d[q[colour].me] = df_coarsest_cell<FRN>(d, q[colour], xbc[colour], r[colour], c);
+                group_sync<WAVE>();
+            }
+        }
+        return;
+    }
     for (int sw = 0; sw < sweeps; sw++) {
         for (int colour = 0; colour < 2; colour++) {
-            for (int t = threadIdx.x; t < (int)g.half; t += blockDim.x) {
-                const int m = t % g.h;
-                const int row = t / g.h;
-                const int j = row % g.n, k = row / g.n;
-                const Nb q = neighbours(g, colour, m, j, k);
-                const double S = (double)d[q.xp] + d[q.xm] + d[q.yp] + d[q.ym] + d[q.zp] + d[q.zm];
-                const double xbc = xb[q.me];
-                const double wb = wpow<FRN>(xbc);
-                const double r = rhs[q.me];
-                // Newton on the increment in FP64 from the current value
-                double dl = d[q.me];
-                for (int it = 0; it < 30; it++) {
-                    double x = xroot<FRN>(fmax(wb + dl, 1.0e-300));
-                    const double F = c.A64 * (S - 6.0 * dl) + dlocal<FRN>(dl, x, xbc, c.C64) - r;
-                    const double Fp = -6.0 * c.A64 + c.C64 / ((double)(FRN + 1) * x * wpow<FRN>(x));
-                    double dn = dl - F / Fp;
-                    if (!(wb + dn > 0.0)) dn = 0.5 * (dl - wb);  // halve the distance to x = 0
-                    const bool done = fabs(dn - dl) <= 1.0e-15 * (fabs(dn) + wb);
-                    dl = dn;
-                    if (done) break;
-                }
-                d[q.me] = (float)dl;
+            for (int t = tid; t < half; t += nthr) {
+                const Nb q = half_cell(g, colour, t);
+                d[q.me] = df_coarsest_cell<FRN>(d, q, xb[q.me], rhs[q.me], c);
             }
-            __syncthreads();
+            group_sync<WAVE>();
         }
     }
 }
@@ -893,6 +970,18 @@ __device__ __forceinline__ void restrict8_cell(const T* __restrict__ fine, T* __
 // the level kernels (a red-black pass, the restrictions and the
 // prolongation do not depend on the order cells are visited in), so the
 // results are identical to the launch-per-operation cycle.
+//
+// The tail runs out of LDS: the first level's R d, R r and xb and every
+// coarser level's xb are copied in, the cycle (from the first level's
+// right-hand side f = D(R d) - R r on) works on the LDS copies, and the first
+// level's d is copied back; coarser levels are internal to the cycle.  The
+// launcher checks that the levels fit in TAIL_LDS_FLOATS and TAIL_CELLS.
+//
+// What bounds it is one CU's issue rate on the 16^3 passes (2048 cells of
+// about 110 instructions each) and the chain of barriers and latencies
+// below.  A thread therefore keeps its cells' offsets, xb and f in registers
+// for the four passes of a block, and levels of at most TAIL_WAVE_HALF cells
+// a colour run in the first wave without barriers.  TAIL_FIGURES
 // ---------------------------------------------------------------------------
 struct TailLevel {
     Geo g;
@@ -905,33 +994,20 @@ constexpr int TAIL_MAX_N = 16;  // levels with n <= 16 run in the tail
 // LDS for the tail's arrays: d, xb, g of its first level and d, xb, g, rres,
 // rd of each coarser one (15208 floats for 16^3 down to 2^3)
 constexpr int TAIL_LDS_FLOATS = 15232;
+constexpr int TAIL_THREADS = 1024;
+constexpr int TAIL_CELLS = 2;         // cells of one colour per thread: half <= TAIL_CELLS * TAIL_THREADS
+constexpr int TAIL_WAVE_HALF = 128;   // levels with half at most this (2 cells per lane) run in one wave
 
 struct TailDesc {
     int nl;  // levels below the first (L[nl] is the coarsest)
     TailLevel L[TAIL_MAXL];
 };
 
-// cell t of a colour half -> the six neighbours' offsets and its own
-__device__ __forceinline__ Nb tail_cell(const Geo& g, int colour, int t)
-{
-    const int m = t % g.h, row = t / g.h;
-    return neighbours(g, colour, m, row % g.n, row / g.n);
-}
-
-template <class OP>
-__device__ __forceinline__ void tail_update(const OP& op, const Geo& g, int colour, int t)
-{
-    const Nb q = tail_cell(g, colour, t);
-    const auto* a = op.field();
-    const unsigned oo = q.me + (colour ? 0u - (unsigned)g.half : (unsigned)g.half);
-    op.update(q.me, oo, op.load(q.me, oo), a[oo], a[q.xp], a[q.xm], a[q.yp], a[q.ym], a[q.zp], a[q.zm]);
-}
-
 template <class OP>
 __device__ __forceinline__ void tail_cell_op(const OP& op, const Geo& g, int t)
 {
     const int colour = t >= (int)g.half ? 1 : 0;
-    const Nb q = tail_cell(g, colour, t - colour * (int)g.half);
+    const Nb q = half_cell(g, colour, t - colour * (int)g.half);
     const auto* a = op.field();
     (void)op.cell(q.me, op.load(q.me), a[q.me], a[q.xp], a[q.xm], a[q.yp], a[q.ym], a[q.zp], a[q.zm]);
 }
@@ -939,16 +1015,18 @@ __device__ __forceinline__ void tail_cell_op(const OP& op, const Geo& g, int t)
 __device__ __forceinline__ void coarse_ijk(const Geo& gc, int t, int& I, int& J, int& K)
 {
     const unsigned n = (unsigned)gc.n;
+    if ((n & (n - 1)) == 0) {
+        const int lg = 31 - __builtin_clz(n);
+        I = t & (int)(n - 1);
+        J = (t >> lg) & (int)(n - 1);
+        K = t >> (2 * lg);
+        return;
+    }
     I = (int)((unsigned)t % n);
     J = (int)(((unsigned)t / n) % n);
     K = (int)((unsigned)t / (n * n));
 }
 
-// The tail runs out of LDS: the first level's d, xb and g and every coarser
-// level's xb are copied in, the cycle works on the LDS copies (the arithmetic
-// and its order are those of the level kernels), and the first level's d is
-// copied back; coarser levels are internal to the cycle.  The launcher checks
-// that the levels fit in TAIL_LDS_FLOATS.
 struct TailArrays {
     float *d, *xb, *f, *rres, *rd;
 };
@@ -964,45 +1042,73 @@ __device__ __forceinline__ TailArrays tail_lds_level(const TailDesc& G, int i, f
     return TailArrays{p, p + cells, p + 2 * cells, i > 0 ? p + 3 * cells : nullptr, i > 0 ? p + 4 * cells : nullptr};
 }
 
-template <int FRN>
-__device__ void df_tail_vcycle(const TailDesc& G)
+// two red-black pairs on a level; each thread's cells, at most TAIL_CELLS per
+// colour, are the same in every pass
+template <int FRN, bool WAVE>
+__device__ __forceinline__ void tail_smooth2(const TailLevel& L, const TailArrays& l)
 {
-    __shared__ float lds[TAIL_LDS_FLOATS];
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    for (int i = 0; i <= G.nl; i++) {
-        const TailArrays A = tail_lds_level(G, i, lds);
-        const int cells = G.L[i].g.n * G.L[i].g.n * G.L[i].g.n;
-        for (int t = tid; t < cells; t += nthr) A.xb[t] = G.L[i].xb[t];
-        if (i == 0)
-            for (int t = tid; t < cells; t += nthr) {
-                A.d[t] = G.L[0].d[t];
-                A.f[t] = G.L[0].f[t];
-            }
-    }
-    __syncthreads();
-    for (int i = 0; i < G.nl; i++) {
-        const TailLevel &L = G.L[i], &C = G.L[i + 1];
-        const TailArrays l = tail_lds_level(G, i, lds), c = tail_lds_level(G, i + 1, lds);
-        for (int it = 0; it < 4; it++) {
-            for (int t = tid; t < (int)L.g.half; t += nthr)
-                tail_update(DfSmoothOp<FRN>{l.d, l.xb, l.f, L.dc}, L.g, it & 1, t);
-            __syncthreads();
+    const int tid = threadIdx.x, nthr = WAVE ? 64 : TAIL_THREADS, half = (int)L.g.half;
+    Nb q[2][TAIL_CELLS];
+    float xb[2][TAIL_CELLS], f[2][TAIL_CELLS];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int r = 0; r < TAIL_CELLS; r++) {
+            const int t = tid + r * nthr;
+            if (t >= half) continue;
+            q[c][r] = half_cell(L.g, c, t);
+            xb[c][r] = l.xb[q[c][r].me];
+            f[c][r] = l.f[q[c][r].me];
         }
+    for (int pair = 0; pair < 2; pair++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+#pragma unroll
+            for (int r = 0; r < TAIL_CELLS; r++) {
+                if (tid + r * nthr >= half) continue;
+                const Nb& b = q[c][r];
+                const float S = l.d[b.xp] + l.d[b.xm] + l.d[b.yp] + l.d[b.ym] + l.d[b.zp] + l.d[b.zm];
+                l.d[b.me] = df_solve<FRN>(S, xb[c][r], f[c][r], L.dc);
+            }
+            group_sync<WAVE>();
+        }
+}
+
+// the cycle from level i0 (its d and f in place) to the coarsest and back to
+// i0; with WAVE by the first wave alone
+template <int FRN, bool WAVE>
+__device__ void df_tail_levels(const TailDesc& G, int i0, float* lds)
+{
+    const int tid = threadIdx.x, nthr = WAVE ? 64 : TAIL_THREADS;
+    int bottom = G.nl;  // the levels from here on run elsewhere, or the coarsest
+    for (int i = i0; i < G.nl; i++) {
+        const TailLevel &L = G.L[i], &C = G.L[i + 1];
+        if (!WAVE && L.g.half <= TAIL_WAVE_HALF) {
+            bottom = i;
+            break;
+        }
+        const TailArrays l = tail_lds_level(G, i, lds), c = tail_lds_level(G, i + 1, lds);
+        tail_smooth2<FRN, WAVE>(L, l);
         const int ncc = C.g.n * C.g.n * C.g.n;
         for (int t = tid; t < ncc; t += nthr) {
             int I, J, K;
             coarse_ijk(C.g, t, I, J, K);
             df_restrict_residual_col<FRN>(l.d, l.xb, l.f, c.rres, c.rd, c.d, L.g, C.g, L.dc, ZCol{I, J, K, K + 1});
         }
-        __syncthreads();
+        group_sync<WAVE>();
         for (int t = tid; t < ncc; t += nthr) tail_cell_op(DfResOp<FRN>{c.rd, c.xb, c.rres, c.f, C.dc}, C.g, t);
-        __syncthreads();
+        group_sync<WAVE>();
     }
-    {
+    if (bottom < G.nl) {
+        if constexpr (!WAVE) {
+            if (tid < 64) df_tail_levels<FRN, true>(G, bottom, lds);
+            __syncthreads();
+        }
+    } else {
         const TailArrays b = tail_lds_level(G, G.nl, lds);
-        df_coarsest_block<FRN>(b.d, b.xb, b.f, G.L[G.nl].g, 8, G.L[G.nl].dc);
+        df_coarsest_block<FRN, WAVE>(b.d, b.xb, b.f, G.L[G.nl].g, 8, G.L[G.nl].dc);
     }
-    for (int i = G.nl - 1; i >= 0; i--) {
+    for (int i = bottom - 1; i >= i0; i--) {
         const TailLevel &L = G.L[i], &C = G.L[i + 1];
         const TailArrays l = tail_lds_level(G, i, lds), c = tail_lds_level(G, i + 1, lds);
         const int ncc = C.g.n * C.g.n * C.g.n;
@@ -1011,16 +1117,247 @@ __device__ void df_tail_vcycle(const TailDesc& G)
             coarse_ijk(C.g, t, I, J, K);
             df_correct_col<FRN>(c.d, c.rd, l.d, l.xb, L.g, C.g, ZCol{I, J, K, K + 1});
         }
-        __syncthreads();
-        for (int it = 0; it < 4; it++) {
-            for (int t = tid; t < (int)L.g.half; t += nthr)
-                tail_update(DfSmoothOp<FRN>{l.d, l.xb, l.f, L.dc}, L.g, it & 1, t);
-            __syncthreads();
-        }
+        group_sync<WAVE>();
+        tail_smooth2<FRN, WAVE>(L, l);
     }
+}
+
+template <int FRN>
+__device__ void df_tail_vcycle(const TailDesc& G)
+{
+    __shared__ float lds[TAIL_LDS_FLOATS];
+    const int tid = threadIdx.x, nthr = TAIL_THREADS;
+    // every load issued before the first is used: one memory latency instead
+    // of one per level and array
+    constexpr int NR = 2 * TAIL_CELLS;
+    float v[3][NR], vc[TAIL_MAXL];
+    const int c0 = 2 * (int)G.L[0].g.half;
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const int t = tid + r * nthr;
+        if (t >= c0) continue;
+        v[0][r] = G.L[0].xb[t];
+        v[1][r] = G.L[0].rd[t];
+        v[2][r] = G.L[0].rres[t];
+    }
+#pragma unroll
+    for (int i = 1; i < TAIL_MAXL; i++)  // at most 8^3 cells
+        if (i <= G.nl && tid < 2 * (int)G.L[i].g.half) vc[i] = G.L[i].xb[tid];
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const int t = tid + r * nthr;
+        if (t >= c0) continue;
+        lds[c0 + t] = v[0][r];
+        lds[t] = v[1][r];
+        lds[2 * c0 + t] = v[2][r];
+    }
+#pragma unroll
+    for (int i = 1; i < TAIL_MAXL; i++)
+        if (i <= G.nl && tid < 2 * (int)G.L[i].g.half) tail_lds_level(G, i, lds).xb[tid] = vc[i];
+    __syncthreads();
     const TailArrays a0 = tail_lds_level(G, 0, lds);
     const int cells0 = G.L[0].g.n * G.L[0].g.n * G.L[0].g.n;
+    // the right-hand side in place of R r (a cell reads only its own)
+    for (int t = tid; t < cells0; t += nthr)
+        tail_cell_op(DfResOp<FRN>{a0.d, a0.xb, a0.f, a0.f, G.L[0].dc}, G.L[0].g, t);
+    __syncthreads();
+    df_tail_levels<FRN, false>(G, 0, lds);
     for (int t = tid; t < cells0; t += nthr) G.L[0].d[t] = a0.d[t];
+}
+
+// ---------------------------------------------------------------------------
+// Half an inner V-cycle's work on one level in one launch, for the levels
+// between the tail and those large enough to keep the GPU busy (n <= 64).  A
+// pass of such a level is one launch of 2.5 to 4 us, nearly all of it launch,
+// drain and memory latency, and a cycle has eleven per level.  Here a block
+// owns a tile of cells, reads it with a halo into LDS, and runs the four
+// colour passes on shrinking boxes, recomputing in the halo what its
+// neighbours compute too: the same arithmetic per cell on the same inputs, so
+// the results are bit-identical to the passes' launches.
+//
+// Halos: a pass needs the other colour one cell further out than it writes.
+// The descending half writes the tile and the cells around it (the restricted
+// residual reads one more), so its passes run at 4, 3, 2, 1 cells beyond the
+// tile and d is read at 5; the ascending half's at 3, 2, 1, 0 with the
+// corrected d at 4.
+//
+// Tiles: 8 x 8 x 4 on 32^3 (128 blocks), 16 x 8 x 8 on 64^3 (256 blocks), the
+// largest that give every second CU or every CU a block: the halo makes the
+// passes 6.6 and 3.7 times the tile's own.  32^3: 10 us down and 7.5 up, where
+// six and five launches took 32 and 20; 64^3 (with single-plane launches
+// otherwise): 17 and 12, where they took 24 and 17.  At 128^3 the launches are
+// long enough and the halo work is not.
+// ---------------------------------------------------------------------------
+template <int BX_, int BY_, int BZ_, int H_>
+struct DfBox {
+    static constexpr int BX = BX_, BY = BY_, BZ = BZ_, H = H_;
+    static constexpr int LX = BX + 2 * H, LY = BY + 2 * H, LZ = BZ + 2 * H, CELLS = LX * LY * LZ;
+    static constexpr int SY = LX, SZ = LX * LY;
+    int x0, y0, z0;  // the tile's first cell (even)
+
+    // block b of the level's tiles, x fastest
+    __device__ __forceinline__ void init(int n, unsigned b)
+    {
+        const unsigned tx = (unsigned)(n / BX), ty = (unsigned)(n / BY);
+        x0 = (int)(b % tx) * BX;
+        y0 = (int)((b / tx) % ty) * BY;
+        z0 = (int)(b / (tx * ty)) * BZ;
+    }
+    static __device__ __forceinline__ int wrap(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
+    // offset on the level of box cell (x, y, z), coordinates from the tile's first cell
+    __device__ __forceinline__ unsigned global(const Geo& g, int x, int y, int z) const
+    {
+        return sidx(g, wrap(x0 + x, g.n), wrap(y0 + y, g.n), wrap(z0 + z, g.n));
+    }
+    static __device__ __forceinline__ int local(int x, int y, int z) { return ((z + H) * LY + (y + H)) * LX + (x + H); }
+};
+
+// f(i, x, y, z) for every cell of the box reaching R cells beyond the tile
+template <class BOX, int R, int NTHR, class F>
+__device__ __forceinline__ void box_each(F f)
+{
+    constexpr int EX = BOX::BX + 2 * R, EY = BOX::BY + 2 * R, EZ = BOX::BZ + 2 * R;
+    // unrolled: the loads of all turns are then in flight together
+#pragma unroll
+    for (int t0 = 0; t0 < EX * EY * EZ; t0 += NTHR) {
+        const int t = t0 + (int)threadIdx.x;
+        if (t0 + NTHR > EX * EY * EZ && t >= EX * EY * EZ) break;
+        const int x = t % EX - R, y = (t / EX) % EY - R, z = t / (EX * EY) - R;
+        f(BOX::local(x, y, z), x, y, z);
+    }
+}
+
+// one colour pass over the box reaching R cells beyond the tile (the tile's
+// first cell is even, so colours are those of the box coordinates)
+template <int FRN, class BOX, int R>
+__device__ __forceinline__ void box_pass(int nthr, int colour, float* d, const float* xb, const float* f, const DfCoef& c)
+{
+    constexpr int EX = (BOX::BX + 2 * R) / 2, EY = BOX::BY + 2 * R, EZ = BOX::BZ + 2 * R;
+    for (int t = threadIdx.x; t < EX * EY * EZ; t += nthr) {
+        const int y = (t / EX) % EY - R, z = t / (EX * EY) - R;
+        const int x = 2 * (t % EX) - R + ((colour + R + y + z) & 1);
+        const int i = BOX::local(x, y, z);
+        const float S = d[i + 1] + d[i - 1] + d[i + BOX::SY] + d[i - BOX::SY] + d[i + BOX::SZ] + d[i - BOX::SZ];
+        d[i] = df_solve<FRN>(S, xb[i], f[i], c);
+    }
+    __syncthreads();
+}
+
+// Descending half: d = R d, f = D(R d) - R r, two red-black pairs, d and f
+// stored for the ascending half, and the residual and d restricted
+// (df_restrict_residual_col's sums in its order).
+template <int FRN, int BX, int BY, int BZ, int NTHR>
+__device__ __forceinline__ void df_block_down(const float* __restrict__ rd, const float* __restrict__ rres,
+                                              const float* __restrict__ xbg, float* __restrict__ dg,
+                                              float* __restrict__ fg, float* __restrict__ rres1,
+                                              float* __restrict__ rd1, float* __restrict__ d1, const Geo& g,
+                                              const Geo& gc, const DfCoef& c)
+{
+    using BOX = DfBox<BX, BY, BZ, 5>;
+    __shared__ float d[BOX::CELLS], xb[BOX::CELLS], f[BOX::CELLS];
+    BOX B;
+    B.init(g.n, blockIdx.x);
+    box_each<BOX, 5, NTHR>([&](int i, int x, int y, int z) {
+        const unsigned o = B.global(g, x, y, z);
+        d[i] = elem(rd, o);
+        xb[i] = elem(xbg, o);
+        f[i] = elem(rres, o);
+    });
+    __syncthreads();
+    box_each<BOX, 4, NTHR>([&](int i, int, int, int) {
+        const DfResOp<FRN> op{d, xb, f, f, c};
+        (void)op.cell((unsigned)i, typename DfResOp<FRN>::Own{xb[i], f[i]}, d[i], d[i + 1], d[i - 1], d[i + BOX::SY],
+                      d[i - BOX::SY], d[i + BOX::SZ], d[i - BOX::SZ]);
+    });
+    __syncthreads();
+    box_pass<FRN, BOX, 4>(NTHR, 0, d, xb, f, c);
+    box_pass<FRN, BOX, 3>(NTHR, 1, d, xb, f, c);
+    box_pass<FRN, BOX, 2>(NTHR, 0, d, xb, f, c);
+    box_pass<FRN, BOX, 1>(NTHR, 1, d, xb, f, c);
+    // the tile out, and each child's local term less its right-hand side in f's place
+    box_each<BOX, 0, NTHR>([&](int i, int x, int y, int z) {
+        const unsigned o = B.global(g, x, y, z);
+        const float dc = d[i], xbc = xb[i], fv = f[i];
+        elem(dg, o) = dc;
+        elem(fg, o) = fv;
+        const float xr = xroot<FRN>(fmaxf(wpow<FRN>(xbc) + dc, 1.0e-30f));
+        f[i] = dlocal<FRN>(dc, xr, xbc, c.C) - fv;
+    });
+    __syncthreads();
+    constexpr int CX = BX / 2, CY = BY / 2, CZ = BZ / 2, SY = BOX::SY, SZ = BOX::SZ;
+    for (int t = threadIdx.x; t < CX * CY * CZ; t += NTHR) {
+        const int I = t % CX, J = (t / CX) % CY, K = t / (CX * CY);
+        const int i = BOX::local(2 * I, 2 * J, 2 * K);
+        const int ch[8] = {0, 1, SY, SY + 1, SZ, SZ + 1, SZ + SY, SZ + SY + 1};
+        float loc = 0.0f, s8 = d[i];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            loc += f[i + ch[q]];
+            if (q > 0) s8 += d[i + ch[q]];
+        }
+        float outer = d[i - 1] + d[i + SY - 1] + d[i + SZ - 1] + d[i + SZ + SY - 1];
+        outer += d[i + 2] + d[i + SY + 2] + d[i + SZ + 2] + d[i + SZ + SY + 2];
+        outer += d[i - SY] + d[i - SY + 1] + d[i + SZ - SY] + d[i + SZ - SY + 1];
+        outer += d[i + 2 * SY] + d[i + 2 * SY + 1] + d[i + SZ + 2 * SY] + d[i + SZ + 2 * SY + 1];
+        outer += d[i - SZ] + d[i - SZ + 1] + d[i - SZ + SY] + d[i - SZ + SY + 1];
+        outer += d[i + 2 * SZ] + d[i + 2 * SZ + 1] + d[i + 2 * SZ + SY] + d[i + 2 * SZ + SY + 1];
+        const unsigned oc = sidx(gc, B.x0 / 2 + I, B.y0 / 2 + J, B.z0 / 2 + K);
+        elem(rres1, oc) = (c.A * (outer - 3.0f * s8) + loc) * 0.125f;
+        const float rdv = s8 / 8.0f;
+        elem(rd1, oc) = rdv;
+        elem(d1, oc) = rdv;
+    }
+}
+
+// Ascending half: the coarse correction of the colour-1 cells (df_sons_new's
+// sums in its order) and two red-black pairs, into dout: a neighbour's halo
+// still reads d.
+template <int FRN, int BX, int BY, int BZ, int NTHR>
+__device__ __forceinline__ void df_block_up(const float* __restrict__ dH, const float* __restrict__ rdc,
+                                            const float* __restrict__ dg, const float* __restrict__ xbg,
+                                            const float* __restrict__ fg, float* __restrict__ dout, const Geo& g,
+                                            const Geo& gc, const DfCoef& c)
+{
+    using BOX = DfBox<BX, BY, BZ, 4>;
+    using CBOX = DfBox<BX / 2, BY / 2, BZ / 2, 3>;  // the coarse cells around the fine box
+    __shared__ float d[BOX::CELLS], xb[BOX::CELLS], f[BOX::CELLS], e[CBOX::CELLS];
+    BOX B;
+    B.init(g.n, blockIdx.x);
+    CBOX C;
+    C.x0 = B.x0 / 2;
+    C.y0 = B.y0 / 2;
+    C.z0 = B.z0 / 2;
+    box_each<CBOX, 3, NTHR>([&](int i, int x, int y, int z) {
+        const unsigned o = C.global(gc, x, y, z);
+        e[i] = elem(dH, o) - elem(rdc, o);
+    });
+    box_each<BOX, 4, NTHR>([&](int i, int x, int y, int z) {
+        const unsigned o = B.global(g, x, y, z);
+        d[i] = elem(dg, o);
+        xb[i] = elem(xbg, o);
+        f[i] = elem(fg, o);
+    });
+    __syncthreads();
+    box_each<BOX, 4, NTHR>([&](int i, int x, int y, int z) {
+        if (!((x + y + z) & 1)) return;
+        const float a = 1.0f / 64.0f, b = 3.0f * a, c9 = 9.0f * a, dd = 27.0f * a;
+        const float wt[8] = {a, b, b, c9, b, c9, c9, dd};
+        // the coarse cell of the son and the side its other contributors lie on
+        const int ic = CBOX::local((x + 4) / 2 - 2, (y + 4) / 2 - 2, (z + 4) / 2 - 2);
+        const int sx = (x & 1) ? 1 : -1, sy = (y & 1) ? CBOX::SY : -CBOX::SY, sz = (z & 1) ? CBOX::SZ : -CBOX::SZ;
+        float P = 0.0f;
+#pragma unroll
+        for (int ind = 0; ind < 8; ind++)
+            P += wt[ind] * e[ic + ((ind & 1) ? 0 : sx) + ((ind & 2) ? 0 : sy) + ((ind & 4) ? 0 : sz)];
+        const float dn = d[i] + P;
+        if (wpow<FRN>(xb[i]) + dn > 0.0f) d[i] = dn;
+    });
+    __syncthreads();
+    box_pass<FRN, BOX, 3>(NTHR, 0, d, xb, f, c);
+    box_pass<FRN, BOX, 2>(NTHR, 1, d, xb, f, c);
+    box_pass<FRN, BOX, 1>(NTHR, 0, d, xb, f, c);
+    box_pass<FRN, BOX, 0>(NTHR, 1, d, xb, f, c);
+    box_each<BOX, 0, NTHR>([&](int i, int x, int y, int z) { elem(dout, B.global(g, x, y, z)) = d[i]; });
 }
 
 }  // namespace mgs

@@ -103,6 +103,7 @@ struct mgs_handle {
     // every cycle; rebuilt when the model scalars change
     hipGraphExec_t g_plain = nullptr;
     hipGraphExec_t g_inner = nullptr;
+    const float* inner_dH = nullptr;  // mixed f(R): the array g_inner leaves level 1's increment in
     // mixed solve: the inner problem's base restricted to every level
     hipGraphExec_t g_rbase = nullptr;
     // recorded after the outer norm's copy to the host (not in arena mode):

@@ -64,8 +64,18 @@ void launch_df_correct(int frn, const float* dH, const float* rd, float* dfine, 
                        hipStream_t s);
 void launch_df_coarsest(int frn, float* d, const float* xb, const float* rhs, int n, int sweeps, const DfCoef& c,
                         hipStream_t s);
-// the inner V-cycle from level lv[0] (<= 16^3 cells) to the coarsest lv[nlev-1]
-// in one single-workgroup launch; false if nlev is out of range
+// the two halves of an inner V-cycle on a level between the tail and the large
+// ones: from R d and R r to the next level's R d and R r (d1: its start value),
+// and from the next level's corrected increment dH to dout.  d and f carry the
+// level from one half to the other.
+inline bool df_block_level(int n) { return n % 8 == 0 && n > 16 && n <= 64; }
+void launch_df_block_down(int frn, const float* rd, const float* rres, const float* xb, float* d, float* f,
+                          float* rres1, float* rd1, float* d1, int n, const DfCoef& c, hipStream_t s);
+void launch_df_block_up(int frn, const float* dH, const float* rdc, const float* d, const float* xb, const float* f,
+                        float* dout, int n, const DfCoef& c, hipStream_t s);
+// the inner V-cycle from level lv[0] (<= 16^3 cells; its R d and R r given) to
+// the coarsest lv[nlev-1] in one single-workgroup launch, the increment into
+// lv[0].d; false if nlev or the sizes are out of range
 struct TailLevelIn {
     int n;
     float *d, *xb, *f, *rres, *rd;

@@ -65,8 +65,12 @@ inline int zrun_length(int n)
     // measured at 512^3 (runs of 2, 4, 6, 8, 16, 32 planes): 4 is best; the
     // window's two prologue loads per run cost less than the lost
     // parallelism of longer runs.  At 256^3 (the 512^3 solve's level 1) runs
-    // of 2, 8 and 16 planes and 64-wide blocks are slower as well.
-    return n >= 4 ? 4 : n;
+    // of 2, 8 and 16 planes and 64-wide blocks are slower as well.  Up to 64^3
+    // a run of 4 leaves CUs idle and puts four dependent cell updates in each
+    // thread's chain: with single planes a 32^3 pass takes 2.6 us instead of
+    // 3.8 (mixed solves: 64^3 1255 -> 1095 us, 128^3 1790 -> 1590 us); at
+    // 128^3 single planes and pairs are slower than runs of 4.
+    return n > 64 ? 4 : 1;
 }
 
 // (TX x TY)-thread blocks over `width` columns x n rows, each thread marching
