@@ -493,6 +493,20 @@ void drop_graphs(mgs_handle* h)
     h->g_rbase = nullptr;
 }
 
+// the right-hand side of level l >= 1 and its V-cycle, from the restricted
+// residual and field; the small levels in one launch
+static int vcycle_plain_from_restricted(mgs_handle* h, int l)
+{
+    if (l < h->lc && h->L[l].n <= h->tail_n && h->use_tail) {
+        prof_begin(h, MGS_KC_COARSE, 16.0 * n3d(h->L[l].n) * 8.0);
+        const bool ok = launch_plain_tail(h, l);
+        prof_end(h);
+        if (ok) return 0;
+    }
+    op_rhs(h, l);
+    return vcycle_plain(h, l);
+}
+
 // V_cycle(ilevel), PMP2extradof.f90:352-555 (Nsmth = 2, :361)
 int vcycle_plain(mgs_handle* h, int l)
 {
@@ -504,14 +518,10 @@ int vcycle_plain(mgs_handle* h, int l)
     if (l > 0) op_residual(h, l, true, nullptr);
     op_restrict_both(h, l + 1);
     if (l == 0) {
-        int rc = run_captured(h, &h->g_plain, [h]() {
-            op_rhs(h, 1);
-            return vcycle_plain(h, 1);
-        });
+        int rc = run_captured(h, &h->g_plain, [h]() { return vcycle_plain_from_restricted(h, 1); });
         if (rc) return rc;
     } else {
-        op_rhs(h, l + 1);
-        vcycle_plain(h, l + 1);
+        vcycle_plain_from_restricted(h, l + 1);
     }
     op_correct(h, l + 1, true);
     op_smooth2(h, l);
@@ -527,8 +537,13 @@ static int cgc_plain(mgs_handle* h, int l, int kind)
 {
     if (l > 0) op_residual(h, l, true, nullptr);
     op_restrict_both(h, l + 1);
-    op_rhs(h, l + 1);
-    int rc = cycle_plain(h, l + 1, kind);
+    int rc;
+    if (kind == 0) {
+        rc = vcycle_plain_from_restricted(h, l + 1);
+    } else {
+        op_rhs(h, l + 1);
+        rc = cycle_plain(h, l + 1, kind);
+    }
     if (rc) return rc;
     op_correct(h, l + 1, true);
     return 0;
@@ -802,6 +817,25 @@ static void dgpm_smooth4(mgs_handle* h, int l, int cls)
     }
 }
 
+static int vcycle_inner_dgp(mgs_handle* h, int l);
+
+// the right-hand side of level l >= 1 and its inner V-cycle, from the
+// restricted residual and increment; the small levels in one launch
+static int dgpm_from_restricted(mgs_handle* h, int l)
+{
+    LevelF& c = h->M[l];
+    if (l < h->lc && c.n <= h->tail_n && h->use_tail) {
+        prof_begin(h, MGS_KC_COARSE, 20.0 * n3d(c.n) * 4.0);
+        const bool ok = launch_dgpm_tail(h, l);
+        prof_end(h);
+        if (ok) return 0;
+    }
+    prof_begin(h, MGS_KC_COARSE, 5.0 * n3d(c.n) * 4.0);
+    launch_dgpm_residual(c.rd, c.xb, h->L[l].rho, c.rho, c.rres, c.f, c.n, dgp_coefs(h->p, l), h->s);
+    prof_end(h);
+    return vcycle_inner_dgp(h, l);
+}
+
 static int vcycle_inner_dgp(mgs_handle* h, int l)
 {
     LevelF& v = h->M[l];
@@ -823,18 +857,12 @@ static int vcycle_inner_dgp(mgs_handle* h, int l)
     launch_restrict8_32(v.res, c.rres, nullptr, c.n, h->s);
     launch_restrict8_32(v.d, c.rd, c.d, c.n, h->s);
     prof_end(h);
-    auto coarse = [h, l, &c]() {
-        prof_begin(h, MGS_KC_COARSE, 5.0 * n3d(c.n) * 4.0);
-        launch_dgpm_residual(c.rd, c.xb, h->L[l + 1].rho, c.rho, c.rres, c.f, c.n, dgp_coefs(h->p, l + 1), h->s);
-        prof_end(h);
-        return vcycle_inner_dgp(h, l + 1);
-    };
-    if (l == 0) {
-        int rc = run_captured(h, &h->g_inner, coarse);
-        if (rc) return rc;
-    } else {
-        coarse();
-    }
+    int rc;
+    if (l == 0)
+        rc = run_captured(h, &h->g_inner, [h]() { return dgpm_from_restricted(h, 1); });
+    else
+        rc = dgpm_from_restricted(h, l + 1);
+    if (rc) return rc;
     prof_begin(h, l == 0 ? MGS_KC_CORRECT : MGS_KC_COARSE, (3.0 * n3d(v.n) + 2.0 * n3d(c.n)) * s);
     launch_dgpm_correct(c.d, c.rd, v.d, c.n, h->s);
     prof_end(h);
@@ -932,10 +960,15 @@ static int dgp_cgc(mgs_handle* h, int l, int kind)
     launch_restrict8_32(v.res, c.rres, nullptr, c.n, h->s);
     launch_restrict8_32(v.d, c.rd, c.d, c.n, h->s);
     prof_end(h);
-    prof_begin(h, MGS_KC_COARSE, 5.0 * n3d(c.n) * 4.0);
-    launch_dgpm_residual(c.rd, c.xb, h->L[l + 1].rho, c.rho, c.rres, c.f, c.n, dgp_coefs(h->p, l + 1), h->s);
-    prof_end(h);
-    const int rc = kind == 0 ? vcycle_inner_dgp(h, l + 1) : fw_inner_dgp(h, l + 1, kind);
+    int rc;
+    if (kind == 0) {
+        rc = dgpm_from_restricted(h, l + 1);
+    } else {
+        prof_begin(h, MGS_KC_COARSE, 5.0 * n3d(c.n) * 4.0);
+        launch_dgpm_residual(c.rd, c.xb, h->L[l + 1].rho, c.rho, c.rres, c.f, c.n, dgp_coefs(h->p, l + 1), h->s);
+        prof_end(h);
+        rc = fw_inner_dgp(h, l + 1, kind);
+    }
     if (rc) return rc;
     prof_begin(h, l == 0 ? MGS_KC_CORRECT : MGS_KC_COARSE, (3.0 * n3d(v.n) + 2.0 * n3d(c.n)) * 4.0);
     launch_dgpm_correct(c.d, c.rd, v.d, c.n, h->s);

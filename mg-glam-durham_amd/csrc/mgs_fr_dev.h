@@ -981,7 +981,10 @@ __device__ __forceinline__ void restrict8_cell(const T* __restrict__ fine, T* __
 // about 110 instructions each) and the chain of barriers and latencies
 // below.  A thread therefore keeps its cells' offsets, xb and f in registers
 // for the four passes of a block, and levels of at most TAIL_WAVE_HALF cells
-// a colour run in the first wave without barriers.  TAIL_FIGURES
+// a colour run in the first wave without barriers; index divisions by the
+// level's side, which made up most of the chain on the small levels, are
+// shifts (half_mjk).  From 16^3: 57 us and a launch of 3.9 for f before, now 41
+// for both, of which two thirds on the 16^3 level and 5 us on the coarsest.
 // ---------------------------------------------------------------------------
 struct TailLevel {
     Geo g;

@@ -200,6 +200,12 @@ void launch_dgpm_zpass(const float* e0, const float* e1, float* out, const float
                        const float* rhs, int n, int colour, const DgpCoef& c, hipStream_t s);
 void launch_round_f32(const double* a, float* b, size_t n, hipStream_t s);
 
+// mgs_tail.hip: the V-cycle on the level l >= 1 whose R u and R r are in
+// place (right-hand side included), in one single-workgroup launch; false,
+// with nothing launched, if its levels are not the launch's
+bool launch_plain_tail(mgs_handle* h, int l);
+bool launch_dgpm_tail(mgs_handle* h, int l);
+
 // mgs_fft.hip
 void fft_release(mgs_handle* h);
 

@@ -36,3 +36,29 @@ def test_mixed_solve_equals_the_served_solve(N, n):
         S.solve(mode=1, rel_tol=1e-9, max_cycles=40)
         ref = S.get_field()
     assert np.max(np.abs(u - ref)) <= 1e-6 * np.max(np.abs(ref))
+
+
+# FP64 cycles whose tail starts at 16, 12 (coarsest 6), 8 and 4 cells a side,
+# and grids without one (coarsest 14 or 10), against the oracle's cycles
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [8, 16, 32, 48, 96, 28, 40])
+@pytest.mark.parametrize("model,n", [(M.MODEL_FR, 0), (M.MODEL_FR, 1), (M.MODEL_FR, 2), (M.MODEL_DGP, 1)])
+def test_fp64_cycles_match_the_oracle(N, model, n):
+    delta = O.lognormal_density(N, 2.0 * N, 1.0, seed=N)
+    cfg = M.Config(N=N, model=model, fr_n=n, box=2.0 * N, fr0=-1e-5)
+    p = O.Params(N=N, model=model, fr_n=n, branch=1, box=2.0 * N, om=0.3, oml=0.7, a=1.0, fr0=-1e-5, h0rc=1.0, polish=1)
+    print(f"[small levels] FP64 N={N} model={model} n={n}", flush=True)
+    with M.Solver(cfg) as S:
+        S.set_density(delta)
+        S.initialise()
+        u0 = S.get_field()
+        for _ in range(2):
+            S.vcycle(0)
+        u = S.get_field()
+    ref = u0.copy()
+    O.vcycles(p, ref, delta, 2, prec="f64")  # in place
+    scale = np.max(np.abs(ref))
+    if model == M.MODEL_DGP:
+        assert np.array_equal(u, ref)
+    else:  # the smoother's root is good to rtol 1e-13
+        assert np.max(np.abs(u - ref)) <= 1e-12 * scale
