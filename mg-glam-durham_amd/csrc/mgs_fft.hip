@@ -19,6 +19,7 @@
 #include "mgs_device.h"
 #include "mgs_internal.h"
 #include "mgs_kernels.h"
+#include "mgs_poisson.h"
 #include "mgs_stencil.h"
 
 namespace mgs {
@@ -32,6 +33,7 @@ struct FftState {
     double* bins = nullptr;          // 6 (N/2 + 1): power, count, sum|m| of the linear and the log bins
     double* binpart = nullptr;       // BIN_BLOCKS such histograms, one per block
     int* logbin = nullptr;           // log bin of every |m|^2 = 0 .. 3 (N/2)^2
+    void* tables = nullptr;          // power-of-two Poisson solve: twiddles and Green's function
 };
 
 // blocks of the binning kernel: each accumulates a private histogram in LDS
@@ -39,27 +41,55 @@ static const int BIN_BLOCKS = 512;
 
 static FftState* fft_of(mgs_handle* h) { return (FftState*)h->fft; }
 
-static int fft_ensure(mgs_handle* h)
+static FftState* fft_state(mgs_handle* h)
 {
     if (!h->fft) h->fft = new FftState();
     FftState* f = fft_of(h);
-    const int N = h->p.ngrid;
-    if (f->N == N && f->real) return 0;
-    f->N = N;
-    const size_t n3 = (size_t)N * N * N;
-    const size_t nc = (size_t)N * N * (N / 2 + 1);
-    if (hipMalloc((void**)&f->real, n3 * sizeof(double)) != hipSuccess) return set_err(h, MGS_E_NOMEM, "FFT buffer");
-    if (hipMalloc((void**)&f->cplx, nc * sizeof(hipfftDoubleComplex)) != hipSuccess)
-        return set_err(h, MGS_E_NOMEM, "FFT buffer");
-    if (hipMalloc((void**)&f->bins, 3 * (size_t)(N + 2) * sizeof(double)) != hipSuccess)
-        return set_err(h, MGS_E_NOMEM, "FFT bins");
-    if (hipMalloc((void**)&f->binpart, (size_t)BIN_BLOCKS * 3 * (N + 2) * sizeof(double)) != hipSuccess)
-        return set_err(h, MGS_E_NOMEM, "FFT bins");
-    if (hipfftPlan3d(&f->fwd, N, N, N, HIPFFT_D2Z) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftPlan3d D2Z");
-    f->have_fwd = true;
+    f->N = h->p.ngrid;  // a handle's grid does not change
+    return f;
+}
+
+static int fft_alloc(mgs_handle* h, void** p, size_t bytes, const char* what)
+{
+    if (*p) return 0;
+    if (hipMalloc(p, bytes) == hipSuccess) return 0;
+    *p = nullptr;
+    return set_err(h, MGS_E_NOMEM, what);
+}
+
+static int fft_ensure_cplx(mgs_handle* h)
+{
+    FftState* f = fft_state(h);
+    const size_t nc = (size_t)f->N * f->N * (f->N / 2 + 1);
+    return fft_alloc(h, (void**)&f->cplx, nc * sizeof(hipfftDoubleComplex), "FFT buffer");
+}
+
+// the library's transforms and their buffers
+static int fft_ensure(mgs_handle* h)
+{
+    FftState* f = fft_state(h);
+    const int N = f->N;
+    int rc;
+    if ((rc = fft_ensure_cplx(h))) return rc;
+    if ((rc = fft_alloc(h, (void**)&f->real, (size_t)N * N * N * sizeof(double), "FFT buffer"))) return rc;
+    if ((rc = fft_alloc(h, (void**)&f->bins, 3 * (size_t)(N + 2) * sizeof(double), "FFT bins"))) return rc;
+    if ((rc = fft_alloc(h, (void**)&f->binpart, (size_t)BIN_BLOCKS * 3 * (N + 2) * sizeof(double), "FFT bins"))) return rc;
+    if (!f->have_fwd) {
+        if (hipfftPlan3d(&f->fwd, N, N, N, HIPFFT_D2Z) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftPlan3d D2Z");
+        f->have_fwd = true;
+        hipfftSetStream(f->fwd, h->s);
+    }
+    return 0;
+}
+
+// the inverse transform's plan (the power spectrum needs none)
+static int fft_ensure_inverse(mgs_handle* h)
+{
+    FftState* f = fft_state(h);
+    const int N = f->N;
+    if (f->have_inv) return 0;
     if (hipfftPlan3d(&f->inv, N, N, N, HIPFFT_Z2D) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftPlan3d Z2D");
     f->have_inv = true;
-    hipfftSetStream(f->fwd, h->s);
     hipfftSetStream(f->inv, h->s);
     return 0;
 }
@@ -75,6 +105,7 @@ void fft_release(mgs_handle* h)
     if (f->bins) (void)hipFree(f->bins);
     if (f->binpart) (void)hipFree(f->binpart);
     if (f->logbin) (void)hipFree(f->logbin);
+    if (f->tables) (void)hipFree(f->tables);
     delete f;
     h->fft = nullptr;
 }
@@ -331,14 +362,6 @@ __global__ __launch_bounds__(256) void k_bin_reduce(const double* __restrict__ p
 // half-complex i = N - k.  The half spectrum (x fastest, N/2+1 of it) is
 // multiplied by trfi / A and by 1/N^3, hipFFT's transforms being
 // unnormalised where FFTPACK5's forward one divides by N per dimension.
-__device__ __forceinline__ double green_g(int k, int N)
-{
-    const double P16 = (double)6.28318530718f;
-    const int i = k <= N / 2 ? k : N - k;
-    if (2 * i == N) return -2.0;
-    return 2.0 * cos(P16 * i / N);
-}
-
 __global__ __launch_bounds__(256) void k_green(hipfftDoubleComplex* __restrict__ c, int N, double trfi,
                                                double inv_n3)
 {
@@ -422,6 +445,7 @@ int mgs_make_lognormal_density(mgs_handle* h, uint64_t seed, double sigma_g, dou
 {
     if (!h || !(sigma_g > 0.0) || !(kcut_frac > 0.0)) return set_err(h, MGS_E_ARG, "lognormal parameters");
     int rc = fft_ensure(h);
+    if (!rc) rc = fft_ensure_inverse(h);
     if (rc) return rc;
     FftState* f = fft_of(h);
     const int N = h->p.ngrid;
@@ -626,26 +650,48 @@ int mgs_power_spectrum(mgs_handle* h, int32_t which, double* k, double* pk, doub
     return mgs_power_spectrum_ex(h, which, 0, 0, k, pk, count, nullptr, nullptr, nullptr);
 }
 
+// the power-of-two form (mgs_poisson.hip)
+static int potential_pow2(mgs_handle* h, float* phi, double trfi)
+{
+    int rc = fft_ensure_cplx(h);
+    if (rc) return rc;
+    FftState* f = fft_of(h);
+    const int N = f->N;
+    if (!f->tables) {
+        if ((rc = fft_alloc(h, &f->tables, poisson_table_bytes(N), "Poisson tables"))) return rc;
+        launch_poisson_tables(f->tables, N, h->s);
+    }
+    launch_poisson(h->L[0].rho, f->cplx, phi, f->tables, N, trfi, h->s);
+    return 0;
+}
+
 int mgs_potential(mgs_handle* h, double trfi)
 {
     if (!h) return MGS_E_ARG;
     if (!std::isfinite(trfi)) return set_err(h, MGS_E_ARG, "trfi not finite");
     if (!h->has_density) return set_err(h, MGS_E_STATE, "no density set");
-    int rc = fft_ensure(h);
-    if (rc) return rc;
     float* phi = pm_potential(h);
     if (!phi) return set_err(h, MGS_E_NOMEM, "potential buffer");
-    FftState* f = fft_of(h);
     const int N = h->p.ngrid;
     const double n3 = (double)N * N * N;
-    prof_begin(h, MGS_KC_PM, 8.0 * n3 * 2.0 + 12.0 * n3);
-    launch_unpack_f64_to_f64(h->L[0].rho, f->real, N, 1.0, h->s);
-    if (hipfftExecD2Z(f->fwd, f->real, f->cplx) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecD2Z");
-    hipLaunchKernelGGL(k_green, grid_for((size_t)N * N * (N / 2 + 1)), dim3(256), 0, h->s, f->cplx, N, trfi, 1.0 / n3);
-    if (hipfftExecZ2D(f->inv, f->cplx, f->real) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecZ2D");
-    // FI is REAL*4 between the reference's transform passes and after them
-    hipLaunchKernelGGL(k_to_f32, grid_for((size_t)n3), dim3(256), 0, h->s, f->real, phi, (size_t)n3);
-    prof_end(h);
+    int rc;
+    if (poisson_grid(N)) {
+        prof_begin(h, MGS_KC_PM, 8.0 * n3 * 2.0 + 12.0 * n3);
+        rc = potential_pow2(h, phi, trfi);
+        prof_end(h);
+        if (rc) return rc;
+    } else {
+        if ((rc = fft_ensure(h)) || (rc = fft_ensure_inverse(h))) return rc;
+        FftState* f = fft_of(h);
+        prof_begin(h, MGS_KC_PM, 8.0 * n3 * 2.0 + 12.0 * n3);
+        launch_unpack_f64_to_f64(h->L[0].rho, f->real, N, 1.0, h->s);
+        if (hipfftExecD2Z(f->fwd, f->real, f->cplx) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecD2Z");
+        hipLaunchKernelGGL(k_green, grid_for((size_t)N * N * (N / 2 + 1)), dim3(256), 0, h->s, f->cplx, N, trfi, 1.0 / n3);
+        if (hipfftExecZ2D(f->inv, f->cplx, f->real) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecZ2D");
+        // FI is REAL*4 between the reference's transform passes and after them
+        hipLaunchKernelGGL(k_to_f32, grid_for((size_t)n3), dim3(256), 0, h->s, f->real, phi, (size_t)n3);
+        prof_end(h);
+    }
     if (hipStreamSynchronize(h->s) != hipSuccess) return set_err(h, MGS_E_HIP, "potential");
     return 0;
 }
