@@ -305,26 +305,24 @@ int op_smooth(mgs_handle* h, int l, int red)
     return 0;
 }
 
-// Nsmth = 2 red-black pairs (colour 0, then 1) on level l.  nDGP levels with
-// z-marching passes ping-pong between u and the second array: after two
-// pairs the field is back in u.
+// Nsmth = 2 red-black pairs (colour 0, then 1) on level l.  nDGP passes are out
+// of place and ping-pong between u and a second array: after two pairs the
+// field is back in u.  (A copy back after each pass made half the launches of
+// the levels below 128^3.)
 static void op_smooth2(mgs_handle* h, int l)
 {
     LevelD& v = h->L[l];
-    if (h->p.model == MGS_MODEL_DGP && h->dgp_spare64 && dgp_zmarch(v.n)) {
+    // below level 0 a whole level fits the scratch of half a level-0 array
+    double* B = h->p.model != MGS_MODEL_DGP ? nullptr : (l == 0 ? h->dgp_spare64 : h->dgp_tmp);
+    if (B) {
         const DgpCoef c = dgp_coefs(h->p, l);
         const size_t half = (size_t)v.n * v.n * (v.n / 2);
-        double* A = v.u;
-        double* B = h->dgp_spare64;
-        for (int s = 0; s < 2; s++) {
-            for (int colour = 0; colour < 2; colour++) {
-                if (l == 0) prof_begin(h, MGS_KC_SMOOTH, 2.0 * n3d(v.n) * 8.0);
-                else prof_begin(h, MGS_KC_COARSE, 2.0 * n3d(v.n) * 8.0);
-                launch_dgp_zpass64(l, colour ? B : A, A + half, B + (size_t)colour * half, v.rho, v.f, v.n, colour, c,
-                                   h->s);
-                prof_end(h);
-            }
-            std::swap(A, B);
+        for (int it = 0; it < 4; it++) {
+            if (l == 0) prof_begin(h, MGS_KC_SMOOTH, 2.0 * n3d(v.n) * 8.0);
+            else prof_begin(h, MGS_KC_COARSE, 2.0 * n3d(v.n) * 8.0);
+            const PingPong<double> q = ping_pong(v.u, B, half, it);
+            launch_dgp_pass64(l, q.h0, q.h1, q.out, v.rho, v.f, v.n, it & 1, c, h->s);
+            prof_end(h);
         }
         return;
     }
@@ -786,33 +784,18 @@ static int solve_plain(mgs_handle* h, const mgs_solve_opts& o, mgs_solve_report*
 }
 
 // ---- nDGP: inner V-cycle on the FP32 increment e (see mgs_dgp.hip) ----------
-// 2 x Nsmth colour passes (0, 1, 0, 1) of the inner smoother on level l;
-// z-marching levels ping-pong between e and the scratch array and end in e
+// 2 x Nsmth colour passes (0, 1, 0, 1) of the inner smoother on level l,
+// ping-ponging between e and the scratch array (a level-0 array of floats) and
+// ending in e
 static void dgpm_smooth4(mgs_handle* h, int l, int cls)
 {
     LevelF& v = h->M[l];
-    LevelD& V = h->L[l];
     const DgpCoef dc = dgp_coefs(h->p, l);
-    float* tmp = (float*)h->dgp_tmp;
-    const double bytes = 3.0 * n3d(v.n) * 4.0;
-    if (dgp_zmarch(v.n) && v.rho) {
-        const size_t half = (size_t)v.n * v.n * (v.n / 2);
-        float* A = v.d;
-        float* B = tmp;  // holds a level-0 array of floats
-        for (int s = 0; s < 2; s++) {
-            for (int colour = 0; colour < 2; colour++) {
-                prof_begin(h, cls, bytes);
-                launch_dgpm_zpass(colour ? B : A, A + half, B + (size_t)colour * half, v.xb, v.rho, v.f, v.n, colour,
-                                  dc, h->s);
-                prof_end(h);
-            }
-            std::swap(A, B);
-        }
-        return;
-    }
+    const size_t half = (size_t)v.n * v.n * (v.n / 2);
     for (int it = 0; it < 4; it++) {
-        prof_begin(h, cls, bytes);
-        launch_dgpm_smooth(v.d, v.xb, V.rho, v.f, tmp, v.n, (it & 1) ? 1 : 0, dc, h->s);
+        prof_begin(h, cls, 3.0 * n3d(v.n) * 4.0);
+        const PingPong<float> q = ping_pong(v.d, (float*)h->dgp_tmp, half, it);
+        launch_dgpm_pass(q.h0, q.h1, q.out, v.xb, h->L[l].rho, v.rho, v.f, v.n, it & 1, dc, h->s);
         prof_end(h);
     }
 }

@@ -75,11 +75,13 @@ static unsigned launch_both_z(const OP& op, double* partials, int n, hipStream_t
     return L.NB;
 }
 
-// relaxation_iterations_DGP, one colour, out of place into tmp (one colour half)
+// relaxation_iterations_DGP, one colour, from the field's colour halves into out
+// (the colour's new half)
 template <bool COARSE>
-__global__ __launch_bounds__(256) void k_dgp_smooth64(const double* __restrict__ u, const double* __restrict__ rho,
-                                                      const double* __restrict__ f, double* __restrict__ tmp, Geo g,
-                                                      int colour, DgpCoef c, int TX, int TY, int XB, unsigned NB)
+__global__ __launch_bounds__(256) void k_dgp_smooth64(const double* __restrict__ h0, const double* __restrict__ h1,
+                                                      const double* __restrict__ rho, const double* __restrict__ f,
+                                                      double* __restrict__ out, Geo g, int colour, DgpCoef c, int TX,
+                                                      int TY, int XB, unsigned NB)
 {
     int m;
     unsigned row;
@@ -87,11 +89,11 @@ __global__ __launch_bounds__(256) void k_dgp_smooth64(const double* __restrict__
     const int j = (int)(row % (unsigned)g.n), k = (int)(row / (unsigned)g.n);
     const int i = 2 * m + ((colour + j + k) & 1);
     const size_t me = (size_t)colour * g.half + row_base(g, j, k) + m;
-    double c0;
-    double L = dgp_L(u, g, i, j, k, rho[me], c, c0);
+    const S19<double> s = s19_halves(h0, h1, g, i, j, k);
+    double L = dgp_L19(s, rho[me], c);
     if constexpr (COARSE) L = L - f[me];
     const double dLphi = -6.0 / c.dx2;
-    tmp[row_base(g, j, k) + m] = c0 - L / dLphi;
+    out[row_base(g, j, k) + m] = s.c0 - L / dLphi;
 }
 
 template <bool COARSE>
@@ -244,17 +246,34 @@ __global__ __launch_bounds__(256) void k_dgp_rhs64(const double* __restrict__ ru
     f[me] = OP;
 }
 
+void launch_dgp_pass64(int level, const double* h0, const double* h1, double* out, const double* rho, const double* f,
+                       int n, int colour, const DgpCoef& c, hipStream_t s)
+{
+    if (dgp_zmarch(n)) {
+        launch_dgp_zpass64(level, h0, h1, out, rho, f, n, colour, c, s);
+        return;
+    }
+    const Geo g = make_geo(n);
+    const Launch L = make_launch(g.h, (long)n * n);
+    if (level == 0)
+        hipLaunchKernelGGL((k_dgp_smooth64<false>), L.grid, L.block, 0, s, h0, h1, rho, f, out, g, colour, c, L.TX, L.TY,
+                           L.XB, L.NB);
+    else
+        hipLaunchKernelGGL((k_dgp_smooth64<true>), L.grid, L.block, 0, s, h0, h1, rho, f, out, g, colour, c, L.TX, L.TY,
+                           L.XB, L.NB);
+}
+
 void launch_dgp_smooth64(int level, double* u, const double* rho, const double* f, double* tmp, int n, int colour,
                          const DgpCoef& c, hipStream_t s)
 {
     const Geo g = make_geo(n);
     const Launch L = make_launch(g.h, (long)n * n);
     if (level == 0)
-        hipLaunchKernelGGL((k_dgp_smooth64<false>), L.grid, L.block, 0, s, u, rho, f, tmp, g, colour, c, L.TX, L.TY,
-                           L.XB, L.NB);
+        hipLaunchKernelGGL((k_dgp_smooth64<false>), L.grid, L.block, 0, s, u, u + g.half, rho, f, tmp, g, colour, c,
+                           L.TX, L.TY, L.XB, L.NB);
     else
-        hipLaunchKernelGGL((k_dgp_smooth64<true>), L.grid, L.block, 0, s, u, rho, f, tmp, g, colour, c, L.TX, L.TY,
-                           L.XB, L.NB);
+        hipLaunchKernelGGL((k_dgp_smooth64<true>), L.grid, L.block, 0, s, u, u + g.half, rho, f, tmp, g, colour, c,
+                           L.TX, L.TY, L.XB, L.NB);
     launch_copy_f64(tmp, u + (size_t)colour * g.half, g.half, s);
 }
 
@@ -306,8 +325,10 @@ int dgp_alloc(mgs_handle* h)
     int rc = dev_alloc(h, half * sizeof(double) + 256, &q, "DGP scratch");
     if (rc) return rc;
     h->dgp_tmp = (double*)q;
-    // FP64 z-marching passes: the second array of the field's ping-pong
-    if (h->p.precision == MGS_PREC_FP64 && dgp_zmarch(h->p.ngrid)) {
+    // FP64 passes: the second array of the level-0 field's ping-pong (not out of
+    // the fixed scratch of mgs_solve_noalloc, whose largest grids it would not
+    // fit beside: level 0 is then copied back)
+    if (h->p.precision == MGS_PREC_FP64 && (dgp_zmarch(h->p.ngrid) || !h->use_arena)) {
         rc = dev_alloc(h, 2 * half * sizeof(double) + 256, &q, "DGP second array");
         if (rc) return rc;
         h->dgp_spare64 = (double*)q;
@@ -332,16 +353,16 @@ int dgp_alloc(mgs_handle* h)
 // keeps converging.  The smoother is the reference's update
 // e <- e - (D(e) - rhs) / (-6/dx^2), colour by colour, out of place.
 
-// one colour of the inner smoother, out of place into tmp (one colour half)
-__global__ __launch_bounds__(256) void k_dgpm_smooth(const float* __restrict__ e, const float* __restrict__ pb,
-                                                     const double* __restrict__ rho, const float* __restrict__ rhs,
-                                                     float* __restrict__ tmp, Geo g, int colour, DgpF c, int TX,
-                                                     int TY, int XB, unsigned NB)
+// one colour of the inner smoother, from the increment's halves into out
+__global__ __launch_bounds__(256) void k_dgpm_smooth(const float* __restrict__ e0, const float* __restrict__ e1,
+                                                     const float* __restrict__ pb, const double* __restrict__ rho,
+                                                     const float* __restrict__ rhs, float* __restrict__ out, Geo g,
+                                                     int colour, DgpF c, int TX, int TY, int XB, unsigned NB)
 {
     int m;
     unsigned row;
     if (!map_xy(g.h, (long)g.n * g.n, TX, TY, XB, NB, m, row)) return;
-    dgpm_smooth_cell(e, pb, rho, rhs, tmp, g, colour, c, m, row);
+    dgpm_smooth_cell(e0, e1, pb, rho, rhs, out, g, colour, c, m, row);
 }
 
 // out = D(e) - rhs on both colours (inner residual; with (e, rhs, out) =
@@ -379,46 +400,6 @@ __global__ __launch_bounds__(1024) void k_dgpm_coarsest(float* __restrict__ e, c
     dgpm_coarsest_block(e, pb, rho, rhs, tmp, g, sweeps, c);
 }
 
-// The same correction z-marching over coarse columns, as k_df_correct: planes
-// of e = e_H - R e_h in registers (x-neighbours from the adjacent lanes), all
-// 8 sons of a coarse cell, software-pipelined (plane K's sons computed, the
-// loads of plane K+1 issued, then plane K's sons stored).  Sums in
-// dgpm_correct_cell's order.
-template <int S3, bool NT>
-__device__ __forceinline__ void dgpm_sons_load(const float* __restrict__ ef, const Geo& gf, int I, int J, int K,
-                                               float* old)
-{
-#pragma unroll
-    for (int t = 0; t < 4; t++) old[t] = ld_once<NT>(elem(ef, son_index(gf, I, J, K, t & 1, t >> 1, S3)));
-}
-
-template <int S3>
-__device__ __forceinline__ void dgpm_sons_new(const float* ez, const float* ek, const float* old, float* nv)
-{
-    const float a = 1.0f / 64.0f, b = 3.0f * a, c9 = 9.0f * a, dd = 27.0f * a;
-    const float wt[8] = {a, b, b, c9, b, c9, c9, dd};
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const int s1 = t & 1, s2 = t >> 1;
-        float P = 0.0f;
-#pragma unroll
-        for (int ind = 0; ind < 8; ind++) {
-            const int x = (ind & 1) ? 1 : (s1 ? 2 : 0);
-            const int y = (ind & 2) ? 1 : (s2 ? 2 : 0);
-            P += wt[ind] * ((ind & 4) ? ek[x + 3 * y] : ez[x + 3 * y]);
-        }
-        nv[t] = old[t] + P;
-    }
-}
-
-template <int S3, bool NT>
-__device__ __forceinline__ void dgpm_sons_store(float* __restrict__ ef, const Geo& gf, int I, int J, int K,
-                                                const float* nv)
-{
-#pragma unroll
-    for (int t = 0; t < 4; t++) st_once<NT>(elem(ef, son_index(gf, I, J, K, t & 1, t >> 1, S3)), nv[t]);
-}
-
 template <bool NT>
 __global__ __launch_bounds__(256) void k_dgpm_zcorrect(const float* __restrict__ eH, const float* __restrict__ rd,
                                                        float* __restrict__ ef, Geo gf, Geo gc, int TX, int TY, int XB,
@@ -431,37 +412,7 @@ __global__ __launch_bounds__(256) void k_dgpm_zcorrect(const float* __restrict__
     const unsigned t = threadIdx.y * (unsigned)TX + threadIdx.x;
     const bool lok = threadIdx.x > 0 && (t & 63u) != 0;
     const bool rok = (int)threadIdx.x + 1 < TX && cc.m + 1 < gc.n && ((t + 1) & 63u) != 0;
-    const int I = cc.m, J = cc.j;
-    Block9 B;
-    B.init(gc, I, J);
-    ERaw wm, wk, wp;  // coarse planes K-1, K, K+1
-    float o0[4], o1[4];
-    e_load<true>(eH, rd, B, wrap_dec(cc.k0, gc.n), lok, rok, wm);
-    e_load<true>(eH, rd, B, cc.k0, lok, rok, wk);
-    e_load<true>(eH, rd, B, wrap_inc(cc.k0, gc.n), lok, rok, wp);
-    dgpm_sons_load<0, NT>(ef, gf, I, J, cc.k0, o0);
-    dgpm_sons_load<1, NT>(ef, gf, I, J, cc.k0, o1);
-    float em[9], ek[9], ep[9];
-    e_form<true>(wm, lok, rok, em);
-    e_form<true>(wk, lok, rok, ek);
-    for (int K = cc.k0; K < cc.k1; K++) {
-        e_form<true>(wp, lok, rok, ep);
-        float n0[4], n1[4];
-        dgpm_sons_new<0>(em, ek, o0, n0);
-        dgpm_sons_new<1>(ep, ek, o1, n1);
-        if (K + 1 < cc.k1) {
-            dgpm_sons_load<0, NT>(ef, gf, I, J, K + 1, o0);
-            dgpm_sons_load<1, NT>(ef, gf, I, J, K + 1, o1);
-            e_load<true>(eH, rd, B, wrap_inc(K + 1, gc.n), lok, rok, wp);
-        }
-        dgpm_sons_store<0, NT>(ef, gf, I, J, K, n0);
-        dgpm_sons_store<1, NT>(ef, gf, I, J, K, n1);
-#pragma unroll
-        for (int q = 0; q < 9; q++) {
-            em[q] = ek[q];
-            ek[q] = ep[q];
-        }
-    }
+    dgpm_correct_col<true, NT>(eH, rd, ef, gf, gc, cc, lok, rok);
 }
 
 // phi += e
@@ -488,14 +439,17 @@ int launch_dgpm_outer(const double* u, const double* rho, float* g32, float* pb,
     return (int)L.NB;
 }
 
-void launch_dgpm_smooth(float* e, const float* pb, const double* rho, const float* rhs, float* tmp, int n, int colour,
-                        const DgpCoef& c, hipStream_t s)
+void launch_dgpm_pass(const float* e0, const float* e1, float* out, const float* pb, const double* rho,
+                      const float* rho32, const float* rhs, int n, int colour, const DgpCoef& c, hipStream_t s)
 {
+    if (dgp_zmarch(n) && rho32) {
+        launch_dgpm_zpass(e0, e1, out, pb, rho32, rhs, n, colour, c, s);
+        return;
+    }
     const Geo g = make_geo(n);
     const Launch L = make_launch(g.h, (long)n * n);
-    hipLaunchKernelGGL(k_dgpm_smooth, L.grid, L.block, 0, s, e, pb, rho, rhs, tmp, g, colour, dgpf(c), L.TX, L.TY,
+    hipLaunchKernelGGL(k_dgpm_smooth, L.grid, L.block, 0, s, e0, e1, pb, rho, rhs, out, g, colour, dgpf(c), L.TX, L.TY,
                        L.XB, L.NB);
-    launch_copy_f32(tmp, e + (size_t)colour * g.half, g.half, s);
 }
 
 void launch_dgpm_residual(const float* e, const float* pb, const double* rho, const float* rho32, const float* rhs,
@@ -615,61 +569,6 @@ __global__ __launch_bounds__(256) void k_dgp_zsmooth64(const double* __restrict_
         dgp_zsmooth64_run<COARSE, true, NT>(h0, h1, out, rho, f, g, colour, c, d, cc.k0);
     else
         dgp_zsmooth64_run<COARSE, false, NT>(h0, h1, out, rho, f, g, colour, c, d, cc.k0);
-}
-
-// one colour of the mixed inner smoother (as k_dgpm_smooth); S0 as above
-template <bool S0, bool NT>
-__device__ __forceinline__ void dgpm_zsmooth_run(const float* __restrict__ e0, const float* __restrict__ e1,
-                                                 float* __restrict__ out, const float* __restrict__ pb,
-                                                 const float* __restrict__ rho32, const float* __restrict__ rhs,
-                                                 const Geo& g, int colour, const DgpF& c, const DCol& d, int k0)
-{
-    // (j + k0) & 1 = S0 ^ colour: wave-uniform
-    const int par0 = (S0 ? 1 : 0) ^ (colour & 1);
-    const DHalves<float> He = dhalves(e0, e1, par0), Hb = dhalves(pb, pb + g.half, par0);
-    const float* rhoc = rho32 + (size_t)colour * g.half;
-    const float* rhsc = rhs + (size_t)colour * g.half;
-    DWin2<float> we, wb;
-    dwin2_init(we, He, d, k0, g.n);
-    dwin2_init(wb, Hb, d, k0, g.n);
-    DSide<float> se, sb;
-    dside_load(He, d, k0, 0, g.n, S0, se);
-    dside_load(Hb, d, k0, 0, g.n, S0, sb);
-    unsigned off = (unsigned)k0 * d.plane + d.rowoff[1] + d.m;
-    float rh = ld_once<NT>(elem(rhoc, off));
-    float fv = ld_once<NT>(elem(rhsc, off));
-#pragma unroll
-    for (int t = 0; t < DGP_KC; t++) {
-        const int k = k0 + t;
-        const bool s = S0 ^ ((t & 1) != 0);
-        DRaw2<float> re, rb;
-        DSide<float> sen, sbn;
-        float rhn = 0.0f, fvn = 0.0f;
-        const unsigned offn = off + d.plane;
-        if (t + 1 < DGP_KC) {
-            const int kn = wrap_inc(k + 1, g.n);
-            draw2_load(He, d, kn, t + 2, re);
-            draw2_load(Hb, d, kn, t + 2, rb);
-            dside_load(He, d, wrap_inc(k, g.n), t + 1, g.n, !s, sen);
-            dside_load(Hb, d, wrap_inc(k, g.n), t + 1, g.n, !s, sbn);
-            rhn = ld_once<NT>(elem(rhoc, offn));
-            fvn = ld_once<NT>(elem(rhsc, offn));
-        }
-        const D2f de = d2_of(s19_win2(we, s, se, d)), db = d2_of(s19_win2(wb, s, sb, d));
-        const float D = dgp_dop(db, de, rh, c) - fv;
-        st_once<NT>(elem(out, off), de.c0 + D / (6.0f * c.inv_dx2));
-        if (t + 1 < DGP_KC) {
-            dwin2_shift(we);
-            dwin2_shift(wb);
-            dwin2_set(we, 2, re);
-            dwin2_set(wb, 2, rb);
-            se = sen;
-            sb = sbn;
-            off = offn;
-            rh = rhn;
-            fv = fvn;
-        }
-    }
 }
 
 template <bool NT>

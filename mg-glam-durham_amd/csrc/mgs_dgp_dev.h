@@ -9,6 +9,7 @@
 #include <cmath>
 
 #include "mgs_device.h"
+#include "mgs_fr_dev.h"
 #include "mgs_internal.h"
 #include "mgs_stencil.h"
 
@@ -27,34 +28,46 @@ struct S19 {
     T yz_pp, yz_mm, yz_pm, yz_mp;  // (i, j+-1, k+-1)
 };
 
+// the stencil of cell (i, j, k) from a field's colour halves
 template <typename T>
-__device__ __forceinline__ S19<T> s19_at(const T* __restrict__ u, const Geo& g, int i, int j, int k)
+__device__ __forceinline__ S19<T> s19_halves(const T* __restrict__ h0, const T* __restrict__ h1, const Geo& g, int i,
+                                             int j, int k)
 {
     const int n = g.n;
     const int im = wrap_dec(i, n), ip = wrap_inc(i, n);
     const int jm = wrap_dec(j, n), jp = wrap_inc(j, n);
     const int km = wrap_dec(k, n), kp = wrap_inc(k, n);
+    // the cell's own colour and the other (n is even: a wrap keeps the parity)
+    const bool c = (i + j + k) & 1;
+    const T *a = c ? h1 : h0, *b = c ? h0 : h1;
+    auto at = [&](const T* h, int x, int y, int z) { return h[row_base(g, y, z) + (unsigned)(x >> 1)]; };
     S19<T> s;
-    s.c0 = u[split_index(g, i, j, k)];
-    s.xp = u[split_index(g, ip, j, k)];
-    s.xm = u[split_index(g, im, j, k)];
-    s.yp = u[split_index(g, i, jp, k)];
-    s.ym = u[split_index(g, i, jm, k)];
-    s.zp = u[split_index(g, i, j, kp)];
-    s.zm = u[split_index(g, i, j, km)];
-    s.xy_pp = u[split_index(g, ip, jp, k)];
-    s.xy_mm = u[split_index(g, im, jm, k)];
-    s.xy_pm = u[split_index(g, ip, jm, k)];
-    s.xy_mp = u[split_index(g, im, jp, k)];
-    s.xz_pp = u[split_index(g, ip, j, kp)];
-    s.xz_mm = u[split_index(g, im, j, km)];
-    s.xz_pm = u[split_index(g, ip, j, km)];
-    s.xz_mp = u[split_index(g, im, j, kp)];
-    s.yz_pp = u[split_index(g, i, jp, kp)];
-    s.yz_mm = u[split_index(g, i, jm, km)];
-    s.yz_pm = u[split_index(g, i, jp, km)];
-    s.yz_mp = u[split_index(g, i, jm, kp)];
+    s.c0 = at(a, i, j, k);
+    s.xp = at(b, ip, j, k);
+    s.xm = at(b, im, j, k);
+    s.yp = at(b, i, jp, k);
+    s.ym = at(b, i, jm, k);
+    s.zp = at(b, i, j, kp);
+    s.zm = at(b, i, j, km);
+    s.xy_pp = at(a, ip, jp, k);
+    s.xy_mm = at(a, im, jm, k);
+    s.xy_pm = at(a, ip, jm, k);
+    s.xy_mp = at(a, im, jp, k);
+    s.xz_pp = at(a, ip, j, kp);
+    s.xz_mm = at(a, im, j, km);
+    s.xz_pm = at(a, ip, j, km);
+    s.xz_mp = at(a, im, j, kp);
+    s.yz_pp = at(a, i, jp, kp);
+    s.yz_mm = at(a, i, jm, km);
+    s.yz_pm = at(a, i, jp, km);
+    s.yz_mp = at(a, i, jm, kp);
     return s;
+}
+
+template <typename T>
+__device__ __forceinline__ S19<T> s19_at(const T* __restrict__ u, const Geo& g, int i, int j, int k)
+{
+    return s19_halves(u, u + g.half, g, i, j, k);
 }
 
 // Sigma's stencil sums and the Laplacian numerator
@@ -154,18 +167,18 @@ __device__ __forceinline__ float dgp_dop(const D2f& b, const D2f& e, float rho, 
 // ---------------------------------------------------------------------------
 
 // one colour pass of the inner smoother at the cell (m, row = j + n k) of
-// colour `colour`, out of place into tmp (one colour half)
-__device__ __forceinline__ void dgpm_smooth_cell(const float* __restrict__ e, const float* __restrict__ pb,
-                                                 const double* __restrict__ rho, const float* __restrict__ rhs,
-                                                 float* __restrict__ tmp, const Geo& g, int colour, const DgpF& c,
-                                                 int m, unsigned row)
+// colour `colour`: the increment's halves e0, e1 in, the colour's new half out
+__device__ __forceinline__ void dgpm_smooth_cell(const float* __restrict__ e0, const float* __restrict__ e1,
+                                                 const float* __restrict__ pb, const double* __restrict__ rho,
+                                                 const float* __restrict__ rhs, float* __restrict__ out, const Geo& g,
+                                                 int colour, const DgpF& c, int m, unsigned row)
 {
     const int j = (int)(row % (unsigned)g.n), k = (int)(row / (unsigned)g.n);
     const int i = 2 * m + ((colour + j + k) & 1);
     const size_t me = (size_t)colour * g.half + row_base(g, j, k) + m;
-    const D2f de = d2_at(e, g, i, j, k), db = d2_at(pb, g, i, j, k);
+    const D2f de = d2_of(s19_halves(e0, e1, g, i, j, k)), db = d2_at(pb, g, i, j, k);
     const float D = dgp_dop(db, de, (float)rho[me], c) - rhs[me];
-    tmp[row_base(g, j, k) + m] = de.c0 + D / (6.0f * c.inv_dx2);
+    out[row_base(g, j, k) + m] = de.c0 + D / (6.0f * c.inv_dx2);
 }
 
 // out = D(e) - rhs at the cell (m, row2) of both colours (row2 < n^2:
@@ -675,8 +688,9 @@ struct DgpmOuterOp {
 };
 
 // the mixed inner residual out = D(e) - rhs (as dgpm_residual_cell, which
-// rounds the FP64 density to FP32: rho32 holds those values); no norm
-template <bool NT = false>
+// rounds the FP64 density to FP32: rho holds those values, or the FP64 ones);
+// no norm
+template <bool NT = false, typename R = float>
 struct DgpmResOp {
     using T = float;
     static constexpr int NF = 2;  // e, phi_b
@@ -685,18 +699,155 @@ struct DgpmResOp {
     };
     const float* e;
     const float* pb;
-    const float* rho32;
+    const R* rho;
     const float* rhs;
     float* out;
     DgpF c;
     unsigned hf;
     __device__ const float* half(int f, int colour) const { return (f ? pb : e) + (colour ? hf : 0u); }
-    __device__ __forceinline__ Own load(unsigned i) const { return Own{ld_once<NT>(rho32[i]), ld_once<NT>(rhs[i])}; }
+    __device__ __forceinline__ Own load(unsigned i) const { return Own{(float)ld_once<NT>(rho[i]), ld_once<NT>(rhs[i])}; }
     __device__ __forceinline__ double cell(unsigned i, const Own& o, const S19<float>* s) const
     {
         st_once<NT>(out[i], dgp_dop(d2_of(s[1]), d2_of(s[0]), o.rho, c) - o.rhs);
         return 0.0;
     }
 };
+
+// one colour of the mixed inner smoother (as dgpm_smooth_cell), z-marching from
+// plane k0.  S0: parity of the column's first cell (the same for a whole wave);
+// with the run unrolled the parity of every step is a constant, so the
+// stencil values are the window's registers themselves.  R: the density's
+// type (rounded to FP32 as it is used).
+template <bool S0, bool NT, typename R>
+__device__ __forceinline__ void dgpm_zsmooth_run(const float* __restrict__ e0, const float* __restrict__ e1,
+                                                 float* __restrict__ out, const float* __restrict__ pb,
+                                                 const R* __restrict__ rho, const float* __restrict__ rhs,
+                                                 const Geo& g, int colour, const DgpF& c, const DCol& d, int k0)
+{
+    // (j + k0) & 1 = S0 ^ colour: wave-uniform
+    const int par0 = (S0 ? 1 : 0) ^ (colour & 1);
+    const DHalves<float> He = dhalves(e0, e1, par0), Hb = dhalves(pb, pb + g.half, par0);
+    const R* rhoc = rho + (size_t)colour * g.half;
+    const float* rhsc = rhs + (size_t)colour * g.half;
+    DWin2<float> we, wb;
+    dwin2_init(we, He, d, k0, g.n);
+    dwin2_init(wb, Hb, d, k0, g.n);
+    DSide<float> se, sb;
+    dside_load(He, d, k0, 0, g.n, S0, se);
+    dside_load(Hb, d, k0, 0, g.n, S0, sb);
+    unsigned off = (unsigned)k0 * d.plane + d.rowoff[1] + d.m;
+    float rh = (float)ld_once<NT>(elem(rhoc, off));
+    float fv = ld_once<NT>(elem(rhsc, off));
+#pragma unroll
+    for (int t = 0; t < DGP_KC; t++) {
+        const int k = k0 + t;
+        const bool s = S0 ^ ((t & 1) != 0);
+        DRaw2<float> re, rb;
+        DSide<float> sen, sbn;
+        float rhn = 0.0f, fvn = 0.0f;
+        const unsigned offn = off + d.plane;
+        if (t + 1 < DGP_KC) {
+            const int kn = wrap_inc(k + 1, g.n);
+            draw2_load(He, d, kn, t + 2, re);
+            draw2_load(Hb, d, kn, t + 2, rb);
+            dside_load(He, d, wrap_inc(k, g.n), t + 1, g.n, !s, sen);
+            dside_load(Hb, d, wrap_inc(k, g.n), t + 1, g.n, !s, sbn);
+            rhn = (float)ld_once<NT>(elem(rhoc, offn));
+            fvn = ld_once<NT>(elem(rhsc, offn));
+        }
+        const D2f de = d2_of(s19_win2(we, s, se, d)), db = d2_of(s19_win2(wb, s, sb, d));
+        const float D = dgp_dop(db, de, rh, c) - fv;
+        st_once<NT>(elem(out, off), de.c0 + D / (6.0f * c.inv_dx2));
+        if (t + 1 < DGP_KC) {
+            dwin2_shift(we);
+            dwin2_shift(wb);
+            dwin2_set(we, 2, re);
+            dwin2_set(wb, 2, rb);
+            se = sen;
+            sb = sbn;
+            off = offn;
+            rh = rhn;
+            fv = fvn;
+        }
+    }
+}
+
+// The same correction z-marching over coarse columns, as k_df_correct: planes
+// of e = e_H - R e_h in registers (x-neighbours from the adjacent lanes), all
+// 8 sons of a coarse cell, software-pipelined (plane K's sons computed, the
+// loads of plane K+1 issued, then plane K's sons stored).  Sums in
+// dgpm_correct_cell's order.
+template <int S3, bool NT>
+__device__ __forceinline__ void dgpm_sons_load(const float* __restrict__ ef, const Geo& gf, int I, int J, int K,
+                                               float* old)
+{
+#pragma unroll
+    for (int t = 0; t < 4; t++) old[t] = ld_once<NT>(elem(ef, son_index(gf, I, J, K, t & 1, t >> 1, S3)));
+}
+
+template <int S3>
+__device__ __forceinline__ void dgpm_sons_new(const float* ez, const float* ek, const float* old, float* nv)
+{
+    const float a = 1.0f / 64.0f, b = 3.0f * a, c9 = 9.0f * a, dd = 27.0f * a;
+    const float wt[8] = {a, b, b, c9, b, c9, c9, dd};
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int s1 = t & 1, s2 = t >> 1;
+        float P = 0.0f;
+#pragma unroll
+        for (int ind = 0; ind < 8; ind++) {
+            const int x = (ind & 1) ? 1 : (s1 ? 2 : 0);
+            const int y = (ind & 2) ? 1 : (s2 ? 2 : 0);
+            P += wt[ind] * ((ind & 4) ? ek[x + 3 * y] : ez[x + 3 * y]);
+        }
+        nv[t] = old[t] + P;
+    }
+}
+
+template <int S3, bool NT>
+__device__ __forceinline__ void dgpm_sons_store(float* __restrict__ ef, const Geo& gf, int I, int J, int K,
+                                                const float* nv)
+{
+#pragma unroll
+    for (int t = 0; t < 4; t++) st_once<NT>(elem(ef, son_index(gf, I, J, K, t & 1, t >> 1, S3)), nv[t]);
+}
+
+template <bool SHFL, bool NT>
+__device__ __forceinline__ void dgpm_correct_col(const float* __restrict__ eH, const float* __restrict__ rd,
+                                                 float* __restrict__ ef, const Geo& gf, const Geo& gc, const ZCol& cc,
+                                                 bool lok = false, bool rok = false)
+{
+    const int I = cc.m, J = cc.j;
+    Block9 B;
+    B.init(gc, I, J);
+    ERaw wm, wk, wp;  // coarse planes K-1, K, K+1
+    float o0[4], o1[4];
+    e_load<SHFL>(eH, rd, B, wrap_dec(cc.k0, gc.n), lok, rok, wm);
+    e_load<SHFL>(eH, rd, B, cc.k0, lok, rok, wk);
+    e_load<SHFL>(eH, rd, B, wrap_inc(cc.k0, gc.n), lok, rok, wp);
+    dgpm_sons_load<0, NT>(ef, gf, I, J, cc.k0, o0);
+    dgpm_sons_load<1, NT>(ef, gf, I, J, cc.k0, o1);
+    float em[9], ek[9], ep[9];
+    e_form<SHFL>(wm, lok, rok, em);
+    e_form<SHFL>(wk, lok, rok, ek);
+    for (int K = cc.k0; K < cc.k1; K++) {
+        e_form<SHFL>(wp, lok, rok, ep);
+        float n0[4], n1[4];
+        dgpm_sons_new<0>(em, ek, o0, n0);
+        dgpm_sons_new<1>(ep, ek, o1, n1);
+        if (K + 1 < cc.k1) {
+            dgpm_sons_load<0, NT>(ef, gf, I, J, K + 1, o0);
+            dgpm_sons_load<1, NT>(ef, gf, I, J, K + 1, o1);
+            e_load<SHFL>(eH, rd, B, wrap_inc(K + 1, gc.n), lok, rok, wp);
+        }
+        dgpm_sons_store<0, NT>(ef, gf, I, J, K, n0);
+        dgpm_sons_store<1, NT>(ef, gf, I, J, K, n1);
+#pragma unroll
+        for (int q = 0; q < 9; q++) {
+            em[q] = ek[q];
+            ek[q] = ep[q];
+        }
+    }
+}
 
 }  // namespace mgs

@@ -302,7 +302,8 @@ __global__ __launch_bounds__(1024) void k_df_coarsest(float* __restrict__ d, con
 template <int FRN>
 __global__ __launch_bounds__(TAIL_THREADS) void k_df_tail(TailDesc T)
 {
-    df_tail_vcycle<FRN>(T);
+    __shared__ float lds[TAIL_LDS_FLOATS];
+    df_tail_vcycle<FRN>(T, lds);
 }
 
 template <int FRN, int BX, int BY, int BZ, int NTHR>
@@ -678,11 +679,7 @@ void launch_df_correct(int frn, const float* dH, const float* rd, float* dfine, 
 
 bool launch_df_tail(int frn, int nlev, const TailLevelIn* lv, hipStream_t s)
 {
-    if (nlev < 2 || nlev > TAIL_MAXL) return false;
-    long lds = 0;  // the LDS copies: d, xb, g of the first level, d, xb, g, rres, rd below
-    for (int i = 0; i < nlev; i++) lds += (i == 0 ? 3L : 5L) * lv[i].n * lv[i].n * lv[i].n;
-    if (lds > TAIL_LDS_FLOATS) return false;
-    if ((long)lv[0].n * lv[0].n * lv[0].n > 2L * TAIL_CELLS * TAIL_THREADS) return false;
+    if (!df_tail_fits(lv[0].n, nlev)) return false;
     TailDesc T;
     T.nl = nlev - 1;
     for (int i = 0; i < nlev; i++) {

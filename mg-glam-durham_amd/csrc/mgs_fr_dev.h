@@ -1006,6 +1006,17 @@ struct TailDesc {
     TailLevel L[TAIL_MAXL];
 };
 
+// nlev levels from n cells a side fit the tail: the LDS copies (d, xb, g of
+// the first level, d, xb, g, rres, rd below) and the cells per thread
+inline bool df_tail_fits(int n, int nlev)
+{
+    if (nlev < 2 || nlev > TAIL_MAXL) return false;
+    if ((long)n * n * n > 2L * TAIL_CELLS * TAIL_THREADS) return false;
+    long lds = 0;
+    for (int i = 0; i < nlev; i++) lds += (i == 0 ? 3L : 5L) * (n >> i) * (n >> i) * (n >> i);
+    return lds <= TAIL_LDS_FLOATS;
+}
+
 template <class OP>
 __device__ __forceinline__ void tail_cell_op(const OP& op, const Geo& g, int t)
 {
@@ -1126,9 +1137,8 @@ __device__ void df_tail_levels(const TailDesc& G, int i0, float* lds)
 }
 
 template <int FRN>
-__device__ void df_tail_vcycle(const TailDesc& G)
+__device__ __forceinline__ void df_tail_vcycle(const TailDesc& G, float* lds)
 {
-    __shared__ float lds[TAIL_LDS_FLOATS];
     const int tid = threadIdx.x, nthr = TAIL_THREADS;
     // every load issued before the first is used: one memory latency instead
     // of one per level and array

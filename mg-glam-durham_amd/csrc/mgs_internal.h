@@ -94,7 +94,7 @@ struct mgs_handle {
     // DGP: out-of-place colour pass target and per-block partials
     double* dgp_tmp = nullptr;     // a colour half of level 0 in FP64 (N^3 floats)
     double* dgp_rms = nullptr;
-    double* dgp_spare64 = nullptr;  // FP64 z-marching passes: second level-0 array
+    double* dgp_spare64 = nullptr;  // FP64: second array of the level-0 passes' ping-pong
     // FFT plans (density generator, power spectrum)
     void* fft = nullptr;
     // particles and the potential of the PM step (mgs_pm.hip)
@@ -161,8 +161,32 @@ int auto_inner_count(int inner_max, double res, double target, double res_prev, 
 bool reference_exit(const mgs_solve_opts& o, int iter, double res, double res1, double res2, bool* conv);
 
 // mgs_dgp.hip
+// Four colour passes (0, 1, 0, 1) out of place between a field `A` and a
+// second array `B`: pass `it` reads the field's halves h0, h1 and writes its
+// colour's new half to out; after the fourth the field is back in A.
+template <typename T>
+struct PingPong {
+    const T *h0, *h1;
+    T* out;
+};
+
+template <typename T>
+__host__ __device__ inline PingPong<T> ping_pong(T* A, T* B, size_t half, int it)
+{
+    switch (it) {
+    case 0: return PingPong<T>{A, A + half, B};
+    case 1: return PingPong<T>{B, A + half, B + half};
+    case 2: return PingPong<T>{B, B + half, A};
+    default: return PingPong<T>{A, B + half, A + half};
+    }
+}
+
 DgpCoef dgp_coefs(const mgs_params& p, int level);
 int dgp_alloc(mgs_handle* h);
+// one colour pass from the field's halves h0, h1 into out (the colour's new half)
+void launch_dgp_pass64(int level, const double* h0, const double* h1, double* out, const double* rho, const double* f,
+                       int n, int colour, const DgpCoef& c, hipStream_t s);
+// the same in place, through tmp (one colour half)
 void launch_dgp_smooth64(int level, double* u, const double* rho, const double* f, double* tmp, int n, int colour,
                          const DgpCoef& c, hipStream_t s);
 int launch_dgp_residual64(int level, const double* u, const double* rho, const double* f, double* res,
@@ -174,8 +198,9 @@ void launch_dgp_rhs64(const double* ru, const double* rho, const double* rres, d
 // mixed-precision DGP (FP32 delta-form inner problem)
 int launch_dgpm_outer(const double* u, const double* rho, float* g32, float* pb, float* e, double* partials, int n,
                       const DgpCoef& c, hipStream_t s);
-void launch_dgpm_smooth(float* e, const float* pb, const double* rho, const float* rhs, float* tmp, int n, int colour,
-                        const DgpCoef& c, hipStream_t s);
+// one colour pass from the increment's halves into out; rho32 as below
+void launch_dgpm_pass(const float* e0, const float* e1, float* out, const float* pb, const double* rho,
+                      const float* rho32, const float* rhs, int n, int colour, const DgpCoef& c, hipStream_t s);
 // rho32: the density rounded to FP32 (used on z-marching levels)
 void launch_dgpm_residual(const float* e, const float* pb, const double* rho, const float* rho32, const float* rhs,
                           float* out, int n, const DgpCoef& c, hipStream_t s);

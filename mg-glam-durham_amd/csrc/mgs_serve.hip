@@ -42,13 +42,17 @@
 #include "mgs_fr_dev.h"
 #include "mgs_internal.h"
 #include "mgs_kernels.h"
+#include "mgs_tail_dev.h"
 
 namespace mgs {
 namespace serve {
 
 constexpr int MAXS = 64;    // slots
 constexpr int MAXL = 11;    // levels of a hierarchy (ngrid <= 1024)
-constexpr int GRID = 8192;  // blocks of a batched stencil/transfer launch (tiles are walked, XCD-contiguous)
+constexpr int GRID = 8192;  // blocks of a batched level-0 launch (tiles are walked, XCD-contiguous)
+// and of one on level l: a level of all slots has an eighth of the cells of
+// the one above, and idle blocks cost a deep launch more than its work
+static int grid_of(int l) { return l == 0 ? GRID : (l == 1 ? GRID / 2 : GRID / 4); }
 constexpr int SWEEPS = 8;   // coarsest-level sweeps (as solve_mixed)
 
 struct Shape {
@@ -62,16 +66,23 @@ struct LevelDesc {
     Geo g;
     float *d, *xb, *f, *rres, *rd;
     DfCoef dc;
-    Shape z;   // stencil passes on this level
+    Shape z;   // stencil passes on this level (nDGP: z-marching levels only)
     Shape zb;  // both-colour passes on this level (residual-type)
     Shape zc;  // coarse-column transfers between this level and the next finer one (levels >= 1)
     // nDGP
     const double* rhol;  // FP64 density of this level
     DgpF gf;
+    int zm;              // passes and residuals z-march (dgp_zmarch)
 };
 
 struct SlotDesc {
     int frn, lc, model, zdgp;  // zdgp: nDGP outer residual on z-marching tiles (dgp_zmarch(ngrid))
+    // the level from which one workgroup runs the rest of the cycle: the
+    // tail's first level, or, without a tail (no level's chain fits it), lc
+    int bot;
+    bool tailed;
+    TailDesc tail;              // f(R)
+    PTailDesc<TailDgpm> dtail;  // nDGP
     double* u;
     const double* rho;
     double* partials;
@@ -87,8 +98,8 @@ struct SlotDesc {
 };
 
 // which requests take part in each batched launch, and prefix sums of their
-// tiles; lists at level l hold the requests with l < lc (standard V-cycle
-// step at l) or lc == l (coarsest solve at l)
+// tiles; lists at level l hold the requests with l < bot (standard V-cycle
+// step at l) or bot == l (the rest of the cycle in one workgroup)
 struct Plan {
     int nres;
     int res_slot[MAXS];
@@ -98,15 +109,21 @@ struct Plan {
     unsigned z_pre[MAXL][MAXS + 1];     // level-l stencil tiles
     unsigned zc_pre[MAXL][MAXS + 1];    // level-(l+1) coarse columns (transfers l <-> l+1)
     unsigned cell_pre[MAXL][MAXS + 1];  // level-(l+1) cells in blocks of 256
-    unsigned zn_pre[MAXL][MAXS + 1];    // level-(l+1) stencil tiles
+    unsigned zn_pre[MAXL][MAXS + 1];    // level-(l+1) stencil tiles (none where the tail starts there)
     int ncoarse[MAXL];
     int coarse_slot[MAXL][MAXS];
-    // nDGP requests, in blocks of 256 cells
+    // nDGP requests, in z-marching tiles where the level has them, else in
+    // blocks of 256 cells
     int nd[MAXL];
     int d_slot[MAXL][MAXS];
-    unsigned dh_pre[MAXL][MAXS + 1];  // level-l cells of one colour
-    unsigned df_pre[MAXL][MAXS + 1];  // level-l cells
-    unsigned dc_pre[MAXL][MAXS + 1];  // level-(l+1) cells
+    unsigned dh_pre[MAXL][MAXS + 1];  // a colour pass of level l
+    unsigned df_pre[MAXL][MAXS + 1];  // a residual of level l
+    unsigned dn_pre[MAXL][MAXS + 1];  // a residual of level l+1 (none where the tail starts there)
+    unsigned dc_pre[MAXL][MAXS + 1];  // level-(l+1) cells in blocks of 256
+    unsigned dz_pre[MAXL][MAXS + 1];  // level-(l+1) coarse columns
+    int ndb[MAXL];                    // base restricted from level l to l+1, l < lc
+    int db_slot[MAXL][MAXS];
+    unsigned db_pre[MAXL][MAXS + 1];  // level-(l+1) cells in blocks of 256
     int ndcoarse[MAXL];
     int dcoarse_slot[MAXL][MAXS];
     int nupd;
@@ -416,34 +433,41 @@ __global__ __launch_bounds__(256) void kb_correct(const SlotDesc* __restrict__ S
     }
 }
 
-// coarsest-level sweeps of the requests whose coarsest level is l, one
-// workgroup each
-__global__ __launch_bounds__(1024) void kb_coarsest(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l)
+// the rest of the cycle of the f(R) requests whose bottom level is l, one
+// workgroup each: the tail, or the coarsest-level sweeps
+__global__ __launch_bounds__(TAIL_THREADS) void kb_bottom(const SlotDesc* __restrict__ S, const Plan* __restrict__ P,
+                                                          int l)
 {
+    __shared__ float lds[TAIL_LDS_FLOATS];
     for (int i = blockIdx.x; i < P->ncoarse[l]; i += gridDim.x) {
         const SlotDesc& sd = S[P->coarse_slot[l][i]];
         const LevelDesc& L = sd.L[l];
-        FRN_SWITCH(sd.frn, df_coarsest_block<FRN>(L.d, L.xb, L.f, L.g, SWEEPS, L.dc));
+        if (sd.tailed) {
+            FRN_SWITCH(sd.frn, df_tail_vcycle<FRN>(sd.tail, lds));
+        } else {
+            FRN_SWITCH(sd.frn, df_coarsest_block<FRN>(L.d, L.xb, L.f, L.g, SWEEPS, L.dc));
+        }
         __syncthreads();
     }
 }
 
 // ---- nDGP (vcycle_inner_dgp's steps) ----------------------------------------
-// Each launch walks blocks of 256 cells of every participating request; the
-// cell bodies are those of the single-request kernels, so the order cells are
-// visited in does not change a value.
+// Each launch walks the z-marching tiles (levels with dgp_zmarch) or blocks of
+// 256 cells of every participating request; the column and cell bodies are
+// those of the single-request kernels, so the order cells are visited in does
+// not change a value.
 
-// body(request, cell) for every cell of the blocks of 256 cells listed by
-// the prefix sums `pre` of the requests `slots`
+// body(request, tile) for every tile listed by the prefix sums `pre` of the
+// requests `slots`
 template <typename Body>
-__device__ __forceinline__ void dgp_cells(const SlotDesc* __restrict__ S, const unsigned* pre, int count,
+__device__ __forceinline__ void dgp_tiles(const SlotDesc* __restrict__ S, const unsigned* pre, int count,
                                           const int* slots, Body body)
 {
     const unsigned total = pre[count];
     for (XcdTiles it(total); it.t < it.end; it.t += it.stride) {
         const unsigned t = it.t;
         const int i = find_slot(pre, count, t);
-        body(S[slots[i]], (t - pre[i]) * 256u + threadIdx.x);
+        body(S[slots[i]], t - pre[i]);
     }
 }
 
@@ -461,8 +485,9 @@ __device__ __forceinline__ Ijk ijk_of(int nc, unsigned cell)
 __global__ __launch_bounds__(256) void kbd_restrict_base(const SlotDesc* __restrict__ S, const Plan* __restrict__ P,
                                                          int l)
 {
-    dgp_cells(S, P->dc_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned cell) {
+    dgp_tiles(S, P->db_pre[l], P->ndb[l], P->db_slot[l], [&](const SlotDesc& sd, unsigned t) {
         const LevelDesc &F = sd.L[l], &C = sd.L[l + 1];
+        const unsigned cell = t * 256u + threadIdx.x;
         if (cell < (unsigned)(2 * C.g.half)) {
             const Ijk c = ijk_of(C.g.n, cell);
             restrict8_cell<float>(F.xb, C.xb, nullptr, F.g, C.g, c.I, c.J, c.K);
@@ -470,44 +495,63 @@ __global__ __launch_bounds__(256) void kbd_restrict_base(const SlotDesc* __restr
     });
 }
 
-// one colour pass of the inner smoother on level l, out of place into scr
+// colour pass `it` (0..3) of two pairs on level l, ping-ponging between d and
+// scr (a pass in place would need its half copied back: half the launches)
 __global__ __launch_bounds__(256) void kbd_smooth(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l,
-                                                  int colour)
+                                                  int it)
 {
-    dgp_cells(S, P->dh_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned cell) {
+    const int colour = it & 1;
+    dgp_tiles(S, P->dh_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned t) {
         const LevelDesc& L = sd.L[l];
+        const PingPong<float> q = ping_pong(L.d, sd.scr, L.g.half, it);
+        if (L.zm) {
+            ZCol c;
+            if (!tile_col(L.g, L.g.h, L.z, t, c)) return;
+            const DCol d = dcol_of(L.g, c.m, c.j);
+            if ((colour + c.j + c.k0) & 1)
+                dgpm_zsmooth_run<true, false>(q.h0, q.h1, q.out, L.xb, L.rhol, L.f, L.g, colour, L.gf, d, c.k0);
+            else
+                dgpm_zsmooth_run<false, false>(q.h0, q.h1, q.out, L.xb, L.rhol, L.f, L.g, colour, L.gf, d, c.k0);
+            return;
+        }
+        const unsigned cell = t * 256u + threadIdx.x;
         if (cell < (unsigned)L.g.half)
-            dgpm_smooth_cell(L.d, L.xb, L.rhol, L.f, sd.scr, L.g, colour, L.gf, (int)(cell % (unsigned)L.g.h),
+            dgpm_smooth_cell(q.h0, q.h1, L.xb, L.rhol, L.f, q.out, L.g, colour, L.gf, (int)(cell % (unsigned)L.g.h),
                              cell / (unsigned)L.g.h);
     });
 }
 
-// the pass's colour half back from scr
-__global__ __launch_bounds__(256) void kbd_copy(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l,
-                                                int colour)
+// out = D(e) - rhs on tile t of a level
+__device__ __forceinline__ void dgp_residual_tile(const LevelDesc& L, const float* e, const float* rhs, float* out,
+                                                  unsigned t)
 {
-    dgp_cells(S, P->dh_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned cell) {
-        const LevelDesc& L = sd.L[l];
-        if (cell < (unsigned)L.g.half) L.d[(size_t)colour * L.g.half + cell] = sd.scr[cell];
-    });
+    if (L.zm) {
+        ZCol c;
+        if (!tile_col(L.g, L.g.h, L.z, t, c)) return;
+        (void)dgp_both_zcol(DgpmResOp<false, double>{e, L.xb, L.rhol, rhs, out, L.gf, (unsigned)L.g.half}, L.g, c.m, c.j,
+                            c.k0);
+        return;
+    }
+    const unsigned cell = t * 256u + threadIdx.x;
+    if (cell < (unsigned)(2 * L.g.half))
+        dgpm_residual_cell(e, L.xb, L.rhol, rhs, out, L.g, L.gf, (int)(cell % (unsigned)L.g.h), cell / (unsigned)L.g.h);
 }
 
 // inner residual D(e) - f of level l into scr
 __global__ __launch_bounds__(256) void kbd_residual(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l)
 {
-    dgp_cells(S, P->df_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned cell) {
+    dgp_tiles(S, P->df_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned t) {
         const LevelDesc& L = sd.L[l];
-        if (cell < (unsigned)(2 * L.g.half))
-            dgpm_residual_cell(L.d, L.xb, L.rhol, L.f, sd.scr, L.g, L.gf, (int)(cell % (unsigned)L.g.h),
-                               cell / (unsigned)L.g.h);
+        dgp_residual_tile(L, L.d, L.f, sd.scr, t);
     });
 }
 
 // R r and R e of level l: rres, and rd and the start value d of level l+1
 __global__ __launch_bounds__(256) void kbd_restrict(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l)
 {
-    dgp_cells(S, P->dc_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned cell) {
+    dgp_tiles(S, P->dc_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned t) {
         const LevelDesc &F = sd.L[l], &C = sd.L[l + 1];
+        const unsigned cell = t * 256u + threadIdx.x;
         if (cell < (unsigned)(2 * C.g.half)) {
             const Ijk c = ijk_of(C.g.n, cell);
             restrict8_cell<float>(sd.scr, C.rres, nullptr, F.g, C.g, c.I, c.J, c.K);
@@ -519,42 +563,45 @@ __global__ __launch_bounds__(256) void kbd_restrict(const SlotDesc* __restrict__
 // FAS right-hand side of level l+1: f = D(R e) - R r
 __global__ __launch_bounds__(256) void kbd_rhs(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l)
 {
-    dgp_cells(S, P->dc_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned cell) {
+    dgp_tiles(S, P->dn_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned t) {
         const LevelDesc& C = sd.L[l + 1];
-        if (cell < (unsigned)(2 * C.g.half))
-            dgpm_residual_cell(C.rd, C.xb, C.rhol, C.rres, C.f, C.g, C.gf, (int)(cell % (unsigned)C.g.h),
-                               cell / (unsigned)C.g.h);
+        dgp_residual_tile(C, C.rd, C.rres, C.f, t);
     });
 }
 
 // coarse-grid correction of level l from level l+1
 __global__ __launch_bounds__(256) void kbd_correct(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l)
 {
-    dgp_cells(S, P->dc_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned cell) {
+    dgp_tiles(S, P->dz_pre[l], P->nd[l], P->d_slot[l], [&](const SlotDesc& sd, unsigned t) {
         const LevelDesc &F = sd.L[l], &C = sd.L[l + 1];
-        if (cell < (unsigned)(2 * C.g.half)) {
-            const Ijk c = ijk_of(C.g.n, cell);
-            dgpm_correct_cell(C.d, C.rd, F.d, F.g, C.g, c.I, c.J, c.K);
-        }
+        ZCol c;
+        if (tile_col(C.g, C.g.n, C.zc, t, c)) dgpm_correct_col<false, false>(C.d, C.rd, F.d, F.g, C.g, c);
     });
 }
 
 // phi += e on level 0
 __global__ __launch_bounds__(256) void kbd_update(const SlotDesc* __restrict__ S, const Plan* __restrict__ P)
 {
-    dgp_cells(S, P->upd_pre, P->nupd, P->upd_slot, [&](const SlotDesc& sd, unsigned cell) {
+    dgp_tiles(S, P->upd_pre, P->nupd, P->upd_slot, [&](const SlotDesc& sd, unsigned t) {
         const LevelDesc& L = sd.L[0];
+        const unsigned cell = t * 256u + threadIdx.x;
         if (cell < (unsigned)(2 * L.g.half)) sd.u[cell] = sd.u[cell] + (double)L.d[cell];
     });
 }
 
-// coarsest-level sweeps of the nDGP requests whose coarsest level is l
-__global__ __launch_bounds__(1024) void kbd_coarsest(const SlotDesc* __restrict__ S, const Plan* __restrict__ P, int l)
+// the rest of the cycle of the nDGP requests whose bottom level is l, one
+// workgroup each: the tail, or the coarsest-level sweeps
+__global__ __launch_bounds__(TAIL_THREADS) void kbd_bottom(const SlotDesc* __restrict__ S, const Plan* __restrict__ P,
+                                                           int l)
 {
+    __shared__ float lds[PTAIL_LDS<TailDgpm>];
     for (int i = blockIdx.x; i < P->ndcoarse[l]; i += gridDim.x) {
         const SlotDesc& sd = S[P->dcoarse_slot[l][i]];
         const LevelDesc& L = sd.L[l];
-        dgpm_coarsest_block(L.d, L.xb, L.rhol, L.f, sd.scr, L.g, SWEEPS, L.gf);
+        if (sd.tailed)
+            ptail_run<TailDgpm>(sd.dtail, lds);
+        else
+            dgpm_coarsest_block(L.d, L.xb, L.rhol, L.f, sd.scr, L.g, SWEEPS, L.gf);
         __syncthreads();
     }
 }
@@ -914,15 +961,34 @@ void fill_desc(SlotDesc& sd, const Hier& h, const mgs_params& p)
         L.f = h.f[l];
         L.rres = h.rres[l];
         L.rd = h.rd[l];
+        if (l > 0) L.zc = shape_of(make_zlaunch(L.g.n, L.g.n));
         if (dgp) {
             L.rhol = h.rhol[l];
             L.gf = dgpf(dgp_coefs(p, l));
+            L.zm = dgp_zmarch(L.g.n) ? 1 : 0;
+            if (L.zm) L.z = shape_of(make_zlaunch(L.g.h, L.g.n, DGP_KC));
             continue;
         }
         L.dc = df_coefs(p, l);
         L.z = shape_of(make_zlaunch(L.g));
         L.zb = shape_of(make_zlaunch_both(L.g));
-        if (l > 0) L.zc = shape_of(make_zlaunch(L.g.n, L.g.n));
+    }
+    // the tail, as mgs_solve's: the first level below the finest whose chain fits
+    sd.bot = h.lc;
+    sd.tailed = false;
+    for (int l = 1; l < h.lc && !sd.tailed; l++) {
+        const int n = h.N >> l, nlev = h.lc - l + 1;
+        if (n > TAIL_MAX_N || !(dgp ? ptail_fits(n, nlev) : df_tail_fits(n, nlev))) continue;
+        sd.bot = l;
+        sd.tailed = true;
+        sd.tail.nl = sd.dtail.nl = nlev - 1;
+        for (int i = 0; i < nlev; i++) {
+            const LevelDesc& L = sd.L[l + i];
+            if (dgp)
+                sd.dtail.L[i] = PTailLevel<TailDgpm>{L.g, L.d, L.f, nullptr, L.rres, L.rd, L.rhol, L.xb, L.gf};
+            else
+                sd.tail.L[i] = TailLevel{L.g, L.d, L.xb, L.f, L.rres, L.rd, L.dc};
+        }
     }
 }
 
@@ -1265,13 +1331,25 @@ void finish_starts(mgs_server* S)
 
 static unsigned blocks256(size_t cells) { return (unsigned)((cells + 255) / 256); }
 
-// participation lists of the next step; *dfr / *ddgp: the deepest f(R) /
-// nDGP hierarchy taking an inner cycle, -1 when there is none
-void build_plan(mgs_server* S, int* dfr, int* ddgp)
+// What a step's launch sequence depends on: per model the deepest bottom level
+// and the deepest hierarchy of the requests taking an inner cycle, -1 when
+// there is none
+struct Depths {
+    int bot[2] = {-1, -1}, lc[2] = {-1, -1};  // f(R), nDGP
+    void add(int m, const SlotDesc& sd)
+    {
+        bot[m] = std::max(bot[m], sd.bot);
+        lc[m] = std::max(lc[m], sd.lc);
+    }
+    int key() const { return (((bot[0] + 1) * 16 + lc[0] + 1) * 16 + bot[1] + 1) * 16 + lc[1] + 1; }
+};
+
+// participation lists of the next step
+void build_plan(mgs_server* S, Depths* D)
 {
     Plan& P = *S->hP;
     std::memset(&P, 0, sizeof(P));
-    *dfr = *ddgp = -1;
+    *D = Depths();
     auto add = [](int& n, int* slot, unsigned* pre, int i, unsigned tiles) {
         slot[n] = i;
         pre[n + 1] = pre[n] + tiles;
@@ -1289,22 +1367,28 @@ void build_plan(mgs_server* S, int* dfr, int* ddgp)
         if (sl.outer_now) add(P.nres, P.res_slot, P.res_pre, i, dgp ? sd.zo.NB : sd.L[0].zb.NB);
         if (sl.fresh) continue;
         if (dgp) {
-            *ddgp = std::max(*ddgp, sd.lc);
-            for (int l = 0; l < sd.lc; l++) {
+            D->add(1, sd);
+            auto residual_tiles = [&](int l) { return sd.L[l].zm ? sd.L[l].z.NB : blocks256(2 * sd.L[l].g.half); };
+            for (int l = 0; l < sd.lc; l++)
+                add(P.ndb[l], P.db_slot[l], P.db_pre[l], i, blocks256(2 * sd.L[l + 1].g.half));
+            for (int l = 0; l < sd.bot; l++) {
                 const int k = P.nd[l];
+                const LevelDesc &F = sd.L[l], &C = sd.L[l + 1];
                 P.d_slot[l][k] = i;
-                P.dh_pre[l][k + 1] = P.dh_pre[l][k] + blocks256(sd.L[l].g.half);
-                P.df_pre[l][k + 1] = P.df_pre[l][k] + blocks256(2 * sd.L[l].g.half);
-                P.dc_pre[l][k + 1] = P.dc_pre[l][k] + blocks256(2 * sd.L[l + 1].g.half);
+                P.dh_pre[l][k + 1] = P.dh_pre[l][k] + (F.zm ? F.z.NB : blocks256(F.g.half));
+                P.df_pre[l][k + 1] = P.df_pre[l][k] + residual_tiles(l);
+                P.dn_pre[l][k + 1] = P.dn_pre[l][k] + (sd.tailed && l + 1 == sd.bot ? 0u : residual_tiles(l + 1));
+                P.dc_pre[l][k + 1] = P.dc_pre[l][k] + blocks256(2 * C.g.half);
+                P.dz_pre[l][k + 1] = P.dz_pre[l][k] + C.zc.NB;
                 P.nd[l]++;
             }
-            P.dcoarse_slot[sd.lc][P.ndcoarse[sd.lc]++] = i;
+            P.dcoarse_slot[sd.bot][P.ndcoarse[sd.bot]++] = i;
             P.upd_slot[P.nupd] = i;
             P.upd_pre[P.nupd + 1] = P.upd_pre[P.nupd] + blocks256(2 * sd.L[0].g.half);
             P.nupd++;
             continue;
         }
-        *dfr = std::max(*dfr, sd.lc);
+        D->add(0, sd);
         const unsigned z0 = sd.L[0].z.NB;
         if (sl.ic > 0) add(P.nnf, P.nf_slot, P.nf_pre, i, z0);
         if (sl.ic == sl.inner - 1)
@@ -1316,7 +1400,7 @@ void build_plan(mgs_server* S, int* dfr, int* ddgp)
                 const unsigned nc = (unsigned)sd.L[l + 1].g.n;
                 add(P.nrb[l], P.rb_slot[l], P.rb_pre[l], i, (nc * nc * nc + 255u) / 256u);
             }
-        for (int l = 0; l < sd.lc; l++) {
+        for (int l = 0; l < sd.bot; l++) {
             const int k = P.ninner[l];
             const LevelDesc& C = sd.L[l + 1];
             const unsigned nc = (unsigned)C.g.n;
@@ -1324,19 +1408,20 @@ void build_plan(mgs_server* S, int* dfr, int* ddgp)
             P.z_pre[l][k + 1] = P.z_pre[l][k] + sd.L[l].z.NB;
             P.zc_pre[l][k + 1] = P.zc_pre[l][k] + C.zc.NB;
             P.cell_pre[l][k + 1] = P.cell_pre[l][k] + (nc * nc * nc + 255u) / 256u;
-            P.zn_pre[l][k + 1] = P.zn_pre[l][k] + C.zb.NB;
+            P.zn_pre[l][k + 1] = P.zn_pre[l][k] + (sd.tailed && l + 1 == sd.bot ? 0u : C.zb.NB);
             P.ninner[l]++;
         }
-        P.coarse_slot[sd.lc][P.ncoarse[sd.lc]++] = i;
+        P.coarse_slot[sd.bot][P.ncoarse[sd.bot]++] = i;
     }
 }
 
-// the inner V-cycle of every non-fresh f(R) request, recursing to `depth`
+// the inner V-cycle of every non-fresh f(R) request, recursing to the deepest
+// bottom level `depth`
 void vcycle_batched(mgs_server* S, int l, int depth)
 {
     hipStream_t s = S->s;
-    const dim3 G(GRID), B(256);
-    hipLaunchKernelGGL(kb_coarsest, dim3(MAXS), dim3(1024), 0, s, S->dS, S->dP, l);
+    const dim3 G(grid_of(l)), G1(grid_of(l + 1)), B(256);
+    if (l > 0) hipLaunchKernelGGL(kb_bottom, dim3(MAXS), dim3(TAIL_THREADS), 0, s, S->dS, S->dP, l);
     if (l >= depth) return;
     // pre-smoothing (level 0: in the first inner cycle of an outer iteration
     // the first colour-0 pass came with the outer residual)
@@ -1347,10 +1432,10 @@ void vcycle_batched(mgs_server* S, int l, int depth)
         else
             hipLaunchKernelGGL(kb_smooth, G, B, 0, s, S->dS, S->dP, l, it & 1);
     }
-    hipLaunchKernelGGL(kb_restrict_residual, G, B, 0, s, S->dS, S->dP, l);
-    hipLaunchKernelGGL(kb_rhs, G, B, 0, s, S->dS, S->dP, l);
+    hipLaunchKernelGGL(kb_restrict_residual, G1, B, 0, s, S->dS, S->dP, l);
+    hipLaunchKernelGGL(kb_rhs, G1, B, 0, s, S->dS, S->dP, l);
     vcycle_batched(S, l + 1, depth);
-    hipLaunchKernelGGL(kb_correct, G, B, 0, s, S->dS, S->dP, l);
+    hipLaunchKernelGGL(kb_correct, G1, B, 0, s, S->dS, S->dP, l);
     // post-smoothing (level 0: in the last inner cycle of an outer iteration
     // the last colour-1 pass is fused with the update)
     const int npost = l == 0 ? 2 * MIXED_POST0 - 1 : 4;
@@ -1366,57 +1451,51 @@ void vcycle_batched(mgs_server* S, int l, int depth)
 void vcycle_dgp(mgs_server* S, int l, int depth)
 {
     hipStream_t s = S->s;
-    const dim3 G(GRID), B(256);
-    hipLaunchKernelGGL(kbd_coarsest, dim3(MAXS), dim3(1024), 0, s, S->dS, S->dP, l);
+    const dim3 G(grid_of(l)), G1(grid_of(l + 1)), B(256);
+    if (l > 0) hipLaunchKernelGGL(kbd_bottom, dim3(MAXS), dim3(TAIL_THREADS), 0, s, S->dS, S->dP, l);
     if (l >= depth) return;
-    for (int it = 0; it < 4; it++) {
-        hipLaunchKernelGGL(kbd_smooth, G, B, 0, s, S->dS, S->dP, l, it & 1);
-        hipLaunchKernelGGL(kbd_copy, G, B, 0, s, S->dS, S->dP, l, it & 1);
-    }
+    for (int it = 0; it < 4; it++) hipLaunchKernelGGL(kbd_smooth, G, B, 0, s, S->dS, S->dP, l, it);
     hipLaunchKernelGGL(kbd_residual, G, B, 0, s, S->dS, S->dP, l);
     hipLaunchKernelGGL(kbd_restrict, G, B, 0, s, S->dS, S->dP, l);
-    hipLaunchKernelGGL(kbd_rhs, G, B, 0, s, S->dS, S->dP, l);
+    hipLaunchKernelGGL(kbd_rhs, G1, B, 0, s, S->dS, S->dP, l);
     vcycle_dgp(S, l + 1, depth);
-    hipLaunchKernelGGL(kbd_correct, G, B, 0, s, S->dS, S->dP, l);
-    for (int it = 0; it < 4; it++) {
-        hipLaunchKernelGGL(kbd_smooth, G, B, 0, s, S->dS, S->dP, l, it & 1);
-        hipLaunchKernelGGL(kbd_copy, G, B, 0, s, S->dS, S->dP, l, it & 1);
-    }
+    hipLaunchKernelGGL(kbd_correct, G1, B, 0, s, S->dS, S->dP, l);
+    for (int it = 0; it < 4; it++) hipLaunchKernelGGL(kbd_smooth, G, B, 0, s, S->dS, S->dP, l, it);
 }
 
 // one step: inner cycle + update of the non-fresh requests, then the outer
-// residual and its norm for all; dfr / ddgp < 0: no f(R) / nDGP inner cycle
-void enqueue_step(mgs_server* S, int dfr, int ddgp)
+// residual and its norm for all
+void enqueue_step(mgs_server* S, const Depths& D)
 {
     hipStream_t s = S->s;
-    if (dfr >= 0) {
-        for (int l = 0; l < dfr; l++)
-            hipLaunchKernelGGL(kb_restrict_base, dim3(GRID), dim3(256), 0, s, S->dS, S->dP, l);
-        vcycle_batched(S, 0, dfr);
+    if (D.bot[0] >= 0) {
+        for (int l = 0; l < D.lc[0]; l++)
+            hipLaunchKernelGGL(kb_restrict_base, dim3(grid_of(l)), dim3(256), 0, s, S->dS, S->dP, l);
+        vcycle_batched(S, 0, D.bot[0]);
     }
-    if (ddgp >= 0) {
-        for (int l = 0; l < ddgp; l++)
-            hipLaunchKernelGGL(kbd_restrict_base, dim3(GRID), dim3(256), 0, s, S->dS, S->dP, l);
-        vcycle_dgp(S, 0, ddgp);
+    if (D.bot[1] >= 0) {
+        for (int l = 0; l < D.lc[1]; l++)
+            hipLaunchKernelGGL(kbd_restrict_base, dim3(grid_of(l)), dim3(256), 0, s, S->dS, S->dP, l);
+        vcycle_dgp(S, 0, D.bot[1]);
         hipLaunchKernelGGL(kbd_update, dim3(GRID), dim3(256), 0, s, S->dS, S->dP);
     }
     hipLaunchKernelGGL(kb_outer_residual, dim3(GRID), dim3(256), 0, s, S->dS, S->dP);
     hipLaunchKernelGGL(kb_sums, dim3(MAXS), dim3(1024), 0, s, S->dS, S->dP, S->dsum);
 }
 
-int run_step(mgs_server* S, int dfr, int ddgp)
+int run_step(mgs_server* S, const Depths& D)
 {
     if (!S->o.use_graphs) {
-        enqueue_step(S, dfr, ddgp);
+        enqueue_step(S, D);
         return hipGetLastError() == hipSuccess ? 0 : MGS_E_HIP;
     }
-    const int key = (dfr + 1) * 64 + (ddgp + 1);
+    const int key = D.key();
     auto it = S->graphs.find(key);
     if (it == S->graphs.end()) {
         hipGraph_t g = nullptr;
         hipGraphExec_t ex = nullptr;
         if (hipStreamBeginCapture(S->s, hipStreamCaptureModeThreadLocal) != hipSuccess) return MGS_E_HIP;
-        enqueue_step(S, dfr, ddgp);
+        enqueue_step(S, D);
         if (hipStreamEndCapture(S->s, &g) != hipSuccess) return MGS_E_HIP;
         const hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
@@ -1471,14 +1550,15 @@ void worker_main(mgs_server* S)
         for (int i = 0; i < S->o.max_active; i++)
             if (S->slots[i].r && S->desc_dirty) fill_desc(S->hS[i], *S->slots[i].h, S->slots[i].r->p);
         const Clock::time_point ts = Clock::now();
-        int dfr = -1, ddgp = -1;
-        build_plan(S, &dfr, &ddgp);
+        Depths depths;
+        build_plan(S, &depths);
         int rc = 0;
-        if (hipMemcpyAsync(S->dS, S->hS, sizeof(SlotDesc) * MAXS, hipMemcpyHostToDevice, S->s) != hipSuccess ||
+        if ((S->desc_dirty && hipMemcpyAsync(S->dS, S->hS, sizeof(SlotDesc) * S->o.max_active, hipMemcpyHostToDevice,
+                                             S->s) != hipSuccess) ||
             hipMemcpyAsync(S->dP, S->hP, sizeof(Plan), hipMemcpyHostToDevice, S->s) != hipSuccess)
             rc = MGS_E_HIP;
         S->desc_dirty = false;
-        if (!rc) rc = run_step(S, dfr, ddgp);
+        if (!rc) rc = run_step(S, depths);
         if (!rc && hipMemcpyAsync(S->hsum, S->dsum, sizeof(double) * MAXS, hipMemcpyDeviceToHost, S->s) != hipSuccess)
             rc = MGS_E_HIP;
         // hS and hP are not touched again before the synchronization below

@@ -62,3 +62,23 @@ def test_fp64_cycles_match_the_oracle(N, model, n):
         assert np.array_equal(u, ref)
     else:  # the smoother's root is good to rtol 1e-13
         assert np.max(np.abs(u - ref)) <= 1e-12 * scale
+
+
+# nDGP: tail from 16 (32: directly below the finest level), per-cell passes
+# (64), z-marching tiles of one, two and four rows (256, 128) in one batch
+@pytest.mark.gpu
+def test_served_ndgp_equals_the_solve():
+    sizes = (32, 64, 128, 256, 16)
+    cfgs = [M.Config(N=N, model=M.MODEL_DGP, branch=1, box=float(N), h0rc=1.0, precision=M.PREC_MIXED) for N in sizes]
+    deltas = [O.lognormal_density(N, float(N), 1.0, seed=N).astype(np.float32) for N in sizes]
+    with M.Server(max_active=4) as srv:
+        tickets = [srv.submit(c, d, max_outer=6, exit_rule=M.EXIT_REFERENCE, res_conv=1e-8)
+                   for c, d in zip(cfgs, deltas)]
+        served = [srv.wait(t) for t in tickets]
+    for c, d, (u, res) in zip(cfgs, deltas, served):
+        print(f"[small levels] nDGP N={c.N}", flush=True)
+        with M.Solver(c) as S:
+            S.set_density(d)
+            rep = S.solve(mode=0, res_conv=1e-8, max_cycles=6)
+            assert rep["outer"] == res["outer"]
+            assert np.array_equal(S.get_field(), u), c.N
