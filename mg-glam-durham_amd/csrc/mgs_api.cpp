@@ -332,6 +332,21 @@ static void op_smooth2(mgs_handle* h, int l)
     }
 }
 
+// count partials summed (launch_sum_partials' order) into hsum[0].  hsum is
+// pinned memory that the device addresses, so the sum's own kernel writes it:
+// a copy behind it would be one more launch (3 us and its gap) in each
+// residual of a small grid.  In arena mode hsum is ordinary host memory.
+int sum_to_host(mgs_handle* h, const double* partials, int count)
+{
+    if (!h->use_arena) {
+        launch_sum_partials(partials, count, h->hsum, h->s);
+        return 0;
+    }
+    launch_sum_partials(partials, count, h->dsum, h->s);
+    HIPCHK(h, hipMemcpyAsync(h->hsum, h->dsum, sizeof(double), hipMemcpyDeviceToHost, h->s));
+    return 0;
+}
+
 // level-l residual, stored in res_l when store; rms returned when rms != null
 int op_residual(mgs_handle* h, int l, bool store, double* rms)
 {
@@ -352,8 +367,8 @@ int op_residual(mgs_handle* h, int l, bool store, double* rms)
                                    h->dgp_rms, h->s);
     prof_end(h);
     if (rms) {
-        launch_sum_partials(h->partials, nb, h->dsum, h->s);
-        HIPCHK(h, hipMemcpyAsync(h->hsum, h->dsum, sizeof(double), hipMemcpyDeviceToHost, h->s));
+        int rc = sum_to_host(h, h->partials, nb);
+        if (rc) return rc;
         HIPCHK(h, hipStreamSynchronize(h->s));
         *rms = std::sqrt(h->hsum[0] / n3d(v.n));
     }
@@ -694,25 +709,21 @@ static int restrict_base_all(mgs_handle* h)
         MGS_KC_RESTRICT);
 }
 
-// The outer norm's partials summed and copied to the host; with_base, the
-// base restriction (which only needs the level-0 base just written) is
-// enqueued behind the copy and the host waits for the copy alone, so that
+// The outer norm's partials summed for the host; with_base, the base
+// restriction (which only needs the level-0 base just written) is enqueued
+// behind the sum and the host waits for the sum alone, so that
 // the restriction runs while the host reads the norm and picks the next
 // inner count (an inner cycle, queued next, runs after it in stream order)
 static int finish_outer_norm(mgs_handle* h, int nb, bool with_base, double* rms)
 {
-    launch_sum_partials(h->partials, nb, h->dsum, h->s);
-    HIPCHK(h, hipMemcpyAsync(h->hsum, h->dsum, sizeof(double), hipMemcpyDeviceToHost, h->s));
+    int rc = sum_to_host(h, h->partials, nb);
+    if (rc) return rc;
     if (with_base && h->ev_norm) {
         HIPCHK(h, hipEventRecord(h->ev_norm, h->s));
-        int rc = restrict_base_all(h);
-        if (rc) return rc;
+        if ((rc = restrict_base_all(h))) return rc;
         HIPCHK(h, hipEventSynchronize(h->ev_norm));
     } else {
-        if (with_base) {
-            int rc = restrict_base_all(h);
-            if (rc) return rc;
-        }
+        if (with_base && (rc = restrict_base_all(h))) return rc;
         HIPCHK(h, hipStreamSynchronize(h->s));
     }
     *rms = std::sqrt(h->hsum[0] / n3d(h->L[0].n));
@@ -786,13 +797,13 @@ static int solve_plain(mgs_handle* h, const mgs_solve_opts& o, mgs_solve_report*
 // ---- nDGP: inner V-cycle on the FP32 increment e (see mgs_dgp.hip) ----------
 // 2 x Nsmth colour passes (0, 1, 0, 1) of the inner smoother on level l,
 // ping-ponging between e and the scratch array (a level-0 array of floats) and
-// ending in e
-static void dgpm_smooth4(mgs_handle* h, int l, int cls)
+// ending in e; without the first pass where the outer residual has taken it
+static void dgpm_smooth4(mgs_handle* h, int l, int cls, bool skip_first = false)
 {
     LevelF& v = h->M[l];
     const DgpCoef dc = dgp_coefs(h->p, l);
     const size_t half = (size_t)v.n * v.n * (v.n / 2);
-    for (int it = 0; it < 4; it++) {
+    for (int it = skip_first ? 1 : 0; it < 4; it++) {
         prof_begin(h, cls, 3.0 * n3d(v.n) * 4.0);
         const PingPong<float> q = ping_pong(v.d, (float*)h->dgp_tmp, half, it);
         launch_dgpm_pass(q.h0, q.h1, q.out, v.xb, h->L[l].rho, v.rho, v.f, v.n, it & 1, dc, h->s);
@@ -800,7 +811,7 @@ static void dgpm_smooth4(mgs_handle* h, int l, int cls)
     }
 }
 
-static int vcycle_inner_dgp(mgs_handle* h, int l);
+static int vcycle_inner_dgp(mgs_handle* h, int l, bool first = false);
 
 // the right-hand side of level l >= 1 and its inner V-cycle, from the
 // restricted residual and increment; the small levels in one launch
@@ -819,7 +830,7 @@ static int dgpm_from_restricted(mgs_handle* h, int l)
     return vcycle_inner_dgp(h, l);
 }
 
-static int vcycle_inner_dgp(mgs_handle* h, int l)
+static int vcycle_inner_dgp(mgs_handle* h, int l, bool first)
 {
     LevelF& v = h->M[l];
     LevelD& V = h->L[l];
@@ -833,7 +844,7 @@ static int vcycle_inner_dgp(mgs_handle* h, int l)
         prof_end(h);
         return 0;
     }
-    dgpm_smooth4(h, l, cls);
+    dgpm_smooth4(h, l, cls, l == 0 && first);
     LevelF& c = h->M[l + 1];
     prof_begin(h, l == 0 ? MGS_KC_RESTRICT : MGS_KC_COARSE, 6.0 * n3d(v.n) * s);
     launch_dgpm_residual(v.d, v.xb, V.rho, v.rho, v.f, v.res, v.n, dc, h->s);
@@ -929,7 +940,7 @@ static int fw_inner(mgs_handle* h, int l, int kind, bool first, bool last)
     return 0;
 }
 
-static int fw_inner_dgp(mgs_handle* h, int l, int kind);
+static int fw_inner_dgp(mgs_handle* h, int l, int kind, bool first = false);
 
 // nDGP coarse-grid correction of level l by a `kind` cycle on level l+1
 // (vcycle_inner_dgp's transfers)
@@ -959,12 +970,12 @@ static int dgp_cgc(mgs_handle* h, int l, int kind)
     return 0;
 }
 
-static int fw_inner_dgp(mgs_handle* h, int l, int kind)
+static int fw_inner_dgp(mgs_handle* h, int l, int kind, bool first)
 {
     if (l >= h->lc) return vcycle_inner_dgp(h, l);  // the coarsest solve
     const int cls = l == 0 ? MGS_KC_SMOOTH : MGS_KC_COARSE;
     int rc;
-    dgpm_smooth4(h, l, cls);
+    dgpm_smooth4(h, l, cls, l == 0 && first);
     if ((rc = dgp_cgc(h, l, kind == 1 ? 1 : 2))) return rc;
     dgpm_smooth4(h, l, cls);
     if ((rc = dgp_cgc(h, l, kind == 1 ? 0 : 2))) return rc;
@@ -977,7 +988,8 @@ static int outer_residual_dgp(mgs_handle* h, double* rms)
     LevelD& v = h->L[0];
     LevelF& m = h->M[0];
     prof_begin(h, MGS_KC_RESIDUAL, 28.0 * n3d(v.n));
-    const int nb = launch_dgpm_outer(v.u, v.rho, m.f, m.xb, m.d, h->partials, v.n, dgp_coefs(h->p, 0), h->s);
+    const int nb = launch_dgpm_outer(v.u, v.rho, m.f, m.xb, m.d, (float*)h->dgp_tmp, h->partials, v.n,
+                                     dgp_coefs(h->p, 0), h->s);
     prof_end(h);
     return finish_outer_norm(h, nb, true, rms);
 }
@@ -1070,7 +1082,7 @@ static int solve_mixed(mgs_handle* h, const mgs_solve_opts& o, mgs_solve_report*
             }
         } else {
             for (int ic = 0; ic < inner; ic++) {
-                if ((rc = o.cycle == 0 ? vcycle_inner_dgp(h, 0) : fw_inner_dgp(h, 0, o.cycle))) return rc;
+                if ((rc = o.cycle == 0 ? vcycle_inner_dgp(h, 0, ic == 0) : fw_inner_dgp(h, 0, o.cycle, ic == 0))) return rc;
                 cycles++;
             }
             prof_begin(h, MGS_KC_UPDATE, 20.0 * n3d(h->L[0].n));

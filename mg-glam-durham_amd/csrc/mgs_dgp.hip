@@ -379,16 +379,16 @@ __global__ __launch_bounds__(256) void k_dgpm_residual(const float* __restrict__
 }
 
 // FP64 outer residual r = L(phi) (partials of r^2), and the inner problem's
-// data: g = -r and phi_b = phi in FP32, e = 0
+// data (dgpm_outer_cell)
 __global__ __launch_bounds__(256) void k_dgpm_outer(const double* __restrict__ u, const double* __restrict__ rho,
                                                     float* __restrict__ g32, float* __restrict__ pb,
-                                                    float* __restrict__ e, double* __restrict__ partials, Geo g,
-                                                    DgpCoef c, int TX, int TY, int XB, unsigned NB)
+                                                    float* __restrict__ e, float* __restrict__ e0,
+                                                    double* __restrict__ partials, Geo g, DgpCoef c, int TX, int TY, int XB, unsigned NB)
 {
     int m;
     unsigned row;
     double acc = 0.0;
-    if (map_xy(g.h, 2L * g.n * g.n, TX, TY, XB, NB, m, row)) acc = dgpm_outer_cell(u, rho, g32, pb, e, g, c, m, row);
+    if (map_xy(g.h, 2L * g.n * g.n, TX, TY, XB, NB, m, row)) acc = dgpm_outer_cell(u, rho, g32, pb, e, e0, g, c, m, row);
     store_partial(partials, NB, block_sum(acc));
 }
 
@@ -424,18 +424,18 @@ __global__ __launch_bounds__(256) void k_dgpm_update(double* __restrict__ u, con
         st_once<NT>(u[i], ld_once<NT>(u[i]) + (double)ld_once<NT>(e[i]));
 }
 
-int launch_dgpm_outer(const double* u, const double* rho, float* g32, float* pb, float* e, double* partials, int n,
-                      const DgpCoef& c, hipStream_t s)
+int launch_dgpm_outer(const double* u, const double* rho, float* g32, float* pb, float* e, float* e0, double* partials,
+                      int n, const DgpCoef& c, hipStream_t s)
 {
     const Geo g = make_geo(n);
     if (dgp_zmarch(n)) {
         if (n >= NT_MIN_N)
-            return (int)launch_both_z(DgpmOuterOp<true>{u, rho, g32, pb, e, c, (unsigned)g.half}, partials, n, s);
-        return (int)launch_both_z(DgpmOuterOp<>{u, rho, g32, pb, e, c, (unsigned)g.half}, partials, n, s);
+            return (int)launch_both_z(DgpmOuterOp<true>{u, rho, g32, pb, e, e0, c, (unsigned)g.half}, partials, n, s);
+        return (int)launch_both_z(DgpmOuterOp<>{u, rho, g32, pb, e, e0, c, (unsigned)g.half}, partials, n, s);
     }
     const Launch L = make_launch(g.h, 2L * n * n);
-    hipLaunchKernelGGL(k_dgpm_outer, L.grid, L.block, 0, s, u, rho, g32, pb, e, partials, g, c, L.TX, L.TY, L.XB,
-                       L.NB);
+    hipLaunchKernelGGL(k_dgpm_outer, L.grid, L.block, 0, s, u, rho, g32, pb, e, e0, partials, g, c, L.TX, L.TY,
+                       L.XB, L.NB);
     return (int)L.NB;
 }
 

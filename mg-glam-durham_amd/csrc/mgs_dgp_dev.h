@@ -197,12 +197,19 @@ __device__ __forceinline__ void dgpm_residual_cell(const float* __restrict__ e, 
     out[me] = dgp_dop(d2_at(pb, g, i, j, k), d2_at(e, g, i, j, k), (float)rho[me], c) - rhs[me];
 }
 
+// The increment of a colour-0 cell after the inner smoother's first pass from
+// e = 0 (where D(0) = 0): 0 + (0 - rhs) / (6 / dx^2), as dgpm_smooth_cell
+// would form it.  The outer residual writes it, which saves that pass.
+__device__ __forceinline__ float dgpm_first(float rhs, float inv_dx2) { return (0.0f - rhs) / (6.0f * inv_dx2); }
+
 // FP64 outer residual r = L(phi) at the cell (m, row2) of both colours, and
-// the inner problem's data there (g = -r, phi_b = phi in FP32, e = 0); r^2
+// the inner problem's data there: g = -r, phi_b = phi in FP32, and the
+// increment after its first colour-0 pass from zero, as the ping-pong has it
+// then: colour 0 in e0 (the second array's half), colour 1 of e zero; r^2
 __device__ __forceinline__ double dgpm_outer_cell(const double* __restrict__ u, const double* __restrict__ rho,
                                                   float* __restrict__ g32, float* __restrict__ pb,
-                                                  float* __restrict__ e, const Geo& g, const DgpCoef& c, int m,
-                                                  unsigned row2)
+                                                  float* __restrict__ e, float* __restrict__ e0, const Geo& g,
+                                                  const DgpCoef& c, int m, unsigned row2)
 {
     const unsigned nn = (unsigned)g.n * (unsigned)g.n;
     const int col = row2 >= nn ? 1 : 0;
@@ -212,9 +219,13 @@ __device__ __forceinline__ double dgpm_outer_cell(const double* __restrict__ u, 
     const size_t me = (size_t)col * g.half + row_base(g, j, k) + m;
     double c0;
     const double OP = dgp_L(u, g, i, j, k, rho[me], c, c0);
-    g32[me] = (float)(-OP);
+    const float gv = (float)(-OP);
+    g32[me] = gv;
     pb[me] = (float)c0;
-    e[me] = 0.0f;
+    if (col == 0)
+        e0[me] = dgpm_first(gv, (float)c.inv_dx2);
+    else
+        e[me] = 0.0f;
     return OP * OP;
 }
 
@@ -660,7 +671,7 @@ struct DgpRes64Op {
 };
 
 // the mixed solve's FP64 outer residual r = L(phi), with the inner problem's
-// data g = -r, phi_b = phi (FP32) and e = 0 (as dgpm_outer_cell)
+// data g = -r, phi_b = phi (FP32) and e after its first pass (as dgpm_outer_cell)
 template <bool NT = false>
 struct DgpmOuterOp {
     using T = double;
@@ -673,6 +684,7 @@ struct DgpmOuterOp {
     float* g32;
     float* pb;
     float* e;
+    float* e0;
     DgpCoef c;
     unsigned hf;
     __device__ const double* half(int, int colour) const { return u + (colour ? hf : 0u); }
@@ -680,9 +692,13 @@ struct DgpmOuterOp {
     __device__ __forceinline__ double cell(unsigned i, const Own& o, const S19<double>* s) const
     {
         const double OP = dgp_L19(s[0], o.rho, c);
-        st_once<NT>(g32[i], (float)(-OP));
+        const float gv = (float)(-OP);
+        st_once<NT>(g32[i], gv);
         st_once<NT>(pb[i], (float)s[0].c0);
-        st_once<NT>(e[i], 0.0f);
+        if (i < hf)
+            st_once<NT>(e0[i], dgpm_first(gv, (float)c.inv_dx2));
+        else
+            st_once<NT>(e[i], 0.0f);
         return OP;
     }
 };

@@ -13,6 +13,7 @@
 
 #include <hipfft/hipfft.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -33,7 +34,7 @@ struct FftState {
     double* bins = nullptr;          // 6 (N/2 + 1): power, count, sum|m| of the linear and the log bins
     double* binpart = nullptr;       // BIN_BLOCKS such histograms, one per block
     int* logbin = nullptr;           // log bin of every |m|^2 = 0 .. 3 (N/2)^2
-    void* tables = nullptr;          // power-of-two Poisson solve: twiddles and Green's function
+    void* tables = nullptr;          // Poisson solve: (power-of-two grids) twiddles, then Green's function
 };
 
 // blocks of the binning kernel: each accumulates a private histogram in LDS
@@ -362,26 +363,31 @@ __global__ __launch_bounds__(256) void k_bin_reduce(const double* __restrict__ p
 // half-complex i = N - k.  The half spectrum (x fastest, N/2+1 of it) is
 // multiplied by trfi / A and by 1/N^3, hipFFT's transforms being
 // unnormalised where FFTPACK5's forward one divides by N per dimension.
-__global__ __launch_bounds__(256) void k_green(hipfftDoubleComplex* __restrict__ c, int N, double trfi,
-                                               double inv_n3)
+// One block row per (ky, kz): G from a table (three cosines and two 64-bit
+// divisions per entry took 84 us at 250^3).
+__global__ __launch_bounds__(256) void k_green(hipfftDoubleComplex* __restrict__ c, int N, double trfi, double inv_n3,
+                                               const double* __restrict__ green)
 {
-    const size_t nh = (size_t)(N / 2 + 1);
-    const size_t total = nh * N * N;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += stride) {
-        const int kx = (int)(q % nh);
-        const size_t r = q / nh;
-        const int ky = (int)(r % N), kz = (int)(r / N);
-        const double gx = green_g(kx, N), gy = green_g(ky, N), gz = green_g(kz, N);
-        double A = gy - 6.0;
-        A = gx + A;
-        A = A + gz;
-        if (fabs(A) < 1.0e-7) A = 1.0;
-        hipfftDoubleComplex v = c[q];
-        v.x = v.x * trfi / A * inv_n3;
-        v.y = v.y * trfi / A * inv_n3;
-        c[q] = v;
+    const unsigned nh = (unsigned)N / 2 + 1, rows = (unsigned)N * (unsigned)N;
+    for (unsigned r = blockIdx.x; r < rows; r += gridDim.x) {
+        const double gy = green[r % (unsigned)N] - 6.0, gz = green[r / (unsigned)N];
+        for (unsigned kx = threadIdx.x; kx < nh; kx += 256) {
+            double A = green[kx] + gy;
+            A = A + gz;
+            if (fabs(A) < 1.0e-7) A = 1.0;
+            const size_t q = (size_t)r * nh + kx;
+            hipfftDoubleComplex v = c[q];
+            v.x = v.x * trfi / A * inv_n3;
+            v.y = v.y * trfi / A * inv_n3;
+            c[q] = v;
+        }
     }
+}
+
+__global__ __launch_bounds__(256) void k_green_table(double* __restrict__ green, int N)
+{
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < N) green[k] = green_g(k, N);
 }
 
 __global__ __launch_bounds__(256) void k_to_f32(const double* __restrict__ a, float* __restrict__ b, size_t n)
@@ -427,9 +433,7 @@ static dim3 grid_for(size_t count)
 
 static int sum_blocks(mgs_handle* h, double* partials, int nblk, double* out)
 {
-    launch_sum_partials(partials, nblk, h->dsum, h->s);
-    if (hipMemcpyAsync(h->hsum, h->dsum, sizeof(double), hipMemcpyDeviceToHost, h->s) != hipSuccess ||
-        hipStreamSynchronize(h->s) != hipSuccess)
+    if (sum_to_host(h, partials, nblk) || hipStreamSynchronize(h->s) != hipSuccess)
         return set_err(h, MGS_E_HIP, "reduction copy");
     *out = h->hsum[0];
     return 0;
@@ -683,10 +687,15 @@ int mgs_potential(mgs_handle* h, double trfi)
     } else {
         if ((rc = fft_ensure(h)) || (rc = fft_ensure_inverse(h))) return rc;
         FftState* f = fft_of(h);
+        if (!f->tables) {
+            if ((rc = fft_alloc(h, &f->tables, (size_t)N * sizeof(double), "Green's function table"))) return rc;
+            hipLaunchKernelGGL(k_green_table, dim3((N + 255) / 256), dim3(256), 0, h->s, (double*)f->tables, N);
+        }
         prof_begin(h, MGS_KC_PM, 8.0 * n3 * 2.0 + 12.0 * n3);
         launch_unpack_f64_to_f64(h->L[0].rho, f->real, N, 1.0, h->s);
         if (hipfftExecD2Z(f->fwd, f->real, f->cplx) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecD2Z");
-        hipLaunchKernelGGL(k_green, grid_for((size_t)N * N * (N / 2 + 1)), dim3(256), 0, h->s, f->cplx, N, trfi, 1.0 / n3);
+        hipLaunchKernelGGL(k_green, dim3((unsigned)std::min(N * N, 65536)), dim3(256), 0, h->s, f->cplx, N, trfi, 1.0 / n3,
+                           (const double*)f->tables);
         if (hipfftExecZ2D(f->inv, f->cplx, f->real) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecZ2D");
         // FI is REAL*4 between the reference's transform passes and after them
         hipLaunchKernelGGL(k_to_f32, grid_for((size_t)n3), dim3(256), 0, h->s, f->real, phi, (size_t)n3);

@@ -147,6 +147,7 @@ void prof_begin(mgs_handle* h, int kc, double bytes);
 void prof_end(mgs_handle* h);
 int vcycle_plain(mgs_handle* h, int l);
 int op_residual(mgs_handle* h, int l, bool store, double* rms);
+int sum_to_host(mgs_handle* h, const double* partials, int count);
 int levelmax_of(int N);
 int levelmin_of(int N);
 // the parameter checks of mgs_create (0 or an MGS_E_* code with a reason)
@@ -196,8 +197,11 @@ void launch_dgp_restrict_residual1_64(const double* u0, const double* delta, dou
 void launch_dgp_rhs64(const double* ru, const double* rho, const double* rres, double* f, int n, const DgpCoef& c,
                       hipStream_t s);
 // mixed-precision DGP (FP32 delta-form inner problem)
-int launch_dgpm_outer(const double* u, const double* rho, float* g32, float* pb, float* e, double* partials, int n,
-                      const DgpCoef& c, hipStream_t s);
+// the outer residual with the inner problem's data; the increment comes after
+// its first colour-0 pass: colour 0 in e0 (one half of the passes' second
+// array), colour 1 zero in e
+int launch_dgpm_outer(const double* u, const double* rho, float* g32, float* pb, float* e, float* e0, double* partials,
+                      int n, const DgpCoef& c, hipStream_t s);
 // one colour pass from the increment's halves into out; rho32 as below
 void launch_dgpm_pass(const float* e0, const float* e1, float* out, const float* pb, const double* rho,
                       const float* rho32, const float* rhs, int n, int colour, const DgpCoef& c, hipStream_t s);

@@ -231,13 +231,13 @@ __global__ __launch_bounds__(256) void kb_outer_residual(const SlotDesc* __restr
         if (sd.model == MGS_MODEL_DGP && sd.zdgp) {
             ZCol c;
             if (tile_col(L.g, L.g.h, sd.zo, lb, c))
-                acc = dgp_both_zcol(DgpmOuterOp<true>{sd.u, sd.rho, L.f, L.xb, L.d, sd.gc0, (unsigned)L.g.half}, L.g,
+                acc = dgp_both_zcol(DgpmOuterOp<true>{sd.u, sd.rho, L.f, L.xb, L.d, sd.scr, sd.gc0, (unsigned)L.g.half}, L.g,
                                     c.m, c.j, c.k0);
         } else if (sd.model == MGS_MODEL_DGP) {
             int m;
             unsigned row;
             if (tile_xy(L.g.h, 2u * (unsigned)L.g.n * (unsigned)L.g.n, sd.zo, lb, m, row))
-                acc = dgpm_outer_cell(sd.u, sd.rho, L.f, L.xb, L.d, L.g, sd.gc0, m, row);
+                acc = dgpm_outer_cell(sd.u, sd.rho, L.f, L.xb, L.d, sd.scr, L.g, sd.gc0, m, row);
         } else {
             ZCol c;
             if (tile_col(L.g, L.g.h, L.zb, lb, c)) {
@@ -1087,7 +1087,7 @@ int start_request(mgs_server* S, Slot& sl, int slot)
     // order); they also set the first inner problem's g, xb and d
     int nb;
     if (h->model == MGS_MODEL_DGP)
-        nb = launch_dgpm_outer(h->u, h->rho, h->f[0], h->xb[0], h->d[0], h->partials, N, dgp_coefs(r->p, 0), cs);
+        nb = launch_dgpm_outer(h->u, h->rho, h->f[0], h->xb[0], h->d[0], h->scr, h->partials, N, dgp_coefs(r->p, 0), cs);
     else
         nb = launch_outer_residual(r->p.fr_n, h->u, h->rho, h->f[0], h->xb[0], h->d[0], h->partials, N,
                                    fr_coefs(r->p, 0), df_coefs(r->p, 0), false, cs);
@@ -1454,7 +1454,9 @@ void vcycle_dgp(mgs_server* S, int l, int depth)
     const dim3 G(grid_of(l)), G1(grid_of(l + 1)), B(256);
     if (l > 0) hipLaunchKernelGGL(kbd_bottom, dim3(MAXS), dim3(TAIL_THREADS), 0, s, S->dS, S->dP, l);
     if (l >= depth) return;
-    for (int it = 0; it < 4; it++) hipLaunchKernelGGL(kbd_smooth, G, B, 0, s, S->dS, S->dP, l, it);
+    // (level 0: every step is an outer iteration, whose first pass came with
+    // the outer residual)
+    for (int it = l == 0 ? 1 : 0; it < 4; it++) hipLaunchKernelGGL(kbd_smooth, G, B, 0, s, S->dS, S->dP, l, it);
     hipLaunchKernelGGL(kbd_residual, G, B, 0, s, S->dS, S->dP, l);
     hipLaunchKernelGGL(kbd_restrict, G, B, 0, s, S->dS, S->dP, l);
     hipLaunchKernelGGL(kbd_rhs, G1, B, 0, s, S->dS, S->dP, l);

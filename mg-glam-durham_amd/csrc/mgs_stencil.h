@@ -65,12 +65,13 @@ inline int zrun_length(int n)
     // measured at 512^3 (runs of 2, 4, 6, 8, 16, 32 planes): 4 is best; the
     // window's two prologue loads per run cost less than the lost
     // parallelism of longer runs.  At 256^3 (the 512^3 solve's level 1) runs
-    // of 2, 8 and 16 planes and 64-wide blocks are slower as well.  Up to 64^3
+    // of 2, 8 and 16 planes and 64-wide blocks are slower as well.  Up to 80^3
     // a run of 4 leaves CUs idle and puts four dependent cell updates in each
     // thread's chain: with single planes a 32^3 pass takes 2.6 us instead of
-    // 3.8 (mixed solves: 64^3 1255 -> 1095 us, 128^3 1790 -> 1590 us); at
-    // 128^3 single planes and pairs are slower than runs of 4.
-    return n > 64 ? 4 : 1;
+    // 3.8 (mixed solves: 64^3 1255 -> 1095 us, 128^3 1790 -> 1590 us; FP64
+    // 160^3 2.83 -> 2.71 ms); at 96^3 they are equal, at 128^3 single planes
+    // and pairs are slower than runs of 4.
+    return n > 80 ? 4 : 1;
 }
 
 // (TX x TY)-thread blocks over `width` columns x n rows, each thread marching
