@@ -32,7 +32,7 @@ struct FftState {
     double* real = nullptr;          // N^3 lexicographic
     hipfftDoubleComplex* cplx = nullptr;  // N*N*(N/2+1)
     double* bins = nullptr;          // 6 (N/2 + 1): power, count, sum|m| of the linear and the log bins
-    double* binpart = nullptr;       // BIN_BLOCKS such histograms, one per block
+    double* binpart = nullptr;       // SPECTRUM_BLOCKS such histograms, one per block
     int* logbin = nullptr;           // log bin of every |m|^2 = 0 .. 3 (N/2)^2
     void* tables = nullptr;          // Poisson solve: (power-of-two grids) twiddles, then Green's function
 };
@@ -65,6 +65,36 @@ static int fft_ensure_cplx(mgs_handle* h)
     return fft_alloc(h, (void**)&f->cplx, nc * sizeof(hipfftDoubleComplex), "FFT buffer");
 }
 
+__global__ __launch_bounds__(256) void k_green_table(double* __restrict__ green, int N)
+{
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < N) green[k] = green_g(k, N);
+}
+
+static int fft_ensure_bins(mgs_handle* h)
+{
+    FftState* f = fft_state(h);
+    const size_t len = 3 * (size_t)(f->N + 2) * sizeof(double);
+    const int rc = fft_alloc(h, (void**)&f->bins, len, "FFT bins");
+    return rc ? rc : fft_alloc(h, (void**)&f->binpart, SPECTRUM_BLOCKS * len, "FFT bins");
+}
+
+// power-of-two grids: twiddles and Green's function; others: the latter alone
+static int fft_ensure_tables(mgs_handle* h)
+{
+    FftState* f = fft_state(h);
+    const int N = f->N;
+    if (f->tables) return 0;
+    const bool pow2 = poisson_grid(N);
+    const int rc = fft_alloc(h, &f->tables, pow2 ? poisson_table_bytes(N) : (size_t)N * sizeof(double), "FFT tables");
+    if (rc) return rc;
+    if (pow2)
+        launch_poisson_tables(f->tables, N, h->s);
+    else
+        hipLaunchKernelGGL(k_green_table, dim3((N + 255) / 256), dim3(256), 0, h->s, (double*)f->tables, N);
+    return 0;
+}
+
 // the library's transforms and their buffers
 static int fft_ensure(mgs_handle* h)
 {
@@ -73,8 +103,6 @@ static int fft_ensure(mgs_handle* h)
     int rc;
     if ((rc = fft_ensure_cplx(h))) return rc;
     if ((rc = fft_alloc(h, (void**)&f->real, (size_t)N * N * N * sizeof(double), "FFT buffer"))) return rc;
-    if ((rc = fft_alloc(h, (void**)&f->bins, 3 * (size_t)(N + 2) * sizeof(double), "FFT bins"))) return rc;
-    if ((rc = fft_alloc(h, (void**)&f->binpart, (size_t)BIN_BLOCKS * 3 * (N + 2) * sizeof(double), "FFT bins"))) return rc;
     if (!f->have_fwd) {
         if (hipfftPlan3d(&f->fwd, N, N, N, HIPFFT_D2Z) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftPlan3d D2Z");
         f->have_fwd = true;
@@ -146,8 +174,6 @@ __global__ __launch_bounds__(256) void k_white_noise(double* __restrict__ w, siz
     }
 }
 
-__device__ __forceinline__ int fold(int a, int N) { return a <= N / 2 ? a : a - N; }
-
 // multiply the half spectrum by k^(slope/2) exp(-k^2 / (4 kc^2)), k = 0 -> 0
 __global__ __launch_bounds__(256) void k_filter(hipfftDoubleComplex* __restrict__ c, int N, double kf, double kc,
                                                 double slope)
@@ -196,15 +222,6 @@ __global__ __launch_bounds__(256) void k_lognormal(const double* __restrict__ g,
     }
 }
 
-// fifth-force potential of a cell with field value v
-__device__ __forceinline__ double psi_of(double v, int model, int frn, double fct, double inv_ubg)
-{
-    if (model == MGS_MODEL_DGP) return 0.5 * v;
-    const double x = v * inv_ubg;
-    const double w = frn == 0 ? x : (frn == 1 ? x * x : x * x * x);
-    return -fct * w;
-}
-
 // psi and its central differences, one thread per pair of cells (2m, 2m+1) of
 // a row, marching over a run of planes with psi of the planes k-1, k, k+1 in
 // registers: every access is a unit-stride run (the pairs of the rows beside
@@ -215,13 +232,12 @@ __device__ __forceinline__ double psi_of(double v, int model, int frn, double fc
 template <typename T>
 __global__ __launch_bounds__(256) void k_fifth_force(const double* __restrict__ u, T* __restrict__ psi,
                                                      T* __restrict__ gx, T* __restrict__ gy, T* __restrict__ gz, Geo g,
-                                                     int model, int frn, double fct, double inv_ubg, int TX, int TY,
-                                                     int XB, int JB, int KC, unsigned NB)
+                                                     PsiOf psi_of, int TX, int TY, int XB, int JB, int KC, unsigned NB)
 {
     ZCol c;
     if (!zcol(g, TX, TY, XB, JB, KC, NB, c)) return;
     const int n = g.n, j = c.j, m = c.m;
-    auto at = [&](size_t q) { return psi_of(u[q], model, frn, fct, inv_ubg); };
+    auto at = [&](size_t q) { return psi_of(u[q]); };
     typedef T V2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));  // a caller's array: aligned as its elements
     double pe, po, me = 0.0, mo = 0.0;  // planes k and k-1
     size_t e, o;
@@ -258,18 +274,9 @@ __global__ __launch_bounds__(256) void k_fifth_force(const double* __restrict__ 
     }
 }
 
-// POWERfft5's binning (PMP2mod_power.f90:359-410) of the half spectrum (x
-// fastest, N/2+1 of it; an entry stands for itself and, but at i = 0 and
-// i = N/2, its conjugate mirror), one private LDS histogram per block written
-// to part[block]: power, mode count and sum of |m| for the linear bins 1..N/2
-// (hist[0 .. nb)), then the same for the log bins (hist[3 nb .. 6 nb)).  |m|,
-// the bin boundaries and the weights are the reference's REAL*4 values (RK =
-// sqrt(REAL(|m|^2)) correctly rounded, as the compiled reference's is); the
-// log bin of each |m|^2 comes from a table the host fills with the C
-// library's log10f, the function the compiled reference calls.  The
-// quadrupole's line of sight is z: the reference fills its bins after the
-// I <-> K transposition (:307-316), so its MI is the z wavenumber.
-// LOGB: also fill the log bins (NGP only; skipped when no log output is asked for)
+// POWERfft5's binning (bin_mode) of the half spectrum of the library's
+// transform (x fastest, N/2+1 of it), one private LDS histogram per block
+// written to part[block]
 template <int IPOL, int ICIC, bool LOGB>
 __global__ __launch_bounds__(256) void k_bin_power(const hipfftDoubleComplex* __restrict__ c, int N, double norm,
                                                    const int* __restrict__ logbin, double* __restrict__ part, int nb)
@@ -284,55 +291,15 @@ __global__ __launch_bounds__(256) void k_bin_power(const hipfftDoubleComplex* __
         const int i = (int)(q % nh);
         const size_t r = q / nh;
         const int j = (int)(r % N), k = (int)(r / N);
-        const int my = fold(j, N), mz = fold(k, N);
-        const int n2 = i * i + my * my + mz * mz;
-        if (n2 == 0) continue;  // RK < 0.5: the mean
-        const float rk = sqrtf((float)n2);
-        const double w = (i == 0 || 2 * i == N) ? 1.0 : 2.0;  // conjugate half
-        double amp = (c[q].x * c[q].x + c[q].y * c[q].y) * norm;
-        if (IPOL) {
-            const float cosmu2 = (float)(mz * mz) / (rk * rk);
-            amp *= (double)(1.5f * cosmu2 - 0.5f);
-        }
-        if (ICIC) {
-            int mp = (int)(rk + 0.0001f);
-            if (mp < 1) mp = 1;
-            const int mp2 = mp + 1 < N ? mp + 1 : N;
-            const float w1 = (float)mp - rk + 1.0f;
-            const float w2 = 1.0f - w1;
-            const float d1 = (float)mp, d2 = d1 + 1.0f;
-            if (mp < nb) {
-                atomicAdd(&hist[mp], w * amp * (double)w1);
-                atomicAdd(&hist[nb + mp], w * (double)w1);
-                atomicAdd(&hist[2 * nb + mp], w * (double)(d1 * w1));
-            }
-            if (mp2 < nb) {
-                atomicAdd(&hist[mp2], w * amp * (double)w2);
-                atomicAdd(&hist[nb + mp2], w * (double)w2);
-                atomicAdd(&hist[2 * nb + mp2], w * (double)(d2 * w2));
-            }
-        } else {
-            int mp = (int)(rk + 0.5f);
-            if (mp < 1) mp = 1;
-            if (mp < nb) {
-                atomicAdd(&hist[mp], w * amp);
-                atomicAdd(&hist[nb + mp], w);
-                atomicAdd(&hist[2 * nb + mp], w * (double)rk);
-            }
-            const int ml = LOGB ? logbin[n2] : nb;
-            if (LOGB && ml < nb) {
-                if (!IPOL) atomicAdd(&hist[3 * nb + ml], w * amp);
-                atomicAdd(&hist[4 * nb + ml], w);
-                atomicAdd(&hist[5 * nb + ml], w * (double)rk);
-            }
-        }
+        bin_mode<IPOL, ICIC, LOGB>(hist, nb, N, i, fold(j, N), fold(k, N), (c[q].x * c[q].x + c[q].y * c[q].y) * norm,
+                                   logbin);
     }
     __syncthreads();
     double* out = part + (size_t)blockIdx.x * 6 * nb;
     for (int t = threadIdx.x; t < 6 * nb; t += blockDim.x) out[t] = hist[t];
 }
 
-// bins[t] = sum over blocks of part[block][t] (nblk = 512 of them): 16 bins of
+// bins[t] = sum over blocks of part[block][t] (some 500 of them): 16 bins of
 // 16 threads each per workgroup, a thread adding every 16th block's value, then
 // the 16 partial sums in order.  One thread per bin walked 512 dependent
 // additions in four workgroups (256^3: 127 us).
@@ -384,12 +351,6 @@ __global__ __launch_bounds__(256) void k_green(hipfftDoubleComplex* __restrict__
     }
 }
 
-__global__ __launch_bounds__(256) void k_green_table(double* __restrict__ green, int N)
-{
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k < N) green[k] = green_g(k, N);
-}
-
 __global__ __launch_bounds__(256) void k_to_f32(const double* __restrict__ a, float* __restrict__ b, size_t n)
 {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -407,8 +368,7 @@ __global__ __launch_bounds__(256) void k_to_f64(const float* __restrict__ a, dou
 // once, as FI = FI + sf does there
 // (one thread per pair of cells; 512^3: 387 us = 5.5 TB/s, one per cell 505)
 __global__ __launch_bounds__(256) void k_add_psi(float* __restrict__ phi, const double* __restrict__ u, Geo g,
-                                                 int model, int frn, double fct, double inv_ubg, int TX, int TY,
-                                                 int XB, unsigned NB)
+                                                 PsiOf psi_of, int TX, int TY, int XB, unsigned NB)
 {
     int m;
     unsigned row;
@@ -418,8 +378,8 @@ __global__ __launch_bounds__(256) void k_add_psi(float* __restrict__ phi, const 
     pair_split(g, m, j, k, e, o);
     Pair<float>* q = reinterpret_cast<Pair<float>*>(phi + ((size_t)row * g.n + 2 * (unsigned)m));
     Pair<float> v = *q;
-    v.a = (float)((double)v.a + psi_of(u[e], model, frn, fct, inv_ubg));
-    v.b = (float)((double)v.b + psi_of(u[o], model, frn, fct, inv_ubg));
+    v.a = (float)((double)v.a + psi_of(u[e]));
+    v.b = (float)((double)v.b + psi_of(u[o]));
     *q = v;
 }
 
@@ -429,6 +389,15 @@ static dim3 grid_for(size_t count)
     if (b > 16384) b = 16384;
     if (b < 1) b = 1;
     return dim3((unsigned)b);
+}
+
+// the fifth-force potential of the handle's model
+static PsiOf psi_of_handle(const mgs_handle* h)
+{
+    double ubg = 1.0;
+    const double fbg = fr_background(h->p, &ubg);
+    const double ctilde = 2.99792458e3 * (double)h->p.ngrid / h->p.box;
+    return PsiOf{h->p.model, h->p.fr_n, ctilde * ctilde * 0.5 * fbg, 1.0 / ubg};
 }
 
 static int sum_blocks(mgs_handle* h, double* partials, int nblk, double* out)
@@ -523,20 +492,17 @@ int mgs_fifth_force(mgs_handle* h, void* psi, void* gx, void* gy, void* gz, int3
             dev[a] = q;
         }
     }
-    double ubg = 1.0;
-    const double fbg = fr_background(h->p, &ubg);
-    const double ctilde = 2.99792458e3 * (double)N / h->p.box;
-    const double fct = ctilde * ctilde * 0.5 * fbg;
+    const PsiOf psi_of = psi_of_handle(h);
     prof_begin(h, MGS_KC_UPDATE, 0.0);
     const ZLaunch L = make_zlaunch(make_geo(N));
     if (dtype == MGS_F32)
         hipLaunchKernelGGL((k_fifth_force<float>), L.grid, L.block, 0, h->s, h->L[0].u, (float*)dev[0],
-                           (float*)dev[1], (float*)dev[2], (float*)dev[3], make_geo(N), h->p.model, h->p.fr_n, fct,
-                           1.0 / ubg, L.TX, L.TY, L.XB, L.JB, L.KC, L.NB);
+                           (float*)dev[1], (float*)dev[2], (float*)dev[3], make_geo(N), psi_of, L.TX, L.TY, L.XB, L.JB, L.KC,
+                           L.NB);
     else
         hipLaunchKernelGGL((k_fifth_force<double>), L.grid, L.block, 0, h->s, h->L[0].u, (double*)dev[0],
-                           (double*)dev[1], (double*)dev[2], (double*)dev[3], make_geo(N), h->p.model, h->p.fr_n,
-                           fct, 1.0 / ubg, L.TX, L.TY, L.XB, L.JB, L.KC, L.NB);
+                           (double*)dev[1], (double*)dev[2], (double*)dev[3], make_geo(N), psi_of, L.TX, L.TY, L.XB, L.JB,
+                           L.KC, L.NB);
     prof_end(h);
     int rc = 0;
     if (where == MGS_HOST)
@@ -572,10 +538,13 @@ int mgs_power_spectrum_ex(mgs_handle* h, int32_t which, int32_t ipol, int32_t ic
     if (which < 0 || which > 2) return set_err(h, MGS_E_ARG, "which must be 0 (delta), 1 (u) or 2 (psi)");
     if (ipol != 0 && ipol != 1) return set_err(h, MGS_E_ARG, "ipol must be 0 (monopole) or 1 (quadrupole)");
     if (icic != 0 && icic != 1) return set_err(h, MGS_E_ARG, "icic must be 0 (NGP bins) or 1 (linear bins)");
-    int rc = fft_ensure(h);
+    const int N = h->p.ngrid;
+    const bool pow2 = poisson_grid(N);  // transforms and binning of mgs_poisson.hip
+    int rc = pow2 ? fft_ensure_cplx(h) : fft_ensure(h);
+    if (!rc) rc = fft_ensure_bins(h);
+    if (!rc && pow2) rc = fft_ensure_tables(h);
     if (rc) return rc;
     FftState* f = fft_of(h);
-    const int N = h->p.ngrid;
     const size_t n3 = (size_t)N * N * N;
     const Geo g = make_geo(N);
     const int n2max = 3 * (N / 2) * (N / 2);
@@ -588,35 +557,38 @@ int mgs_power_spectrum_ex(mgs_handle* h, int32_t which, int32_t ipol, int32_t ic
             hipStreamSynchronize(h->s) != hipSuccess)
             return set_err(h, MGS_E_HIP, "log bin table copy");
     }
-    if (which == 0)
-        launch_unpack_f64_to_f64(h->L[0].rho, f->real, N, 1.0, h->s);
-    else if (which == 1)
-        launch_unpack_f64_to_f64(h->L[0].u, f->real, N, 1.0, h->s);
-    else {
-        double ubg = 1.0;
-        const double fbg = fr_background(h->p, &ubg);
-        const double ctilde = 2.99792458e3 * (double)N / h->p.box;
-        const ZLaunch L = make_zlaunch(g);
-        hipLaunchKernelGGL((k_fifth_force<double>), L.grid, L.block, 0, h->s, h->L[0].u, f->real,
-                           (double*)nullptr, (double*)nullptr, (double*)nullptr, g, h->p.model, h->p.fr_n,
-                           ctilde * ctilde * 0.5 * fbg, 1.0 / ubg, L.TX, L.TY, L.XB, L.JB, L.KC, L.NB);
-    }
-    if (hipfftExecD2Z(f->fwd, f->real, f->cplx) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecD2Z");
     const int nb = N / 2 + 1;  // bins 1..N/2 are returned
     const double norm = 1.0 / ((double)n3 * (double)n3);
-    const size_t lds = 6 * (size_t)nb * sizeof(double);
-    const dim3 G(BIN_BLOCKS), B(256);
-    if (icic)
-        hipLaunchKernelGGL((ipol ? k_bin_power<1, 1, false> : k_bin_power<0, 1, false>), G, B, lds, h->s, f->cplx, N,
-                           norm, (const int*)f->logbin, f->binpart, nb);
-    else if (logb)
-        hipLaunchKernelGGL((ipol ? k_bin_power<1, 0, true> : k_bin_power<0, 0, true>), G, B, lds, h->s, f->cplx, N,
-                           norm, (const int*)f->logbin, f->binpart, nb);
-    else
-        hipLaunchKernelGGL((ipol ? k_bin_power<1, 0, false> : k_bin_power<0, 0, false>), G, B, lds, h->s, f->cplx, N,
-                           norm, (const int*)f->logbin, f->binpart, nb);
+    const PsiOf psi = psi_of_handle(h);
+    int nblk = BIN_BLOCKS;
+    if (pow2) {
+        nblk = launch_spectrum(which == 0 ? h->L[0].rho : h->L[0].u, which == 2 ? &psi : nullptr, f->cplx, f->tables, N,
+                               norm, ipol, icic, logb, f->logbin, f->binpart, h->s);
+    } else {
+        if (which == 0)
+            launch_unpack_f64_to_f64(h->L[0].rho, f->real, N, 1.0, h->s);
+        else if (which == 1)
+            launch_unpack_f64_to_f64(h->L[0].u, f->real, N, 1.0, h->s);
+        else {
+            const ZLaunch L = make_zlaunch(g);
+            hipLaunchKernelGGL((k_fifth_force<double>), L.grid, L.block, 0, h->s, h->L[0].u, f->real, (double*)nullptr,
+                               (double*)nullptr, (double*)nullptr, g, psi, L.TX, L.TY, L.XB, L.JB, L.KC, L.NB);
+        }
+        if (hipfftExecD2Z(f->fwd, f->real, f->cplx) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecD2Z");
+        const size_t lds = 6 * (size_t)nb * sizeof(double);
+        const dim3 G(BIN_BLOCKS), B(256);
+        if (icic)
+            hipLaunchKernelGGL((ipol ? k_bin_power<1, 1, false> : k_bin_power<0, 1, false>), G, B, lds, h->s, f->cplx, N,
+                               norm, (const int*)f->logbin, f->binpart, nb);
+        else if (logb)
+            hipLaunchKernelGGL((ipol ? k_bin_power<1, 0, true> : k_bin_power<0, 0, true>), G, B, lds, h->s, f->cplx, N,
+                               norm, (const int*)f->logbin, f->binpart, nb);
+        else
+            hipLaunchKernelGGL((ipol ? k_bin_power<1, 0, false> : k_bin_power<0, 0, false>), G, B, lds, h->s, f->cplx, N,
+                               norm, (const int*)f->logbin, f->binpart, nb);
+    }
     hipLaunchKernelGGL(k_bin_reduce, dim3((6 * nb + 15) / 16), dim3(256), 0, h->s, (const double*)f->binpart,
-                       BIN_BLOCKS, 6 * nb, f->bins);
+                       nblk, 6 * nb, f->bins);
     std::vector<double> hb(6 * (size_t)nb);
     if (hipMemcpyAsync(hb.data(), f->bins, hb.size() * sizeof(double), hipMemcpyDeviceToHost, h->s) != hipSuccess ||
         hipStreamSynchronize(h->s) != hipSuccess)
@@ -661,10 +633,7 @@ static int potential_pow2(mgs_handle* h, float* phi, double trfi)
     if (rc) return rc;
     FftState* f = fft_of(h);
     const int N = f->N;
-    if (!f->tables) {
-        if ((rc = fft_alloc(h, &f->tables, poisson_table_bytes(N), "Poisson tables"))) return rc;
-        launch_poisson_tables(f->tables, N, h->s);
-    }
+    if ((rc = fft_ensure_tables(h))) return rc;
     launch_poisson(h->L[0].rho, f->cplx, phi, f->tables, N, trfi, h->s);
     return 0;
 }
@@ -687,10 +656,7 @@ int mgs_potential(mgs_handle* h, double trfi)
     } else {
         if ((rc = fft_ensure(h)) || (rc = fft_ensure_inverse(h))) return rc;
         FftState* f = fft_of(h);
-        if (!f->tables) {
-            if ((rc = fft_alloc(h, &f->tables, (size_t)N * sizeof(double), "Green's function table"))) return rc;
-            hipLaunchKernelGGL(k_green_table, dim3((N + 255) / 256), dim3(256), 0, h->s, (double*)f->tables, N);
-        }
+        if ((rc = fft_ensure_tables(h))) return rc;
         prof_begin(h, MGS_KC_PM, 8.0 * n3 * 2.0 + 12.0 * n3);
         launch_unpack_f64_to_f64(h->L[0].rho, f->real, N, 1.0, h->s);
         if (hipfftExecD2Z(f->fwd, f->real, f->cplx) != HIPFFT_SUCCESS) return set_err(h, MGS_E_HIP, "hipfftExecD2Z");
@@ -712,13 +678,10 @@ int mgs_potential_add_fifth_force(mgs_handle* h)
     if (!phi) return set_err(h, MGS_E_NOMEM, "potential buffer");
     const int N = h->p.ngrid;
     const size_t n3 = (size_t)N * N * N;
-    double ubg = 1.0;
-    const double fbg = fr_background(h->p, &ubg);
-    const double ctilde = 2.99792458e3 * (double)N / h->p.box;
     prof_begin(h, MGS_KC_PM, 16.0 * (double)n3);
     const Launch L = make_launch(N / 2, (long)N * N);
-    hipLaunchKernelGGL(k_add_psi, L.grid, L.block, 0, h->s, phi, h->L[0].u, make_geo(N), h->p.model, h->p.fr_n,
-                       ctilde * ctilde * 0.5 * fbg, 1.0 / ubg, L.TX, L.TY, L.XB, L.NB);
+    hipLaunchKernelGGL(k_add_psi, L.grid, L.block, 0, h->s, phi, h->L[0].u, make_geo(N), psi_of_handle(h), L.TX, L.TY,
+                       L.XB, L.NB);
     prof_end(h);
     if (hipStreamSynchronize(h->s) != hipSuccess) return set_err(h, MGS_E_HIP, "fifth-force potential");
     return 0;
