@@ -118,6 +118,54 @@ __device__ __forceinline__ void st_once(T& r, T v)
         r = v;
 }
 
+// Element `base` of an array, base the same for a whole wave, as a pointer in
+// scalar registers: ld_at(plane_ptr(a, base), i) is one access with a 32-bit
+// vector offset.  Left to itself the compiler hoists the vector sum a + i and
+// adds every base to it, a 64-bit vector add per access; the empty asm keeps
+// the scalar sum in one piece (and hides where the pointer comes from, so its
+// address space is spelled out).
+template <typename T>
+using Global = T __attribute__((address_space(1)));
+
+template <typename T>
+__device__ __forceinline__ Global<T>* plane_ptr(T* a, size_t base)
+{
+    const unsigned long long v = (unsigned long long)(a + base);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
+    unsigned long long u = ((unsigned long long)hi << 32) | lo;
+    asm("" : "+s"(u));
+    return reinterpret_cast<Global<T>*>(u);
+}
+
+template <bool NT = false, typename T>
+__device__ __forceinline__ T ld_at(Global<const T>* a, unsigned i)
+{
+    auto* p = reinterpret_cast<Global<const T>*>(reinterpret_cast<Global<const char>*>(a) + i * (unsigned)sizeof(T));
+    if constexpr (NT)
+        return __builtin_nontemporal_load(p);
+    else
+        return *p;
+}
+
+template <bool NT = false, typename T>
+__device__ __forceinline__ void st_at(Global<T>* a, unsigned i, T v)
+{
+    auto* p = reinterpret_cast<Global<T>*>(reinterpret_cast<Global<char>*>(a) + i * (unsigned)sizeof(T));
+    if constexpr (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
+// element i, i the same for a whole wave, of an array that this launch does not
+// write: a scalar load
+template <typename T>
+__device__ __forceinline__ T ld_scalar(const T* a, size_t i)
+{
+    return *reinterpret_cast<const T __attribute__((address_space(4)))*>((unsigned long long)(a + i));
+}
+
 // element i of a whole level's array (up to 2^30 cells): elem() where the
 // byte offset fits 32 bits for any index (4-byte elements), a[i] otherwise
 template <typename T>

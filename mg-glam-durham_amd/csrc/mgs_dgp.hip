@@ -13,8 +13,8 @@
 // sees the already-updated values of the edge neighbours that precede it in
 // memory order.  A parallel colour pass cannot reproduce that order; here
 // every cell of the colour is updated from the values the colour had before
-// the pass (the pass writes into a scratch half-array that is then copied
-// back).  The CPU oracle implements both orders (orc_dgp_smooth, lexi=0/1)
+// the pass: it writes them elsewhere, and a pair of passes moves the field to
+// its second array and on every second pair back.  The CPU oracle implements both orders (orc_dgp_smooth, lexi=0/1)
 // and both converge to the same discrete solution.
 
 #include <math.h>
@@ -513,8 +513,9 @@ template <bool COARSE, bool S0, bool NT>
 __device__ __forceinline__ void dgp_zsmooth64_run(const double* __restrict__ h0, const double* __restrict__ h1,
                                                   double* __restrict__ out, const double* __restrict__ rho,
                                                   const double* __restrict__ f, const Geo& g, int colour,
-                                                  const DgpCoef& c, const DCol& d, int k0)
+                                                  const DgpCoef& c, const DCol& d, int k0v)
 {
+    const int k0 = __builtin_amdgcn_readfirstlane(k0v);
     // (j + k0) & 1 = S0 ^ colour: wave-uniform
     const DHalves<double> H = dhalves(h0, h1, (S0 ? 1 : 0) ^ (colour & 1));
     const double* rhoc = rho + (size_t)colour * g.half;
@@ -524,35 +525,35 @@ __device__ __forceinline__ void dgp_zsmooth64_run(const double* __restrict__ h0,
     DSide<double> sd;
     dside_load(H, d, k0, 0, g.n, S0, sd);
     const double dLphi = -6.0 / c.dx2;
-    unsigned off = (unsigned)k0 * d.plane + d.rowoff[1] + d.m;
-    double rh = ld_once<NT>(elem(rhoc, off));
-    double fv = COARSE ? ld_once<NT>(elem(fc, off)) : 0.0;
+    const unsigned i = d.off[1];
+    size_t b = (size_t)((unsigned)k0 * d.plane);
+    double rh = ld_at<NT>(plane_ptr(rhoc, b), i);
+    double fv = COARSE ? ld_at<NT>(plane_ptr(fc, b), i) : 0.0;
 #pragma unroll
     for (int t = 0; t < DGP_KC; t++) {
         const int k = k0 + t;
         const bool s = S0 ^ ((t & 1) != 0);
         DRaw2<double> r;
-        DSide<double> sdn;
         double rhn = 0.0, fvn = 0.0;
-        const unsigned offn = off + d.plane;
+        const size_t bn = b + d.plane;
         if (t + 1 < DGP_KC) {
             draw2_load(H, d, wrap_inc(k + 1, g.n), t + 2, r);
-            dside_load(H, d, wrap_inc(k, g.n), t + 1, g.n, !s, sdn);
-            rhn = ld_once<NT>(elem(rhoc, offn));
-            if constexpr (COARSE) fvn = ld_once<NT>(elem(fc, offn));
+            rhn = ld_at<NT>(plane_ptr(rhoc, bn), i);
+            if constexpr (COARSE) fvn = ld_at<NT>(plane_ptr(fc, bn), i);
         }
-        const S19<double> u = s19_win2(w, s, sd, d);
+        const S19<double> u = s19_win2(w, s, sd);
+        if (t + 1 < DGP_KC) dside_load(H, d, wrap_inc(k, g.n), t + 1, g.n, !s, sd);
         double L = dgp_L19(u, rh, c);
         if constexpr (COARSE) L = L - fv;
-        st_once<NT>(elem(out, off), u.c0 - L / dLphi);
+        st_at<NT>(plane_ptr(out, b), i, u.c0 - L / dLphi);
         if (t + 1 < DGP_KC) {
             dwin2_shift(w);
             dwin2_set(w, 2, r);
-            sd = sdn;
-            off = offn;
+            b = bn;
             rh = rhn;
             fv = fvn;
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 

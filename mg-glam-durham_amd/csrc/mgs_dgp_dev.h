@@ -135,12 +135,40 @@ __device__ __forceinline__ D2f d2_at(const float* __restrict__ u, const Geo& g, 
 
 struct DgpF {
     float alpha, fct1, inv_dx2, inv_dx4, sgn;
+    float six, rsix;  // 6 / dx^2 and its reciprocal
 };
 
 inline DgpF dgpf(const DgpCoef& c)
 {
-    return DgpF{(float)c.alpha, (float)c.fct1, (float)(1.0 / c.dx2), (float)(1.0 / c.dx4),
-                (float)std::copysign(1.0, c.alpha)};
+    const float inv_dx2 = (float)(1.0 / c.dx2), six = 6.0f * inv_dx2;
+    return DgpF{(float)c.alpha, (float)c.fct1, inv_dx2, (float)(1.0 / c.dx4), (float)std::copysign(1.0, c.alpha),
+                six,            1.0f / six};
+}
+
+// The passes of the large levels are bound by the vector ALU (a cell is some
+// 200 instructions), so the quotient and the roots come without the scaling
+// steps that general ones carry for results or operands near the ends of the
+// FP32 range.
+
+// x / c.six, correctly rounded: two corrections by the exact remainder with the
+// correctly rounded reciprocal (the first leaves q within an ulp, where the
+// second is exact rounding).  Within a rounding of a denormal where |x| < 2^-100.
+__device__ __forceinline__ float over_six(float x, const DgpF& c)
+{
+    float q = x * c.rsix;
+    q = fmaf(fmaf(-q, c.six, x), c.rsix, q);
+    return fmaf(fmaf(-q, c.six, x), c.rsix, q);
+}
+
+// sqrt(x), x >= 0, correctly rounded for x >= 2^-100 (below, to an ulp): the
+// hardware's root is within an ulp, the neighbours' remainders pick the right one
+__device__ __forceinline__ float sqrt_pos(float x)
+{
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float lo = __int_as_float(__float_as_int(s) - 1), hi = __int_as_float(__float_as_int(s) + 1);
+    const float rl = fmaf(-lo, s, x), rh = fmaf(-hi, s, x);
+    const float t = rl <= 0.0f ? lo : s;
+    return rh > 0.0f ? hi : t;
 }
 
 // D(e) at a cell from the base's and the increment's second differences
@@ -155,10 +183,11 @@ __device__ __forceinline__ float dgp_dop(const D2f& b, const D2f& e, float rho, 
     const float cross = 2.0f * (b.xy * e.xy + b.xz * e.xz + b.yz * e.yz) + e.xy * e.xy + e.xz * e.xz + e.yz * e.yz;
     const float dSig = ((2.0f / 3.0f) * (lin + Qe) + 0.125f * cross) * c.inv_dx4;
     const float a2 = c.alpha * c.alpha;
-    const float So = sqrtf(fmaxf(a2 + (8.0f / 3.0f) * Sig, 0.0f));
-    const float Sn = sqrtf(fmaxf(a2 + (8.0f / 3.0f) * (Sig + dSig), 0.0f));
+    const float So = sqrt_pos(fmaxf(a2 + (8.0f / 3.0f) * Sig, 0.0f));
+    const float Sn = sqrt_pos(fmaxf(a2 + (8.0f / 3.0f) * (Sig + dSig), 0.0f));
     const float den = So + Sn;
-    const float nl = den > 0.0f ? 2.0f * c.sgn * dSig / den : 0.0f;
+    const bool ok = den > 0.0f;  // (a division per lane rather than a branch around it)
+    const float q = 2.0f * c.sgn * dSig / (ok ? den : 1.0f), nl = ok ? q : 0.0f;
     return (e.s6 - 6.0f * e.c0) * c.inv_dx2 - nl;
 }
 
@@ -178,7 +207,7 @@ __device__ __forceinline__ void dgpm_smooth_cell(const float* __restrict__ e0, c
     const size_t me = (size_t)colour * g.half + row_base(g, j, k) + m;
     const D2f de = d2_of(s19_halves(e0, e1, g, i, j, k)), db = d2_at(pb, g, i, j, k);
     const float D = dgp_dop(db, de, (float)rho[me], c) - rhs[me];
-    out[row_base(g, j, k) + m] = de.c0 + D / (6.0f * c.inv_dx2);
+    out[row_base(g, j, k) + m] = de.c0 + over_six(D, c);
 }
 
 // out = D(e) - rhs at the cell (m, row2) of both colours (row2 < n^2:
@@ -302,40 +331,52 @@ __device__ __forceinline__ void dgpm_coarsest_block(float* __restrict__ e, const
 // window (DWin2) holds, for planes k-1, k, k+1 and rows j-1, j, j+1, the
 // pair at x = 2m, 2m+1; with x = 2m-1 and 2m+2 at the five slots the
 // stencil reaches off the column (taken from the neighbouring lanes by a
-// shuffle, or loaded by the lane at the wave's edge), that is every point of
-// the 19-point stencil of the cell of either colour at (m, j, k).  A step
-// loads the pair at m of plane k+2 in the three rows (both colour halves at
-// one offset); plane k+2, the edge lanes' side values and the next cell's
-// own data are loaded before plane k is computed.  The stencil values go
-// through S19 like the per-cell kernels', so every result is bit-identical
-// to theirs.
+// shift; past the wave's edge by a scalar load), that is every point of the
+// 19-point stencil of the cell of either colour at (m, j, k).  A step loads
+// the pair at m of plane k+2 in the three rows (both colour halves at one
+// offset) and the next cell's own data before plane k is computed, the next
+// side values as soon as the present ones are in the stencils.  The stencil
+// values go through S19 like the per-cell kernels', so every result is
+// bit-identical to theirs.
+//
+// Bound by the vector ALU and by memory about equally, so the march itself
+// costs no vector instructions: planes move scalar base pointers, a row's
+// 32-bit offset stays in its register, and the value past the edge is the
+// shift's own operand for the lane that has no neighbour.  The barriers to the
+// scheduler keep it from raising every address sum of the unrolled run, which
+// spills scalar registers into vector lanes.  Instructions per cell: FP32 pass
+// 239 -> 175, FP32 residual 238 -> 177, FP64 residual 162 -> 111; at 512^3:
+// FP32 pass 456 -> 399 us (4.9 TB/s), FP32 residual 718 -> 610, FP64 outer
+// residual 880 -> 730 (5.1 TB/s).  Side values by vector loads: 459, 673 and
+// 1043; by scalar loads a whole plane ahead: 531, 882 and 738 (scalar
+// registers spill).
 //
 // The field is read through its two colour halves (h0, h1) and the pass
 // writes the new values of its colour to `out`, a half of a second array: a
 // pair of passes (colour 0, then colour 1 reading the new colour 0) moves
 // the field into the second array without the per-cell kernels' copy.
 struct DCol {
-    unsigned plane, m, mm, mp;
-    unsigned rowoff[3];
-    int jr[3];
-    bool lload, rload;
+    unsigned plane;
+    unsigned off[3];    // (m, row j-1..j+1) in a plane of a colour half
+    unsigned left[3];   // (first lane's m - 1, ...): wave-uniform
+    unsigned right[3];  // (last lane's m + 1, ...)
 };
 
 __device__ __forceinline__ DCol dcol_of(const Geo& g, int m, int j)
 {
     DCol d;
     d.plane = (unsigned)g.n * (unsigned)g.h;
-    d.m = (unsigned)m;
-    d.mm = (unsigned)(m == 0 ? g.h - 1 : m - 1);
-    d.mp = (unsigned)(m + 1 == g.h ? 0 : m + 1);
-    d.jr[0] = wrap_dec(j, g.n);
-    d.jr[1] = j;
-    d.jr[2] = wrap_inc(j, g.n);
+    // a wave is 64 consecutive m of one row
+    const int ma = __builtin_amdgcn_readfirstlane(m), mz = ma + 63, ju = __builtin_amdgcn_readfirstlane(j);
+    const unsigned mm = (unsigned)(ma == 0 ? g.h - 1 : ma - 1), mp = (unsigned)(mz + 1 == g.h ? 0 : mz + 1);
+    const int jr[3] = {wrap_dec(ju, g.n), ju, wrap_inc(ju, g.n)};
 #pragma unroll
-    for (int R = 0; R < 3; R++) d.rowoff[R] = (unsigned)d.jr[R] * (unsigned)g.h;
-    const unsigned lane = (threadIdx.x + threadIdx.y * blockDim.x) & 63u;
-    d.lload = lane == 0;
-    d.rload = lane == 63;
+    for (int R = 0; R < 3; R++) {
+        const unsigned row = (unsigned)jr[R] * (unsigned)g.h;
+        d.off[R] = row + (unsigned)m;
+        d.left[R] = row + mm;
+        d.right[R] = row + mp;
+    }
     return d;
 }
 
@@ -343,10 +384,9 @@ __device__ __forceinline__ DCol dcol_of(const Geo& g, int m, int j)
 // The cell of parity s needs the third x at five (plane, row) slots, q =
 // 0..4: (1,1), (1,0), (1,2), (0,1), (2,1): x = 2m-1 when s = 0 (the o value
 // of lane m-1) and x = 2m+2 when s = 1 (the e value of lane m+1), taken by a
-// shuffle at use.  A wave is 64 consecutive m of one row and plane, so s is
-// the same for all its lanes; only the edge lane on that side loads the five
-// values itself (DSide, one step ahead).  The stencil values are the same
-// numbers as DWin's, so results are bit-identical to its passes.
+// shift at use.  A wave is 64 consecutive m of one row and plane, so s is the
+// same for all its lanes, and so are the five values its edge lane on that
+// side needs (DSide).
 template <typename T>
 struct DWin2 {
     T e[3][3], o[3][3];  // [plane k-1, k, k+1][row j-1, j, j+1]: x = 2m, 2m+1
@@ -392,74 +432,27 @@ __device__ __forceinline__ DHalves<T> dhalves(const T* h0, const T* h1, int par0
 template <typename T>
 __device__ __forceinline__ void draw2_load(const DHalves<T>& H, const DCol& d, int K, int dk, DRaw2<T>& r)
 {
+    const size_t kp = (size_t)((unsigned)K * d.plane);
 #pragma unroll
     for (int R = 0; R < 3; R++) {
-        const unsigned idx = (unsigned)K * d.plane + d.rowoff[R] + d.m;
         const int f = (R + 1 + dk) & 1;
-        r.ev[R] = elem(H.p[f], idx);
-        r.ov[R] = elem(H.p[f ^ 1], idx);
+        r.ev[R] = ld_at(plane_ptr(H.p[f], kp), d.off[R]);
+        r.ov[R] = ld_at(plane_ptr(H.p[f ^ 1], kp), d.off[R]);
     }
 }
 
-// the five side values of the cell at plane k (dk = k - k0) with parity s
-// (edge lane only)
+// the five side values of the cell at plane k (dk = k - k0) with parity s:
+// x = 2m+2 has the colour of x = 2m, x = 2m-1 that of 2m+1
 template <typename T>
 __device__ __forceinline__ void dside_load(const DHalves<T>& H, const DCol& d, int k, int dk, int n, bool s,
                                            DSide<T>& sd)
 {
 #pragma unroll
-    for (int q = 0; q < 5; q++) sd.v[q] = T(0);
-    if (s ? d.rload : d.lload) {
-#pragma unroll
-        for (int q = 0; q < 5; q++) {
-            const int P = side_plane(q), R = side_row(q);
-            const int K = P == 0 ? wrap_dec(k, n) : (P == 2 ? wrap_inc(k, n) : k);
-            const unsigned base = (unsigned)K * d.plane + d.rowoff[R];
-            const int f = (R + P + dk) & 1;
-            // x = 2m+2 has the colour of x = 2m, x = 2m-1 that of 2m+1
-            sd.v[q] = s ? elem(H.p[f], base + d.mp) : elem(H.p[f ^ 1], base + d.mm);
-        }
-    }
-}
-
-// both sides at once, for passes that evaluate both cells of the pair: the
-// left edge lane loads x = 2m-1 (the side of the cell at 2m), the right edge
-// lane x = 2m+2 (the side of the cell at 2m+1), into the same five slots.
-// Measured at 512^3: FP64 windows run faster with one branch per edge
-// (scalar half bases); the two-field FP32 window of the mixed residual needs
-// 129 registers that way (three waves per SIMD, 10% slower) and 118 with
-// one branch choosing the half per lane.
-template <typename T>
-__device__ __forceinline__ void dside_load_edges(const DHalves<T>& H, const DCol& d, int k, int dk, int n,
-                                                 DSide<T>& sd)
-{
-#pragma unroll
-    for (int q = 0; q < 5; q++) sd.v[q] = T(0);
-    if constexpr (sizeof(T) == 8) {
-        if (d.lload) {
-#pragma unroll
-            for (int q = 0; q < 5; q++) {
-                const int P = side_plane(q), R = side_row(q);
-                const int K = P == 0 ? wrap_dec(k, n) : (P == 2 ? wrap_inc(k, n) : k);
-                sd.v[q] = elem(H.p[((R + P + dk) & 1) ^ 1], (unsigned)K * d.plane + d.rowoff[R] + d.mm);
-            }
-        } else if (d.rload) {
-#pragma unroll
-            for (int q = 0; q < 5; q++) {
-                const int P = side_plane(q), R = side_row(q);
-                const int K = P == 0 ? wrap_dec(k, n) : (P == 2 ? wrap_inc(k, n) : k);
-                sd.v[q] = elem(H.p[(R + P + dk) & 1], (unsigned)K * d.plane + d.rowoff[R] + d.mp);
-            }
-        }
-    } else if (d.lload || d.rload) {
-        const unsigned mo = d.rload ? d.mp : d.mm;
-#pragma unroll
-        for (int q = 0; q < 5; q++) {
-            const int P = side_plane(q), R = side_row(q);
-            const int K = P == 0 ? wrap_dec(k, n) : (P == 2 ? wrap_inc(k, n) : k);
-            const int f = (R + P + dk) & 1;
-            sd.v[q] = elem(d.rload ? H.p[f] : H.p[f ^ 1], (unsigned)K * d.plane + d.rowoff[R] + mo);
-        }
+    for (int q = 0; q < 5; q++) {
+        const int P = side_plane(q), R = side_row(q);
+        const unsigned kp = (unsigned)(P == 0 ? wrap_dec(k, n) : (P == 2 ? wrap_inc(k, n) : k)) * d.plane;
+        const int f = ((R + P + dk) & 1) ^ (s ? 0 : 1);
+        sd.v[q] = ld_scalar(H.p[f], (size_t)kp + (s ? d.right[R] : d.left[R]));
     }
 }
 
@@ -498,44 +491,40 @@ __device__ __forceinline__ void dwin2_init(DWin2<T>& w, const DHalves<T>& H, con
 }
 
 // the value of lane + 1 (FROM_RIGHT) or lane - 1 of the wave, by a DPP
-// whole-wave shift (wave_shl:1 / wave_shr:1); the last / first lane, which
-// has no such neighbour, keeps its own value
+// whole-wave shift (wave_shl:1 / wave_shr:1); the last / first lane, which has
+// no such neighbour, takes its own `edge`
 template <bool FROM_RIGHT>
-__device__ __forceinline__ int wave_shift1(int v)
+__device__ __forceinline__ int wave_shift1(int edge, int v)
 {
-    if constexpr (FROM_RIGHT)
-        return __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false);
-    else
-        return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false);
+    return __builtin_amdgcn_update_dpp(edge, v, FROM_RIGHT ? 0x130 : 0x138, 0xf, 0xf, false);
 }
 
 template <bool FROM_RIGHT>
-__device__ __forceinline__ float wave_shift1(float v)
+__device__ __forceinline__ float wave_shift1(float edge, float v)
 {
-    return __int_as_float(wave_shift1<FROM_RIGHT>(__float_as_int(v)));
+    return __int_as_float(wave_shift1<FROM_RIGHT>(__float_as_int(edge), __float_as_int(v)));
 }
 
 template <bool FROM_RIGHT>
-__device__ __forceinline__ double wave_shift1(double v)
+__device__ __forceinline__ double wave_shift1(double edge, double v)
 {
+    const unsigned long long a = (unsigned long long)__double_as_longlong(edge);
     const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-    const unsigned lo = (unsigned)wave_shift1<FROM_RIGHT>((int)(unsigned)u);
-    const unsigned hi = (unsigned)wave_shift1<FROM_RIGHT>((int)(unsigned)(u >> 32));
+    const unsigned lo = (unsigned)wave_shift1<FROM_RIGHT>((int)(unsigned)a, (int)(unsigned)u);
+    const unsigned hi = (unsigned)wave_shift1<FROM_RIGHT>((int)(unsigned)(a >> 32), (int)(unsigned)(u >> 32));
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 // the 19 stencil values of the cell of parity s (all lanes of the wave
 // execute the shifts)
 template <typename T>
-__device__ __forceinline__ S19<T> s19_win2(const DWin2<T>& w, bool s, const DSide<T>& sd, const DCol& d)
+__device__ __forceinline__ S19<T> s19_win2(const DWin2<T>& w, bool s, const DSide<T>& sd)
 {
-    const bool edge = s ? d.rload : d.lload;  // the lane whose neighbour is outside the wave keeps sd
     T v[5];
 #pragma unroll
     for (int q = 0; q < 5; q++) {
         const int P = side_plane(q), R = side_row(q);
-        const T sh = s ? wave_shift1<true>(w.e[P][R]) : wave_shift1<false>(w.o[P][R]);
-        v[q] = edge ? sd.v[q] : sh;
+        v[q] = s ? wave_shift1<true>(sd.v[q], w.e[P][R]) : wave_shift1<false>(sd.v[q], w.o[P][R]);
     }
     // x = i + dx at slot (P, R), i = 2m + s; q: the side slot of (P, R)
     auto X = [&](int P, int R, int dx, int q) -> T {
@@ -569,77 +558,91 @@ __device__ __forceinline__ S19<T> s19_win2(const DWin2<T>& w, bool s, const DSid
 // Both cells of the pair at (m, j) over the run [k0, k0 + DGP_KC), from one
 // window per field (OP::NF fields of type OP::T, colour halves
 // op.half(f, 0/1)).  Per plane the cell at x = 2m comes first, then x = 2m+1;
-// OP::load(index) loads a cell's own data, OP::cell(index, own, stencils)
-// returns a value whose square is accumulated (the sum is returned).  The
+// OP::load(colour, b, i) loads a cell's own data from element b + i of its
+// colour's half, OP::cell(colour, b, i, own, stencils) returns a value whose square is accumulated (the sum is returned).  The
 // next plane's window values and own data are loaded before a plane is
 // evaluated.
-template <class OP>
-__device__ __forceinline__ double dgp_both_zcol(const OP& op, const Geo& g, int m, int j, int k0)
+template <bool PAR0, class OP>
+__device__ __forceinline__ double dgp_both_run(const OP& op, const Geo& g, DCol d, int k0)
 {
+    // (32-bit offsets made in this block: the compiler then knows them as such)
+#pragma unroll
+    for (int R = 0; R < 3; R++) asm("" : "+v"(d.off[R]));
     using T = typename OP::T;
     using Own = typename OP::Own;
     constexpr int NF = OP::NF;
-    const DCol d = dcol_of(g, m, j);
-    const unsigned half = (unsigned)g.half;
-    const int par0 = __builtin_amdgcn_readfirstlane((j + k0) & 1);  // wave-uniform
     DHalves<T> H[NF];
     DWin2<T> w[NF];
-    DSide<T> sd[NF];
+    DSide<T> sl[NF], sr[NF];  // of the cells at x = 2m and 2m+1
 #pragma unroll
     for (int f = 0; f < NF; f++) {
-        H[f] = dhalves(op.half(f, 0), op.half(f, 1), par0);
+        H[f] = dhalves(op.half(f, 0), op.half(f, 1), PAR0);
         dwin2_init(w[f], H[f], d, k0, g.n);
-        dside_load_edges(H[f], d, k0, 0, g.n, sd[f]);
+        dside_load(H[f], d, k0, 0, g.n, false, sl[f]);
+        dside_load(H[f], d, k0, 0, g.n, true, sr[f]);
     }
-    unsigned off = (unsigned)k0 * d.plane + d.rowoff[1] + d.m;
-    unsigned par = (unsigned)((j + k0) & 1);  // colour of x = 2m
-    Own o0 = op.load(par * half + off), o1 = op.load((1u - par) * half + off);
+    const unsigned i = d.off[1];
+    size_t b = (size_t)((unsigned)k0 * d.plane);
+    Own o0 = op.load(PAR0, b, i), o1 = op.load(!PAR0, b, i);
     double acc = 0.0;
 #pragma unroll
     for (int t = 0; t < DGP_KC; t++) {
-        const int k = k0 + t;
+        const int k = k0 + t, kn = wrap_inc(k, g.n);
+        const bool par = PAR0 ^ ((t & 1) != 0);  // colour of x = 2m
+        const bool more = t + 1 < DGP_KC;
         DRaw2<T> r[NF];
-        DSide<T> sdn[NF];
         Own n0 = o0, n1 = o1;
-        const unsigned offn = off + d.plane, parn = par ^ 1u;
-        if (t + 1 < DGP_KC) {
+        if (more) {
 #pragma unroll
-            for (int f = 0; f < NF; f++) {
-                draw2_load(H[f], d, wrap_inc(k + 1, g.n), t + 2, r[f]);
-                dside_load_edges(H[f], d, wrap_inc(k, g.n), t + 1, g.n, sdn[f]);
-            }
-            n0 = op.load(parn * half + offn);
-            n1 = op.load((1u - parn) * half + offn);
+            for (int f = 0; f < NF; f++) draw2_load(H[f], d, wrap_inc(k + 1, g.n), t + 2, r[f]);
+            n0 = op.load(!par, b + d.plane, i);
+            n1 = op.load(par, b + d.plane, i);
         }
-        // one cell's stencils at a time (fewer live values)
+        // one cell's stencils at a time (fewer live values); its side values
+        // are reloaded for the next plane once they are in the stencils
         double r0, r1;
         {
             S19<T> s0[NF];
 #pragma unroll
-            for (int f = 0; f < NF; f++) s0[f] = s19_win2(w[f], false, sd[f], d);
-            r0 = op.cell(par * half + off, o0, s0);
+            for (int f = 0; f < NF; f++) {
+                s0[f] = s19_win2(w[f], false, sl[f]);
+                if (more) dside_load(H[f], d, kn, t + 1, g.n, false, sl[f]);
+            }
+            r0 = op.cell(par, b, i, o0, s0);
         }
+        __builtin_amdgcn_sched_barrier(0);
         {
             S19<T> s1[NF];
 #pragma unroll
-            for (int f = 0; f < NF; f++) s1[f] = s19_win2(w[f], true, sd[f], d);
-            r1 = op.cell((1u - par) * half + off, o1, s1);
+            for (int f = 0; f < NF; f++) {
+                s1[f] = s19_win2(w[f], true, sr[f]);
+                if (more) dside_load(H[f], d, kn, t + 1, g.n, true, sr[f]);
+            }
+            r1 = op.cell(!par, b, i, o1, s1);
         }
         acc += r0 * r0 + r1 * r1;
-        if (t + 1 < DGP_KC) {
+        if (more) {
 #pragma unroll
             for (int f = 0; f < NF; f++) {
                 dwin2_shift(w[f]);
                 dwin2_set(w[f], 2, r[f]);
-                sd[f] = sdn[f];
             }
-            off = offn;
-            par = parn;
+            b += d.plane;
             o0 = n0;
             o1 = n1;
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
     return acc;
+}
+
+template <class OP>
+__device__ __forceinline__ double dgp_both_zcol(const OP& op, const Geo& g, int m, int j, int k0)
+{
+    const DCol d = dcol_of(g, m, j);
+    const int k = __builtin_amdgcn_readfirstlane(k0);
+    return (__builtin_amdgcn_readfirstlane(j) + k) & 1 ? dgp_both_run<true>(op, g, d, k)
+                                                       : dgp_both_run<false>(op, g, d, k);
 }
 
 // FP64 residual L(phi) (- f on coarse levels), stored in res when non-null
@@ -657,15 +660,17 @@ struct DgpRes64Op {
     DgpCoef c;
     unsigned hf;
     __device__ const double* half(int, int colour) const { return u + (colour ? hf : 0u); }
-    __device__ __forceinline__ Own load(unsigned i) const
+    __device__ __forceinline__ Own load(bool colour, size_t b, unsigned i) const
     {
-        return Own{ld_once<NT>(rho[i]), COARSE ? ld_once<NT>(f[i]) : 0.0};
+        if (colour) b += hf;
+        return Own{ld_at<NT>(plane_ptr(rho, b), i), COARSE ? ld_at<NT>(plane_ptr(f, b), i) : 0.0};
     }
-    __device__ __forceinline__ double cell(unsigned i, const Own& o, const S19<double>* s) const
+    __device__ __forceinline__ double cell(bool colour, size_t b, unsigned i, const Own& o, const S19<double>* s) const
     {
+        if (colour) b += hf;
         double OP = dgp_L19(s[0], o.rho, c);
         if constexpr (COARSE) OP = OP - o.f;
-        if (res) st_once<NT>(res[i], OP);
+        if (res) st_at<NT>(plane_ptr(res, b), i, OP);
         return OP;
     }
 };
@@ -688,17 +693,22 @@ struct DgpmOuterOp {
     DgpCoef c;
     unsigned hf;
     __device__ const double* half(int, int colour) const { return u + (colour ? hf : 0u); }
-    __device__ __forceinline__ Own load(unsigned i) const { return Own{ld_once<NT>(rho[i])}; }
-    __device__ __forceinline__ double cell(unsigned i, const Own& o, const S19<double>* s) const
+    __device__ __forceinline__ Own load(bool colour, size_t b, unsigned i) const
     {
+        if (colour) b += hf;
+        return Own{ld_at<NT>(plane_ptr(rho, b), i)};
+    }
+    __device__ __forceinline__ double cell(bool colour, size_t b, unsigned i, const Own& o, const S19<double>* s) const
+    {
+        if (colour) b += hf;
         const double OP = dgp_L19(s[0], o.rho, c);
         const float gv = (float)(-OP);
-        st_once<NT>(g32[i], gv);
-        st_once<NT>(pb[i], (float)s[0].c0);
-        if (i < hf)
-            st_once<NT>(e0[i], dgpm_first(gv, (float)c.inv_dx2));
+        st_at<NT>(plane_ptr(g32, b), i, gv);
+        st_at<NT>(plane_ptr(pb, b), i, (float)s[0].c0);
+        if (colour)
+            st_at<NT>(plane_ptr(e, b), i, 0.0f);
         else
-            st_once<NT>(e[i], 0.0f);
+            st_at<NT>(plane_ptr(e0, b), i, dgpm_first(gv, (float)c.inv_dx2));
         return OP;
     }
 };
@@ -721,10 +731,15 @@ struct DgpmResOp {
     DgpF c;
     unsigned hf;
     __device__ const float* half(int f, int colour) const { return (f ? pb : e) + (colour ? hf : 0u); }
-    __device__ __forceinline__ Own load(unsigned i) const { return Own{(float)ld_once<NT>(rho[i]), ld_once<NT>(rhs[i])}; }
-    __device__ __forceinline__ double cell(unsigned i, const Own& o, const S19<float>* s) const
+    __device__ __forceinline__ Own load(bool colour, size_t b, unsigned i) const
     {
-        st_once<NT>(out[i], dgp_dop(d2_of(s[1]), d2_of(s[0]), o.rho, c) - o.rhs);
+        if (colour) b += hf;
+        return Own{(float)ld_at<NT>(plane_ptr(rho, b), i), ld_at<NT>(plane_ptr(rhs, b), i)};
+    }
+    __device__ __forceinline__ double cell(bool colour, size_t b, unsigned i, const Own& o, const S19<float>* s) const
+    {
+        if (colour) b += hf;
+        st_at<NT>(plane_ptr(out, b), i, dgp_dop(d2_of(s[1]), d2_of(s[0]), o.rho, c) - o.rhs);
         return 0.0;
     }
 };
@@ -738,8 +753,9 @@ template <bool S0, bool NT, typename R>
 __device__ __forceinline__ void dgpm_zsmooth_run(const float* __restrict__ e0, const float* __restrict__ e1,
                                                  float* __restrict__ out, const float* __restrict__ pb,
                                                  const R* __restrict__ rho, const float* __restrict__ rhs,
-                                                 const Geo& g, int colour, const DgpF& c, const DCol& d, int k0)
+                                                 const Geo& g, int colour, const DgpF& c, const DCol& d, int k0v)
 {
+    const int k0 = __builtin_amdgcn_readfirstlane(k0v);
     // (j + k0) & 1 = S0 ^ colour: wave-uniform
     const int par0 = (S0 ? 1 : 0) ^ (colour & 1);
     const DHalves<float> He = dhalves(e0, e1, par0), Hb = dhalves(pb, pb + g.half, par0);
@@ -751,40 +767,41 @@ __device__ __forceinline__ void dgpm_zsmooth_run(const float* __restrict__ e0, c
     DSide<float> se, sb;
     dside_load(He, d, k0, 0, g.n, S0, se);
     dside_load(Hb, d, k0, 0, g.n, S0, sb);
-    unsigned off = (unsigned)k0 * d.plane + d.rowoff[1] + d.m;
-    float rh = (float)ld_once<NT>(elem(rhoc, off));
-    float fv = ld_once<NT>(elem(rhsc, off));
+    const unsigned i = d.off[1];
+    size_t b = (size_t)((unsigned)k0 * d.plane);
+    float rh = (float)ld_at<NT>(plane_ptr(rhoc, b), i);
+    float fv = ld_at<NT>(plane_ptr(rhsc, b), i);
 #pragma unroll
     for (int t = 0; t < DGP_KC; t++) {
         const int k = k0 + t;
         const bool s = S0 ^ ((t & 1) != 0);
         DRaw2<float> re, rb;
-        DSide<float> sen, sbn;
         float rhn = 0.0f, fvn = 0.0f;
-        const unsigned offn = off + d.plane;
+        const size_t bn = b + d.plane;
         if (t + 1 < DGP_KC) {
             const int kn = wrap_inc(k + 1, g.n);
             draw2_load(He, d, kn, t + 2, re);
             draw2_load(Hb, d, kn, t + 2, rb);
-            dside_load(He, d, wrap_inc(k, g.n), t + 1, g.n, !s, sen);
-            dside_load(Hb, d, wrap_inc(k, g.n), t + 1, g.n, !s, sbn);
-            rhn = (float)ld_once<NT>(elem(rhoc, offn));
-            fvn = ld_once<NT>(elem(rhsc, offn));
+            rhn = (float)ld_at<NT>(plane_ptr(rhoc, bn), i);
+            fvn = ld_at<NT>(plane_ptr(rhsc, bn), i);
         }
-        const D2f de = d2_of(s19_win2(we, s, se, d)), db = d2_of(s19_win2(wb, s, sb, d));
+        const D2f de = d2_of(s19_win2(we, s, se)), db = d2_of(s19_win2(wb, s, sb));
+        if (t + 1 < DGP_KC) {
+            dside_load(He, d, wrap_inc(k, g.n), t + 1, g.n, !s, se);
+            dside_load(Hb, d, wrap_inc(k, g.n), t + 1, g.n, !s, sb);
+        }
         const float D = dgp_dop(db, de, rh, c) - fv;
-        st_once<NT>(elem(out, off), de.c0 + D / (6.0f * c.inv_dx2));
+        st_at<NT>(plane_ptr(out, b), i, de.c0 + over_six(D, c));
         if (t + 1 < DGP_KC) {
             dwin2_shift(we);
             dwin2_shift(wb);
             dwin2_set(we, 2, re);
             dwin2_set(wb, 2, rb);
-            se = sen;
-            sb = sbn;
-            off = offn;
+            b = bn;
             rh = rhn;
             fv = fvn;
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 

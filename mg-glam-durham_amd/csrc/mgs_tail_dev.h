@@ -143,7 +143,7 @@ struct TailDgpm {
             return (float)((double)de.c0 + D / (6.0 * (double)c.inv_dx2));
         }
         const float D = dgp_dop(db, de, rho, c) - f;
-        return de.c0 + D / (6.0f * c.inv_dx2);
+        return de.c0 + over_six(D, c);
     }
     static __device__ __forceinline__ void add(float& P, float w, float vh, float vr) { P += w * (vh - vr); }
     static __device__ __forceinline__ bool keep(float) { return true; }
