@@ -186,6 +186,39 @@ __device__ __forceinline__ T& lvl(T* a, unsigned i)
         return a[i];
 }
 
+// Index of a cell of a level in a z-marching pass: base + i, base the same for
+// a whole wave (its plane and colour), i within the plane.  The operators take
+// either this or a plain index.
+struct PlaneIndex {
+    size_t base;
+    unsigned i;
+    __device__ __forceinline__ bool below(size_t half) const { return base < half; }  // half: whole planes
+};
+
+template <bool NT, typename T>
+__device__ __forceinline__ T ld_cell(const T* a, PlaneIndex o)
+{
+    return ld_at<NT>(plane_ptr(a, o.base), o.i);
+}
+
+template <bool NT, typename T>
+__device__ __forceinline__ T ld_cell(const T* a, unsigned o)
+{
+    return ld_once<NT>(lvl(a, o));
+}
+
+template <bool NT, typename T>
+__device__ __forceinline__ void st_cell(T* a, PlaneIndex o, T v)
+{
+    st_at<NT>(plane_ptr(a, o.base), o.i, v);
+}
+
+template <bool NT, typename T>
+__device__ __forceinline__ void st_cell(T* a, unsigned o, T v)
+{
+    st_once<NT>(lvl(a, o), v);
+}
+
 // the cells x = 2m, 2m+1 of a row of a lexicographic array, loaded or stored
 // by one instruction; aligned as an element, since a caller's array need be
 template <typename T>

@@ -162,14 +162,16 @@ struct FrSmoothOp {
     const double* f;
     FrCoef c;
     __device__ double* field() const { return u; }
-    __device__ __forceinline__ Own load(unsigned o, unsigned) const
+    template <class I>
+    __device__ __forceinline__ Own load(I o, I) const
     {
         Own w;
-        w.rho = ld_once<NT>(rho[o]);
-        w.f = COARSE ? ld_once<NT>(f[o]) : 0.0;
+        w.rho = ld_cell<NT>(rho, o);
+        w.f = COARSE ? ld_cell<NT>(f, o) : 0.0;
         return w;
     }
-    __device__ __forceinline__ void update(unsigned o, unsigned, const Own& w, double, double xp, double xm,
+    template <class I>
+    __device__ __forceinline__ void update(I o, I, const Own& w, double, double xp, double xm,
                                            double yp, double ym, double zp, double zm) const
     {
         const double S =
@@ -180,11 +182,11 @@ struct FrSmoothOp {
         else
             P = c.fct1s * w.rho - c.Q2 + c.fct2s * w.f - S / 6.0;
         if constexpr (REFROOT) {
-            st_once<NT>(u[o], fr_root64<FRN>(P, c));
+            st_cell<NT>(u, o, fr_root64<FRN>(P, c));
         } else {
             float x = seed_root<FRN>((float)(P * c.inv_w), (float)(c.Q2 * c.inv_w));
             if (!(x > 0.0f) || !(x < 3.0e38f)) x = 1.0f;  // Newton from u_bg
-            st_once<NT>(u[o], newton_root64<FRN>((double)x * c.ubg, P, c.Q));
+            st_cell<NT>(u, o, newton_root64<FRN>((double)x * c.ubg, P, c.Q));
         }
     }
 };
@@ -204,14 +206,16 @@ struct FrResOp {
     double* out;
     FrCoef c;
     __device__ const double* field() const { return u; }
-    __device__ __forceinline__ Own load(unsigned o) const
+    template <class I>
+    __device__ __forceinline__ Own load(I o) const
     {
         Own w;
-        w.rho = ld_once<NT>(rho[o]);
-        w.f = COARSE ? ld_once<NT>(f[o]) : 0.0;
+        w.rho = ld_cell<NT>(rho, o);
+        w.f = COARSE ? ld_cell<NT>(f, o) : 0.0;
         return w;
     }
-    __device__ __forceinline__ double cell(unsigned o, const Own& w, double uc, double xp, double xm, double yp,
+    template <class I>
+    __device__ __forceinline__ double cell(I o, const Own& w, double uc, double xp, double xm, double yp,
                                            double ym, double zp, double zm) const
     {
         const double S =
@@ -221,7 +225,7 @@ struct FrResOp {
         OP = OP + c.fct1r * w.rho;
         OP = OP + c.fct2r * (c.a_fR_rt / uc - 1.0);
         if constexpr (COARSE) OP = OP - w.f;
-        if (out) st_once<NT>(out[o], OP);
+        if (out) st_cell<NT>(out, o, OP);
         return OP;
     }
 };
@@ -438,15 +442,17 @@ struct DfSmoothOp {
     const float* rhs;
     DfCoef c;
     __device__ float* field() const { return d; }
-    __device__ __forceinline__ Own load(unsigned o, unsigned) const
+    template <class I>
+    __device__ __forceinline__ Own load(I o, I) const
     {
-        return Own{ld_once<NT>(elem(xb, o)), ld_once<NT>(elem(rhs, o))};
+        return Own{ld_cell<NT>(xb, o), ld_cell<NT>(rhs, o)};
     }
-    __device__ __forceinline__ void update(unsigned o, unsigned, const Own& w, float, float xp, float xm, float yp,
+    template <class I>
+    __device__ __forceinline__ void update(I o, I, const Own& w, float, float xp, float xm, float yp,
                                            float ym, float zp, float zm) const
     {
         const float S = xp + xm + yp + ym + zp + zm;
-        st_once<NT>(elem(d, o), df_solve<FRN>(S, w.xb, w.rhs, c));
+        st_cell<NT>(d, o, df_solve<FRN>(S, w.xb, w.rhs, c));
     }
 };
 
@@ -480,22 +486,24 @@ struct DfSmoothUpdateOp {
     DfCoef c;
     double ubg;
     __device__ const float* field() const { return d; }
-    __device__ __forceinline__ Own load(unsigned o, unsigned oo) const
+    template <class I>
+    __device__ __forceinline__ Own load(I o, I oo) const
     {
         Own w;
-        w.xb = ld_once<NT>(elem(xb, o));
-        w.rhs = ld_once<NT>(elem(rhs, o));
-        w.u = ld_once<NT>(u[o]);
-        w.xbo = ld_once<NT>(elem(xb, oo));
-        w.uo = ld_once<NT>(u[oo]);
+        w.xb = ld_cell<NT>(xb, o);
+        w.rhs = ld_cell<NT>(rhs, o);
+        w.u = ld_cell<NT>(u, o);
+        w.xbo = ld_cell<NT>(xb, oo);
+        w.uo = ld_cell<NT>(u, oo);
         return w;
     }
-    __device__ __forceinline__ void update(unsigned o, unsigned oo, const Own& w, float dother, float xp, float xm,
+    template <class I>
+    __device__ __forceinline__ void update(I o, I oo, const Own& w, float dother, float xp, float xm,
                                            float yp, float ym, float zp, float zm) const
     {
         const float S = xp + xm + yp + ym + zp + zm;
-        st_once<NT>(u[o], outer_updated<FRN>(w.u, df_solve<FRN>(S, w.xb, w.rhs, c), w.xb, ubg));
-        st_once<NT>(u[oo], outer_updated<FRN>(w.uo, dother, w.xbo, ubg));
+        st_cell<NT>(u, o, outer_updated<FRN>(w.u, df_solve<FRN>(S, w.xb, w.rhs, c), w.xb, ubg));
+        st_cell<NT>(u, oo, outer_updated<FRN>(w.uo, dother, w.xbo, ubg));
     }
 };
 
@@ -521,8 +529,10 @@ struct FrOuterOp {
         double delta;
     };
     __device__ const double* field() const { return u; }
-    __device__ __forceinline__ Own load(unsigned o) const { return Own{ld_once<NT>(delta[o])}; }
-    __device__ __forceinline__ double cell(unsigned o, const Own& w, double uc, double xp, double xm, double yp,
+    template <class I>
+    __device__ __forceinline__ Own load(I o) const { return Own{ld_cell<NT>(delta, o)}; }
+    template <class I>
+    __device__ __forceinline__ double cell(I o, const Own& w, double uc, double xp, double xm, double yp,
                                            double ym, double zp, double zm) const
     {
         const double S =
@@ -537,9 +547,9 @@ struct FrOuterOp {
         OP = OP + c.fct2r * (c.a_fR_rt * ru - 1.0);
         if constexpr (!NORM_ONLY) {
             const float gv = (float)(-OP), xv = (float)(uc * c.inv_ubg);
-            st_once<NT>(elem(g, o), gv);
-            st_once<NT>(elem(xb, o), xv);
-            if (o < half) st_once<NT>(elem(d, o), df_solve<FRN>(0.0f, xv, gv, dc));
+            st_cell<NT>(g, o, gv);
+            st_cell<NT>(xb, o, xv);
+            if (o.below(half)) st_cell<NT>(d, o, df_solve<FRN>(0.0f, xv, gv, dc));
         }
         return OP;
     }
@@ -559,15 +569,17 @@ struct DfResOp {
         float xb, rhs;
     };
     __device__ const float* field() const { return d; }
-    __device__ __forceinline__ Own load(unsigned o) const { return Own{ld_once<NT>(elem(xb, o)), ld_once<NT>(elem(rhs, o))}; }
-    __device__ __forceinline__ double cell(unsigned o, const Own& w, float dc, float xp, float xm, float yp, float ym,
+    template <class I>
+    __device__ __forceinline__ Own load(I o) const { return Own{ld_cell<NT>(xb, o), ld_cell<NT>(rhs, o)}; }
+    template <class I>
+    __device__ __forceinline__ double cell(I o, const Own& w, float dc, float xp, float xm, float yp, float ym,
                                            float zp, float zm) const
     {
         const float S = xp + xm + yp + ym + zp + zm;
         const float xbc = w.xb;
         const float x = xroot<FRN>(fmaxf(wpow<FRN>(xbc) + dc, 1.0e-30f));
         const float r = c.A * (S - 6.0f * dc) + dlocal<FRN>(dc, x, xbc, c.C) - w.rhs;
-        st_once<NT>(elem(out, o), r);
+        st_cell<NT>(out, o, r);
         return 0.0;
     }
 };

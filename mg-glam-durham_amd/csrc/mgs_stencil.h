@@ -193,12 +193,14 @@ __device__ __forceinline__ bool zcol(const Geo& g, int TX, int TY, int XB, int J
     return zcol(g.h, g.n, TX, TY, XB, JB, KC, NB, c);
 }
 
-// Column window over one colour half `a` (32-bit offsets; a level holds at
-// most 2^30 cells).  fetch(k) issues the loads that give the six neighbour
-// values of the opposite-colour cell at (m, j, k), whose x-parity is s;
-// apply() turns them into the neighbours and advances the window to k+1.
-// Splitting the two lets a loop issue the loads of plane k+1 before it
-// computes and stores plane k.
+// Column window over one colour half `a`.  fetch(k) issues the loads that give
+// the six neighbour values of the opposite-colour cell at (m, j, k), whose
+// x-parity is s; apply() turns them into the neighbours and advances the window
+// to k+1.  Splitting the two lets a loop issue the loads of plane k+1 before it
+// computes and stores plane k.  Planes move a scalar base, the offsets within a
+// plane stay in registers (see plane_ptr): the FP32 passes are bound by the
+// vector ALU as well as by memory.  For the same reason the two x-neighbours
+// come in either order: every operator adds them first, and a + b = b + a.
 template <typename T>
 struct ZPre {
     T next, xo, yp, ym;
@@ -207,43 +209,45 @@ struct ZPre {
 template <typename T>
 struct ZWin {
     const T* __restrict__ a;
-    unsigned n, h, m, jrow, jprow, jmrow;  // row offsets are j*h etc. within a plane
-    unsigned plane;                         // n * h
+    unsigned n, plane;             // plane: n * h
+    unsigned at, aty, atm, xl, xr;  // (m, j), (m, j+1), (m, j-1), (m-1, j), (m+1, j)
     T prev, cur;
 
     __device__ __forceinline__ void init(const T* base, const Geo& g, int m_, int j, int k0)
     {
         a = base;
         n = (unsigned)g.n;
-        h = (unsigned)g.h;
-        m = (unsigned)m_;
+        const unsigned h = (unsigned)g.h, m = (unsigned)m_, row = (unsigned)j * h;
         plane = n * h;
-        jrow = (unsigned)j * h;
-        jprow = (unsigned)wrap_inc(j, g.n) * h;
-        jmrow = (unsigned)wrap_dec(j, g.n) * h;
-        prev = elem(a, (unsigned)wrap_dec(k0, g.n) * plane + jrow + m);
-        cur = elem(a, (unsigned)k0 * plane + jrow + m);
+        at = row + m;
+        aty = (unsigned)wrap_inc(j, g.n) * h + m;
+        atm = (unsigned)wrap_dec(j, g.n) * h + m;
+        xl = row + (m == 0 ? h - 1 : m - 1);
+        xr = row + (m + 1 == h ? 0u : m + 1);
+        prev = ld_at(plane_ptr(a, (unsigned)wrap_dec(k0, g.n) * plane), at);
+        cur = ld_at(plane_ptr(a, (unsigned)k0 * plane), at);
     }
+
+    // offsets made anew in the caller's block: the compiler then knows them to
+    // be 32 bits wide there and folds them into the accesses
+    __device__ __forceinline__ void localize() { asm("" : "+v"(at), "+v"(aty), "+v"(atm), "+v"(xl), "+v"(xr)); }
 
     __device__ __forceinline__ ZPre<T> fetch(int k, int s) const
     {
         const unsigned kp = (unsigned)(k + 1 == (int)n ? 0 : k + 1);
-        const unsigned pk = (unsigned)k * plane;
-        unsigned mo;
-        if (s) mo = (m + 1 == h) ? 0u : m + 1;
-        else mo = (m == 0) ? h - 1 : m - 1;
+        const auto* pk = plane_ptr(a, (unsigned)k * plane);
         ZPre<T> p;
-        p.next = elem(a, kp * plane + jrow + m);
-        p.xo = elem(a, pk + jrow + mo);
-        p.yp = elem(a, pk + jprow + m);
-        p.ym = elem(a, pk + jmrow + m);
+        p.next = ld_at(plane_ptr(a, kp * plane), at);
+        p.xo = ld_at(pk, s ? xr : xl);
+        p.yp = ld_at(pk, aty);
+        p.ym = ld_at(pk, atm);
         return p;
     }
 
-    __device__ __forceinline__ void apply(const ZPre<T>& p, int s, T& xp, T& xm, T& yp, T& ym, T& zp, T& zm)
+    __device__ __forceinline__ void apply(const ZPre<T>& p, T& xp, T& xm, T& yp, T& ym, T& zp, T& zm)
     {
-        xp = s ? p.xo : cur;
-        xm = s ? cur : p.xo;
+        xp = p.xo;
+        xm = cur;
         yp = p.yp;
         ym = p.ym;
         zp = p.next;
@@ -263,26 +267,27 @@ struct ZWin {
 // before the first update (R + 2 window values, R own records), and the
 // window needs no register rotation.
 template <int R, class OP>
-__device__ __forceinline__ void colour_pass_run(const OP& op, ZWin<typename OP::T>& w, unsigned own, unsigned oth,
-                                                unsigned col, int s0, int k0)
+__device__ __forceinline__ void colour_pass_run(const OP& op, ZWin<typename OP::T>& w, size_t own, size_t oth,
+                                                int s0, int k0)
 {
     using T = typename OP::T;
     using Own = typename OP::Own;
     ZPre<T> p[R];
     Own o[R];
+    w.localize();
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const unsigned rel = (unsigned)(k0 + r) * w.plane + col;
+        const size_t rel = (unsigned)(k0 + r) * w.plane;
         p[r] = w.fetch(k0 + r, s0 ^ (r & 1));
-        o[r] = op.load(own + rel, oth + rel);
+        o[r] = op.load(PlaneIndex{own + rel, w.at}, PlaneIndex{oth + rel, w.at});
     }
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const unsigned rel = (unsigned)(k0 + r) * w.plane + col;
+        const size_t rel = (unsigned)(k0 + r) * w.plane;
         const T other = w.cur;
         T xp, xm, yp, ym, zp, zm;
-        w.apply(p[r], s0 ^ (r & 1), xp, xm, yp, ym, zp, zm);
-        op.update(own + rel, oth + rel, o[r], other, xp, xm, yp, ym, zp, zm);
+        w.apply(p[r], xp, xm, yp, ym, zp, zm);
+        op.update(PlaneIndex{own + rel, w.at}, PlaneIndex{oth + rel, w.at}, o[r], other, xp, xm, yp, ym, zp, zm);
     }
 }
 
@@ -295,30 +300,29 @@ __device__ __forceinline__ void colour_pass_col(const OP& op, const Geo& g, int 
     using T = typename OP::T;
     using Own = typename OP::Own;
     ZWin<T> w;
-    w.init(op.field() + (size_t)(1 - colour) * g.half, g, c.m, c.j, c.k0);
-    const unsigned own = (unsigned)colour * (unsigned)g.half;
-    const unsigned oth = (unsigned)(1 - colour) * (unsigned)g.half;
-    const unsigned col = w.jrow + w.m;
-    if (c.k1 - c.k0 == ZRUN_UNROLLED) {
-        colour_pass_run<ZRUN_UNROLLED>(op, w, own, oth, col, (colour + c.j + c.k0) & 1, c.k0);
+    const int k0 = __builtin_amdgcn_readfirstlane(c.k0), k1 = __builtin_amdgcn_readfirstlane(c.k1);
+    w.init(op.field() + (size_t)(1 - colour) * g.half, g, c.m, c.j, k0);
+    const size_t own = (size_t)colour * g.half, oth = (size_t)(1 - colour) * g.half;
+    if (k1 - k0 == ZRUN_UNROLLED) {
+        colour_pass_run<ZRUN_UNROLLED>(op, w, own, oth, (colour + c.j + k0) & 1, k0);
         return;
     }
-    int k = c.k0;
+    int k = k0;
     ZPre<T> pc = w.fetch(k, (colour + c.j + k) & 1);
-    Own oc = op.load(own + (unsigned)k * w.plane + col, oth + (unsigned)k * w.plane + col);
-    for (; k < c.k1; k++) {
+    Own oc = op.load(PlaneIndex{own + (unsigned)k * w.plane, w.at}, PlaneIndex{oth + (unsigned)k * w.plane, w.at});
+    for (; k < k1; k++) {
         ZPre<T> pn = pc;
         Own on = oc;
-        if (k + 1 < c.k1) {
-            const unsigned rel = (unsigned)(k + 1) * w.plane + col;
+        if (k + 1 < k1) {
+            const size_t rel = (unsigned)(k + 1) * w.plane;
             pn = w.fetch(k + 1, (colour + c.j + k + 1) & 1);
-            on = op.load(own + rel, oth + rel);
+            on = op.load(PlaneIndex{own + rel, w.at}, PlaneIndex{oth + rel, w.at});
         }
-        const unsigned rel = (unsigned)k * w.plane + col;
+        const size_t rel = (unsigned)k * w.plane;
         const T other = w.cur;
         T xp, xm, yp, ym, zp, zm;
-        w.apply(pc, (colour + c.j + k) & 1, xp, xm, yp, ym, zp, zm);
-        op.update(own + rel, oth + rel, oc, other, xp, xm, yp, ym, zp, zm);
+        w.apply(pc, xp, xm, yp, ym, zp, zm);
+        op.update(PlaneIndex{own + rel, w.at}, PlaneIndex{oth + rel, w.at}, oc, other, xp, xm, yp, ym, zp, zm);
         pc = pn;
         oc = on;
     }
@@ -342,30 +346,32 @@ __global__ __launch_bounds__(256) void k_colour_pass(OP op, Geo g, int colour, i
 // the squares are accumulated in the same order as the loop below.
 template <int R, class OP>
 __device__ __forceinline__ double both_colours_run(const OP& op, ZWin<typename OP::T>& w0, ZWin<typename OP::T>& w1,
-                                                   unsigned half, unsigned col, int j, int k0)
+                                                   size_t half, int j, int k0)
 {
     using T = typename OP::T;
     using Own = typename OP::Own;
     ZPre<T> p0[R], p1[R];
     Own o0[R], o1[R];
+    w0.localize();
+    w1.at = w0.at, w1.aty = w0.aty, w1.atm = w0.atm, w1.xl = w0.xl, w1.xr = w0.xr;  // one column
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const unsigned rel = (unsigned)(k0 + r) * w0.plane + col;
+        const size_t rel = (unsigned)(k0 + r) * w0.plane;
         p1[r] = w1.fetch(k0 + r, (j + k0 + r) & 1);
         p0[r] = w0.fetch(k0 + r, (1 + j + k0 + r) & 1);
-        o0[r] = op.load(rel);
-        o1[r] = op.load(half + rel);
+        o0[r] = op.load(PlaneIndex{rel, w0.at});
+        o1[r] = op.load(PlaneIndex{half + rel, w0.at});
     }
     double acc = 0.0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const T c0 = w0.cur, c1 = w1.cur;
-        const unsigned off = (unsigned)(k0 + r) * w0.plane + col;
+        const size_t off = (unsigned)(k0 + r) * w0.plane;
         T xp, xm, yp, ym, zp, zm;
-        w1.apply(p1[r], (j + k0 + r) & 1, xp, xm, yp, ym, zp, zm);
-        const double r0 = op.cell(off, o0[r], c0, xp, xm, yp, ym, zp, zm);
-        w0.apply(p0[r], (1 + j + k0 + r) & 1, xp, xm, yp, ym, zp, zm);
-        const double r1 = op.cell(half + off, o1[r], c1, xp, xm, yp, ym, zp, zm);
+        w1.apply(p1[r], xp, xm, yp, ym, zp, zm);
+        const double r0 = op.cell(PlaneIndex{off, w0.at}, o0[r], c0, xp, xm, yp, ym, zp, zm);
+        w0.apply(p0[r], xp, xm, yp, ym, zp, zm);
+        const double r1 = op.cell(PlaneIndex{half + off, w0.at}, o1[r], c1, xp, xm, yp, ym, zp, zm);
         acc += r0 * r0 + r1 * r1;
     }
     return acc;
@@ -378,35 +384,35 @@ __device__ __forceinline__ double both_colours_col(const OP& op, const Geo& g, c
     using Own = typename OP::Own;
     double acc = 0.0;
     ZWin<T> w0, w1;  // windows over the red (0) and black (1) halves
-    w0.init(op.field(), g, c.m, c.j, c.k0);
-    w1.init(op.field() + g.half, g, c.m, c.j, c.k0);
-    const unsigned half = (unsigned)g.half;
-    const unsigned col = w0.jrow + w0.m;
-    if (c.k1 - c.k0 == ZRUN_UNROLLED) return both_colours_run<ZRUN_UNROLLED>(op, w0, w1, half, col, c.j, c.k0);
-    int k = c.k0;
+    const int k0 = __builtin_amdgcn_readfirstlane(c.k0), k1 = __builtin_amdgcn_readfirstlane(c.k1);
+    w0.init(op.field(), g, c.m, c.j, k0);
+    w1.init(op.field() + g.half, g, c.m, c.j, k0);
+    const size_t half = (size_t)g.half;
+    if (k1 - k0 == ZRUN_UNROLLED) return both_colours_run<ZRUN_UNROLLED>(op, w0, w1, half, c.j, k0);
+    int k = k0;
     // red cell: neighbours in the black half, x-parity (j+k)&1;
     // black cell: neighbours in the red half, x-parity (1+j+k)&1
     ZPre<T> p1 = w1.fetch(k, (c.j + k) & 1);
     ZPre<T> p0 = w0.fetch(k, (1 + c.j + k) & 1);
-    Own o0 = op.load((unsigned)k * w0.plane + col);
-    Own o1 = op.load(half + (unsigned)k * w0.plane + col);
-    for (; k < c.k1; k++) {
+    Own o0 = op.load(PlaneIndex{(size_t)((unsigned)k * w0.plane), w0.at});
+    Own o1 = op.load(PlaneIndex{half + (unsigned)k * w0.plane, w0.at});
+    for (; k < k1; k++) {
         ZPre<T> q1 = p1, q0 = p0;
         Own n0 = o0, n1 = o1;
-        if (k + 1 < c.k1) {
-            const unsigned rel = (unsigned)(k + 1) * w0.plane + col;
+        if (k + 1 < k1) {
+            const size_t rel = (unsigned)(k + 1) * w0.plane;
             q1 = w1.fetch(k + 1, (c.j + k + 1) & 1);
             q0 = w0.fetch(k + 1, (1 + c.j + k + 1) & 1);
-            n0 = op.load(rel);
-            n1 = op.load(half + rel);
+            n0 = op.load(PlaneIndex{rel, w0.at});
+            n1 = op.load(PlaneIndex{half + rel, w0.at});
         }
         const T c0 = w0.cur, c1 = w1.cur;
-        const unsigned off = (unsigned)k * w0.plane + col;
+        const size_t off = (unsigned)k * w0.plane;
         T xp, xm, yp, ym, zp, zm;
-        w1.apply(p1, (c.j + k) & 1, xp, xm, yp, ym, zp, zm);
-        const double r0 = op.cell(off, o0, c0, xp, xm, yp, ym, zp, zm);
-        w0.apply(p0, (1 + c.j + k) & 1, xp, xm, yp, ym, zp, zm);
-        const double r1 = op.cell(half + off, o1, c1, xp, xm, yp, ym, zp, zm);
+        w1.apply(p1, xp, xm, yp, ym, zp, zm);
+        const double r0 = op.cell(PlaneIndex{off, w0.at}, o0, c0, xp, xm, yp, ym, zp, zm);
+        w0.apply(p0, xp, xm, yp, ym, zp, zm);
+        const double r1 = op.cell(PlaneIndex{half + off, w0.at}, o1, c1, xp, xm, yp, ym, zp, zm);
         acc += r0 * r0 + r1 * r1;
         p1 = q1;
         p0 = q0;
