@@ -345,11 +345,13 @@ __device__ __forceinline__ void dgpm_coarsest_block(float* __restrict__ e, const
 // shift's own operand for the lane that has no neighbour.  The barriers to the
 // scheduler keep it from raising every address sum of the unrolled run, which
 // spills scalar registers into vector lanes.  Instructions per cell: FP32 pass
-// 239 -> 175, FP32 residual 238 -> 177, FP64 residual 162 -> 111; at 512^3:
-// FP32 pass 456 -> 399 us (4.9 TB/s), FP32 residual 718 -> 610, FP64 outer
-// residual 880 -> 730 (5.1 TB/s).  Side values by vector loads: 459, 673 and
-// 1043; by scalar loads a whole plane ahead: 531, 882 and 738 (scalar
-// registers spill).
+// 239 -> 175, FP32 residual 238 -> 160, FP64 residual 162 -> 111.  At 512^3, by
+// where the arrays lie in memory (two runs that each kept their times): FP32
+// pass 456-484 -> 399-444 us, FP32 residual 718-850 -> 673-705, FP64 outer
+// residual 880-921 -> 730-745 (5.1 TB/s), FP64 pass 632 -> 460.  Side values of
+// the FP32 pass by vector loads: 467 where scalar ones take 444; of the FP32
+// residual by scalar loads: 610 in the one run, 910 in the other; of the FP64
+// residual by vector loads: 1043.
 //
 // The field is read through its two colour halves (h0, h1) and the pass
 // writes the new values of its colour to `out`, a half of a second array: a
@@ -442,8 +444,10 @@ __device__ __forceinline__ void draw2_load(const DHalves<T>& H, const DCol& d, i
 }
 
 // the five side values of the cell at plane k (dk = k - k0) with parity s:
-// x = 2m+2 has the colour of x = 2m, x = 2m-1 that of 2m+1
-template <typename T>
+// x = 2m+2 has the colour of x = 2m, x = 2m-1 that of 2m+1.  Scalar loads, or
+// with VECTOR one address in every lane: for the residual of two fields, whose
+// twenty values a plane crowd the scalar registers and the scalar cache.
+template <bool VECTOR = false, typename T>
 __device__ __forceinline__ void dside_load(const DHalves<T>& H, const DCol& d, int k, int dk, int n, bool s,
                                            DSide<T>& sd)
 {
@@ -452,7 +456,13 @@ __device__ __forceinline__ void dside_load(const DHalves<T>& H, const DCol& d, i
         const int P = side_plane(q), R = side_row(q);
         const unsigned kp = (unsigned)(P == 0 ? wrap_dec(k, n) : (P == 2 ? wrap_inc(k, n) : k)) * d.plane;
         const int f = ((R + P + dk) & 1) ^ (s ? 0 : 1);
-        sd.v[q] = ld_scalar(H.p[f], (size_t)kp + (s ? d.right[R] : d.left[R]));
+        unsigned o = s ? d.right[R] : d.left[R];
+        if constexpr (VECTOR) {
+            asm("" : "+v"(o));
+            sd.v[q] = ld_at(plane_ptr(H.p[f], kp), o);
+        } else {
+            sd.v[q] = ld_scalar(H.p[f], (size_t)kp + o);
+        }
     }
 }
 
@@ -578,8 +588,8 @@ __device__ __forceinline__ double dgp_both_run(const OP& op, const Geo& g, DCol 
     for (int f = 0; f < NF; f++) {
         H[f] = dhalves(op.half(f, 0), op.half(f, 1), PAR0);
         dwin2_init(w[f], H[f], d, k0, g.n);
-        dside_load(H[f], d, k0, 0, g.n, false, sl[f]);
-        dside_load(H[f], d, k0, 0, g.n, true, sr[f]);
+        dside_load<(NF > 1)>(H[f], d, k0, 0, g.n, false, sl[f]);
+        dside_load<(NF > 1)>(H[f], d, k0, 0, g.n, true, sr[f]);
     }
     const unsigned i = d.off[1];
     size_t b = (size_t)((unsigned)k0 * d.plane);
@@ -606,7 +616,7 @@ __device__ __forceinline__ double dgp_both_run(const OP& op, const Geo& g, DCol 
 #pragma unroll
             for (int f = 0; f < NF; f++) {
                 s0[f] = s19_win2(w[f], false, sl[f]);
-                if (more) dside_load(H[f], d, kn, t + 1, g.n, false, sl[f]);
+                if (more) dside_load<(NF > 1)>(H[f], d, kn, t + 1, g.n, false, sl[f]);
             }
             r0 = op.cell(par, b, i, o0, s0);
         }
@@ -616,7 +626,7 @@ __device__ __forceinline__ double dgp_both_run(const OP& op, const Geo& g, DCol 
 #pragma unroll
             for (int f = 0; f < NF; f++) {
                 s1[f] = s19_win2(w[f], true, sr[f]);
-                if (more) dside_load(H[f], d, kn, t + 1, g.n, true, sr[f]);
+                if (more) dside_load<(NF > 1)>(H[f], d, kn, t + 1, g.n, true, sr[f]);
             }
             r1 = op.cell(!par, b, i, o1, s1);
         }
