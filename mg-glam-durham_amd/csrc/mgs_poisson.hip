@@ -189,7 +189,9 @@ __global__ __launch_bounds__(RowPlan<N>::THREADS) void k_x_forward(const double*
     auto at = [](int p) { return p + (p >> 3); };
     Cx v[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = Cx{val(even[j + e * P::T]), val(other[j + e * P::T])};
+    for (int e = 0; e < 8; e++) v[e] = Cx{even[j + e * P::T], other[j + e * P::T]};
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = Cx{val(v[e].x), val(v[e].y)};  // (branches: after every load is issued)
     fft_from<P::M, 2, -1, 1>(v, j, tw, l, at);
     // X[k] = (Z[k] + Z*[M-k]) / 2 - i/2 exp(-2 pi i k / N) (Z[k] - Z*[M-k])
     __syncthreads();
@@ -344,8 +346,9 @@ __global__ __launch_bounds__(N / 4) void k_z_pair(Cx* __restrict__ a, const Cx* 
 // The x and y passes as above; the spectrum is binned from registers and never
 // stored.  Blocks walk the column tiles with a histogram in LDS each.  Bound by
 // the histogram's LDS atomics (24 per thread and tile): 73 us at 256^3, where
-// the read alone takes 25.  With psi formed as the x pass reads (60 us) and the
-// y pass (42 us) a spectrum of psi takes 0.19 ms; a pass for psi, the library's
+// the read alone takes 25.  With psi formed in the x pass once every load is
+// issued (44 us; 60 as each value arrives) and the y pass (42 us) a spectrum of
+// psi takes 0.17 ms; a pass for psi, the library's
 // transform and a binning pass took 0.31.
 template <int IPOL, int ICIC, bool LOGB, int N>
 __global__ __launch_bounds__(ColPlan<N>::THREADS) void k_z_bin(const Cx* __restrict__ a, const Cx* __restrict__ tw,
