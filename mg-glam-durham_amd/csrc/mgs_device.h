@@ -237,7 +237,7 @@ __device__ __forceinline__ void pair_split(const Geo& g, int m, int j, int k, si
 }
 
 template <int FRN, typename T>
-__device__ __forceinline__ T wpow(T x)
+__host__ __device__ __forceinline__ T wpow(T x)
 {
     if constexpr (FRN == 0)
         return x;

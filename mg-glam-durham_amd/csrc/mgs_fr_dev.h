@@ -105,11 +105,33 @@ __device__ __forceinline__ float seed_root(float P, float Q)
     }
 }
 
-// 1/x in FP64 from the hardware estimate and one Newton-Raphson correction
-// (relative error ~1e-15: enough for a Newton step's length)
-__device__ __forceinline__ double rcp64(double x)
+// The hardware's estimates of 1/x and 1/sqrt(x) in FP64: the instructions
+// promise 2^29 ulp, a relative error of 1.2e-7.  On the host, where the cell
+// solves built on them are checked, values that far off.
+__host__ __device__ __forceinline__ double rcp_estimate(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_rcp(x);
+#else
+    return (1.0 + 0x1p-23) / x;
+#endif
+}
+
+__host__ __device__ __forceinline__ double rsq_estimate(double x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_rsq(x);
+#else
+    return (1.0 + 0x1p-23) / sqrt(x);
+#endif
+}
+
+// 1/x in FP64 from the estimate and one Newton-Raphson correction (relative
+// error at most 1.5e-14, the estimate's squared: enough for a Newton step's
+// length)
+__host__ __device__ __forceinline__ double rcp64(double x)
+{
+    double r = rcp_estimate(x);
     const double e = __builtin_fma(-x, r, 1.0);
     return __builtin_fma(r, e, r);
 }
@@ -369,7 +391,7 @@ __device__ __forceinline__ void correct64_sons_apply(const double* hz, const dou
 
 // x from w = x^{n+1}
 template <int FRN, typename T>
-__device__ __forceinline__ T xroot(T w)
+__host__ __device__ __forceinline__ T xroot(T w)
 {
     if constexpr (FRN == 0)
         return w;
@@ -381,7 +403,7 @@ __device__ __forceinline__ T xroot(T w)
 
 // (x^{n+1} - xb^{n+1}) / (x - xb)
 template <int FRN, typename T>
-__device__ __forceinline__ T dden(T x, T xb)
+__host__ __device__ __forceinline__ T dden(T x, T xb)
 {
     if constexpr (FRN == 0)
         return (T)1;
@@ -836,13 +858,14 @@ __device__ __forceinline__ void df_correct_col(const float* __restrict__ dH, con
     }
 }
 
-// x = w^{1/(n+1)} and 1/x in FP64, w > 0, to a few times 1e-16: for n = 1 both
-// from the hardware's reciprocal square root refined once
+// x = w^{1/(n+1)} and 1/x in FP64, w > 0: for n = 1 both from the reciprocal
+// square root's estimate refined once (relative error at most 2.2e-14, 1.5
+// times the estimate's squared), else 1/x by rcp64
 template <int FRN>
-__device__ __forceinline__ void xroot_rcp64(double w, double& x, double& rx)
+__host__ __device__ __forceinline__ void xroot_rcp64(double w, double& x, double& rx)
 {
     if constexpr (FRN == 1) {
-        double y = __builtin_amdgcn_rsq(w);
+        double y = rsq_estimate(w);
         y = __builtin_fma(0.5 * y, __builtin_fma(-w * y, y, 1.0), y);
         rx = y;
         x = w * y;
@@ -853,15 +876,18 @@ __device__ __forceinline__ void xroot_rcp64(double w, double& x, double& rx)
 }
 
 // Newton's method in FP64 on D(d) = r at one cell from d = dl, with neighbour
-// sum S.  A step of relative length s leaves a relative error of order s^2
-// d / xb^{n+1}, so a step below 1e-6 d leaves one far below the FP32 rounding
-// the result is stored with.  Reciprocals are the hardware's refined once
-// (relative error about 1e-15).  The coarsest level is a chain of such
-// solves: with four divisions and a square root per step, iterated to
-// 1e-15, the 2^3 level took 10 us of each V-cycle.
+// sum S.  The scale on which D bends is w = xb^{n+1} + d, the distance to the
+// edge of the domain: a Newton step of length s leaves an error of about
+// s^2 / w.  So a step ends the iteration that is below 1e-6 of both d and w
+// (the error left is then below 1e-12 of either), or of the rounding of
+// xb^{n+1} + d; a step that was halved to stay in the domain never does, as it
+// has not solved anything.  Reciprocals and n = 1's root are estimates refined
+// once.  The coarsest level is a chain of such solves: with four divisions and
+// a square root per step, iterated to 1e-15, the 2^3 level took 10 us of each
+// V-cycle.
 template <int FRN>
-__device__ __forceinline__ double df_newton64(double dl, double S, double xbc, double wb, double rxb, double r,
-                                              const DfCoef& c)
+__host__ __device__ __forceinline__ double df_newton64(double dl, double S, double xbc, double wb, double rxb, double r,
+                                                       const DfCoef& c)
 {
     for (int it = 0; it < 30; it++) {
         double x, rx;
@@ -869,8 +895,12 @@ __device__ __forceinline__ double df_newton64(double dl, double S, double xbc, d
         const double F = c.A64 * (S - 6.0 * dl) + c.C64 * dl * rcp64(dden<FRN>(x, xbc)) * (rx * rxb) - r;
         const double Fp = -6.0 * c.A64 + c.C64 * (1.0 / (double)(FRN + 1)) * rx * wpow<FRN>(rx);
         double dn = dl - F * rcp64(Fp);
-        if (!(wb + dn > 0.0)) dn = 0.5 * (dl - wb);  // halve the distance to x = 0
-        const bool done = fabs(dn - dl) <= 1.0e-6 * fabs(dn);
+        const double w = wb + dn, step = fabs(dn - dl);
+        bool done = step <= fmax(1.0e-6 * fmin(fabs(dn), w), 1.0e-15 * (fabs(dn) + wb));
+        if (!(w > 0.0)) {  // halve the distance to x = 0
+            dn = 0.5 * (dl - wb);
+            done = false;
+        }
         dl = dn;
         if (done) break;
     }

@@ -1,0 +1,87 @@
+"""Scalar arithmetic of the device's cell solves, compiled for the host from the
+library's own headers and checked against wider arithmetic."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from conftest import ROOT
+
+CSRC = os.path.join(ROOT, "mg-glam-durham_amd", "csrc")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+SOURCE = r"""
+#include <math.h>
+#include "mgs_fr_dev.h"
+using namespace mgs;
+extern "C" double newton(int n, double d, double S, double xb, double r, double A, double C)
+{
+    DfCoef c{};
+    c.A64 = A;
+    c.C64 = C;
+    if (n == 0) return df_newton64<0>(d, S, xb, wpow<0>(xb), rcp64(xb), r, c);
+    if (n == 1) return df_newton64<1>(d, S, xb, wpow<1>(xb), rcp64(xb), r, c);
+    return df_newton64<2>(d, S, xb, wpow<2>(xb), rcp64(xb), r, c);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def cells(tmp_path_factory):
+    d = tmp_path_factory.mktemp("cells")
+    src, lib = str(d / "cells.hip"), str(d / "cells.so")
+    with open(src, "w") as f:
+        f.write(SOURCE)
+    r = subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-O2", "-std=c++17", "-ffp-contract=off", "-fPIC",
+                        "-shared", "-I", CSRC, src, "-o", lib], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    L = C.CDLL(lib)
+    L.newton.restype = C.c_double
+    L.newton.argtypes = [C.c_int] + [C.c_double] * 6
+    return L
+
+
+def _root(n, S, xb, r, A, C64):
+    """w = x^{n+1} with A (S - 6 (w - wb)) + C (1/xb - 1/x) = r, by bisection in
+    extended precision (the left side increases with w: A < 0 < C)"""
+    q = np.longdouble
+    wb, e = q(xb) ** (n + 1), -q(1) / q(n + 1)
+
+    def F(w):
+        return q(A) * (q(S) - 6 * (w - wb)) + q(C64) * (1 / q(xb) - w ** e) - q(r)
+
+    lo, hi = q(1e-30), q(1e10)
+    assert F(lo) < 0 < F(hi)
+    for _ in range(200):
+        mid = np.sqrt(lo * hi)
+        lo, hi = (mid, hi) if F(mid) < 0 else (lo, mid)
+    return hi
+
+
+# screened cells: the root lies far below the base, the start at the base, or a
+# factor above or below the root; A as on fine and on coarse levels
+@pytest.mark.parametrize("n", [0, 1, 2])
+@pytest.mark.parametrize("A", [-1e-3, -1.0, -100.0])
+def test_coarsest_newton_solves_screened_cells(cells, n, A):
+    q = np.longdouble
+    C64, xb, S = 1e-3, 1.0, 0.25
+    # each start reaches its root in fewer than the routine's 30 steps: a
+    # halving step gains a factor 2, a Newton step from below about n + 3
+    cases = [(w, w0) for w in (1.0, 0.3, 1e-2, 1e-3, 1e-4, 1e-5, 1e-6, 1e-7)
+             for w0 in (1.0, 3e3 * w, 30.0 * w, 1.1 * w, 0.5 * w, 1e-3 * w) if w0 <= 1.0]
+    for w, w0 in cases:
+        d = w - 1.0
+        r = A * (S - 6.0 * d) + C64 * (1.0 / xb - w ** (-1.0 / (n + 1)))
+        ws = _root(n, S, xb, r, A, C64)
+        ds = ws - 1
+        got = q(cells.newton(n, w0 - 1.0, S, xb, r, A, C64))
+        # the rounding of F over its slope (16 roundings, and the local term's
+        # reciprocals and root: four times 2.2e-14), and of the result itself
+        x = float(ws) ** (1.0 / (n + 1))
+        local = C64 * abs(1.0 / xb - 1.0 / x)
+        slope = -6.0 * A + C64 / ((n + 1) * x ** (n + 2))
+        noise = (16 * 2.0 ** -53 * (abs(A) * (S + 6.0 * abs(d)) + local + abs(r)) + 8.8e-14 * local) / slope
+        tol = 1e-11 * min(abs(float(ds)), float(ws)) + noise + 2.0 ** -52
+        assert abs(float(got - ds)) <= tol, (w, w0, float(got - ds), tol)
