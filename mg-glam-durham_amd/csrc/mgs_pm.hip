@@ -55,7 +55,7 @@ struct PmState {
     unsigned* order = nullptr;  // nbin particle indices
     int nbins = 0;
     int* count = nullptr;
-    int64_t* first = nullptr;
+    unsigned* first = nullptr;
     void* scan_tmp = nullptr;
     size_t scan_bytes = 0;
 };
@@ -275,20 +275,40 @@ struct __attribute__((packed, aligned(4))) Words4 {
 };
 
 // the particles' indices in bin order (the deposit takes fewer than 2^31
-// particles); one wave per PM_WCHUNK particles.  Bound by the number of
-// scattered stores: a run's words go out in stores of 4, 2 and 1 (512^3
-// particles of a clustered lattice: 0.52 ms, 0.68 with one store per word)
+// particles); one wave per PM_WCHUNK particles, its records and their bins'
+// starts loaded before the first store.  Bound by the scattered stores: a run's
+// words go out in stores of 4, 2 and 1.  A bin's line is filled a word at a time
+// by whichever waves meet the bin, so the more waves are under way the more
+// partly filled lines there are, and the L2 writes them out and takes them in
+// again: PM_SCATTER_LDS of unused LDS holds a CU to three blocks.  Measured with
+// eight blocks (and records loaded one by one) -> three, in ms: shuffled
+// lattices of 480^3 particles 3.39 -> 1.76, 400^3 1.93 -> 1.06 (four 1.61, two
+// 0.82); in order, clustered, 512^3 0.52 -> 0.46 (0.45, 0.52), 250^3 0.046 ->
+// 0.045 (0.042, 0.052).
+constexpr int PM_SCATTER_LDS = 53000;
+
 __global__ __launch_bounds__(PM_BLOCK) void k_bin_scatter(int64_t nwaves, const unsigned long long* __restrict__ recs,
                                                           const int* __restrict__ nrec,
-                                                          const int64_t* __restrict__ first,
+                                                          const unsigned* __restrict__ first,
                                                           unsigned* __restrict__ order)
 {
     const int64_t wave = (int64_t)blockIdx.x * (PM_BLOCK / 64) + (threadIdx.x >> 6);
     if (wave >= nwaves) return;
     const int n = nrec[wave];
-    for (int i = threadIdx.x & 63; i < n; i += 64) {
-        const unsigned long long r = recs[wave * PM_WCHUNK + i];
-        unsigned* o = order + first[(unsigned)(r >> 12) & 0x1fffffu] + (int64_t)(r >> 33);
+    const int lane = threadIdx.x & 63;
+    unsigned long long rec[PM_RUN];
+    unsigned at[PM_RUN];
+#pragma unroll
+    for (int q = 0; q < PM_RUN; q++)
+        if (lane + 64 * q < n) rec[q] = recs[wave * PM_WCHUNK + lane + 64 * q];
+#pragma unroll
+    for (int q = 0; q < PM_RUN; q++)
+        if (lane + 64 * q < n) at[q] = first[(unsigned)(rec[q] >> 12) & 0x1fffffu] + (unsigned)(rec[q] >> 33);
+#pragma unroll
+    for (int q = 0; q < PM_RUN; q++) {
+        if (lane + 64 * q >= n) continue;
+        const unsigned long long r = rec[q];
+        unsigned* o = order + at[q];
         const unsigned p = (unsigned)(wave * PM_WCHUNK) + ((unsigned)(r >> 3) & 511u);
         const unsigned len = ((unsigned)r & 7u) + 1u;
         unsigned u = 0;
@@ -373,7 +393,7 @@ __global__ __launch_bounds__(PM_DBLOCK) void k_tile_deposit(const float* __restr
                                                             const float* __restrict__ zs,
                                                             const unsigned* __restrict__ order,
                                                             const int* __restrict__ count,
-                                                            const int64_t* __restrict__ first, unsigned ntiles,
+                                                            const unsigned* __restrict__ first, unsigned ntiles,
                                                             PmTiles T, double* __restrict__ rho, Geo g, double wpar)
 {
     __shared__ unsigned long long acc[PM_TCELLS];
@@ -398,7 +418,7 @@ __global__ __launch_bounds__(PM_DBLOCK) void k_tile_deposit(const float* __restr
                       bz = (d & 4) ? wrap_dec(tz, T.z) : tz;
             const int b = ((bz * T.y + by) * T.x + bx) * 8 + flag[s];
             start = first[b];
-            items = s == 1 ? first[b + 6] + count[b + 6] - start : (int64_t)count[b];
+            items = s == 1 ? (int64_t)first[b + 6] + count[b + 6] - start : (int64_t)count[b];
             seg_dir[s] = d;
         }
         int64_t end = items;
@@ -734,7 +754,7 @@ static int pm_ensure_bins(mgs_handle* h, PmState* p, int nbins)
         p->nbins = 0;
         size_t bytes = 0;
         if (hipMalloc((void**)&p->count, (size_t)nbins * sizeof(int)) != hipSuccess ||
-            hipMalloc((void**)&p->first, (size_t)nbins * sizeof(int64_t)) != hipSuccess ||
+            hipMalloc((void**)&p->first, (size_t)nbins * sizeof(unsigned)) != hipSuccess ||
             hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, p->count, p->first, nbins, h->s) != hipSuccess ||
             hipMalloc(&p->scan_tmp, bytes + 256) != hipSuccess)
             return set_err(h, MGS_E_NOMEM, "deposit tile arrays");
@@ -769,7 +789,7 @@ int mgs_cic_deposit(mgs_handle* h)
     if (hipcub::DeviceScan::ExclusiveSum(p->scan_tmp, p->scan_bytes, p->count, p->first, p->nbins, h->s) !=
         hipSuccess)
         return set_err(h, MGS_E_HIP, "deposit scan");
-    hipLaunchKernelGGL(k_bin_scatter, dim3(gbin), dim3(PM_BLOCK), 0, h->s, nwaves, p->recs, p->nrec, p->first,
+    hipLaunchKernelGGL(k_bin_scatter, dim3(gbin), dim3(PM_BLOCK), PM_SCATTER_LDS, h->s, nwaves, p->recs, p->nrec, p->first,
                        p->order);
     const double wpar = wpar_of(N, np);
     const unsigned gt = ((unsigned)ntiles + 7) / 8 * 8;  // map_block
