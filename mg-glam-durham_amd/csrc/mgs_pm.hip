@@ -741,7 +741,7 @@ static int pm_ensure_bins(mgs_handle* h, PmState* p, int nbins)
         const size_t waves = ((size_t)p->np + PM_WCHUNK - 1) / PM_WCHUNK;
         if (hipMalloc((void**)&p->recs, waves * PM_WCHUNK * sizeof(unsigned long long)) != hipSuccess ||
             hipMalloc((void**)&p->nrec, waves * sizeof(int)) != hipSuccess ||
-            hipMalloc((void**)&p->order, (size_t)p->np * sizeof(int64_t)) != hipSuccess)
+            hipMalloc((void**)&p->order, (size_t)p->np * sizeof(unsigned)) != hipSuccess)
             return set_err(h, MGS_E_NOMEM, "deposit binning arrays");
         p->nbin = p->np;
     }

@@ -1,0 +1,30 @@
+"""Device memory that calls take beside their inputs."""
+import numpy as np
+import pytest
+
+import mgsolve as M
+
+MIB = 1 << 20
+
+
+# per particle a record of 8 bytes and an index of 4, and a word per 512
+# particles; allocations are rounded up, to 2 MiB at most
+@pytest.mark.gpu
+def test_deposit_takes_twelve_bytes_a_particle():
+    import torch
+
+    N, n = 32, 1 << 24
+    rng = np.random.default_rng(5)
+    pos = [rng.uniform(1.0, N + 0.99, n).astype(np.float32) for _ in range(3)]
+    with M.Solver(M.Config(N=N, model=M.MODEL_FR, fr_n=1, box=2.0 * N, fr0=-1e-5, precision=M.PREC_FP64)) as S:
+        S.set_particles(*[a[:1000] for a in pos])
+        S.cic_deposit()  # loads the kernels and makes the per-tile arrays
+        S.set_particles(*pos)
+        print(f"[memory] deposit of {n} particles", flush=True)
+        before = torch.cuda.mem_get_info()[0]
+        S.cic_deposit()
+        taken = before - torch.cuda.mem_get_info()[0]
+        mean = S.get_density(np.float64).mean()
+    assert taken <= 12 * n + 4 * n // 512 + 3 * 2 * MIB, taken / MIB
+    # eight weights a particle, each rounded to a multiple of 2^-40
+    assert abs(mean) <= 8 * n / N ** 3 * 2.0 ** -41 + 1e-12
