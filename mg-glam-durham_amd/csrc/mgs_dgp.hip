@@ -327,10 +327,16 @@ int dgp_alloc(mgs_handle* h)
     h->dgp_tmp = (double*)q;
     // FP64 passes: the second array of the level-0 field's ping-pong (not out of
     // the fixed scratch of mgs_solve_noalloc, whose largest grids it would not
-    // fit beside: level 0 is then copied back)
-    if (h->p.precision == MGS_PREC_FP64 && (dgp_zmarch(h->p.ngrid) || !h->use_arena)) {
+    // fit beside).  Grids without z-marching passes do without it where it does
+    // not fit: each pass of level 0 is then copied back.
+    const bool zmarch = dgp_zmarch(h->p.ngrid);
+    if (h->p.precision == MGS_PREC_FP64 && (zmarch || !h->use_arena)) {
         rc = dev_alloc(h, 2 * half * sizeof(double) + 256, &q, "DGP second array");
-        if (rc) return rc;
+        if (rc && zmarch) return rc;
+        if (rc) {
+            (void)hipGetLastError();  // the refused allocation's
+            h->err.clear();
+        }
         h->dgp_spare64 = (double*)q;
     }
     return 0;
