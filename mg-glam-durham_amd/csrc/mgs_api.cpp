@@ -218,7 +218,9 @@ static int alloc_hierarchy(mgs_handle* h)
     if (h->use_arena) {
         h->hsum = h->hsum_host;
     } else {
-        HIPCHK(h, hipHostMalloc((void**)&h->hsum, 16 * sizeof(double), hipHostMallocDefault));
+        // (coherent: kernels write it and the host reads it after an event, see sum_to_host)
+        HIPCHK(h, hipHostMalloc((void**)&h->hsum, 16 * sizeof(double),
+                                hipHostMallocMapped | hipHostMallocCoherent));
         HIPCHK(h, hipEventCreateWithFlags(&h->ev_norm, hipEventDisableTiming));
     }
     return 0;
@@ -333,9 +335,10 @@ static void op_smooth2(mgs_handle* h, int l)
 }
 
 // count partials summed (launch_sum_partials' order) into hsum[0].  hsum is
-// pinned memory that the device addresses, so the sum's own kernel writes it:
-// a copy behind it would be one more launch (3 us and its gap) in each
-// residual of a small grid.  In arena mode hsum is ordinary host memory.
+// pinned, coherent memory that the device addresses, so the sum's own kernel
+// writes it, and the host sees the value once it has waited for the stream or
+// for an event recorded behind the sum.  A copy would be one more launch (3 us
+// and its gap) in each residual of a small grid.  In arena mode hsum is ordinary host memory.
 int sum_to_host(mgs_handle* h, const double* partials, int count)
 {
     if (!h->use_arena) {
