@@ -150,18 +150,24 @@ inline DgpF dgpf(const DgpCoef& c)
 // steps that general ones carry for results or operands near the ends of the
 // FP32 range.
 
-// x / c.six, correctly rounded: two corrections by the exact remainder with the
-// correctly rounded reciprocal (the first leaves q within an ulp, where the
-// second is exact rounding).  Within a rounding of a denormal where |x| < 2^-100.
-__device__ __forceinline__ float over_six(float x, const DgpF& c)
+// x / c.six, correctly rounded where |x| >= 2^-100: two corrections by the exact
+// remainder with the correctly rounded reciprocal (the first leaves q within an
+// ulp, where the second is exact rounding); below, where the remainder itself is
+// rounded, within 2^-149 / c.six of that.  An infinity, a NaN
+// and an overflow of the first product (for c.six < 1, where the quotient
+// overflows too, but for its last place) pass through, as in a division.
+__host__ __device__ __forceinline__ float over_six(float x, const DgpF& c)
 {
-    float q = x * c.rsix;
+    const float p = x * c.rsix;
+    float q = fmaf(fmaf(-p, c.six, x), c.rsix, p);
     q = fmaf(fmaf(-q, c.six, x), c.rsix, q);
-    return fmaf(fmaf(-q, c.six, x), c.rsix, q);
+    return fabsf(p) <= __FLT_MAX__ ? q : p;
 }
 
-// sqrt(x), x >= 0, correctly rounded for x >= 2^-100 (below, to an ulp): the
-// hardware's root is within an ulp, the neighbours' remainders pick the right one
+// sqrt(x), x >= 0, correctly rounded for x >= 2^-100 and infinite x (below, to an
+// ulp; dgp_dop's operands are 0 or at least 2^-25 alpha^2): the hardware's root
+// is within an ulp, and the signs of the fused remainders x - lo s and x - hi s
+// with its two neighbours lo and hi, the usual correction, pick the right one
 __device__ __forceinline__ float sqrt_pos(float x)
 {
     const float s = __builtin_amdgcn_sqrtf(x);

@@ -14,8 +14,16 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCE = r"""
 #include <math.h>
+#include "mgs_dgp_dev.h"
 #include "mgs_fr_dev.h"
 using namespace mgs;
+extern "C" void sixths(const float* x, float* q, int n, int level)
+{
+    DgpCoef c{};
+    c.dx2 = (double)(1 << level) * (double)(1 << level);
+    const DgpF f = dgpf(c);
+    for (int i = 0; i < n; i++) q[i] = over_six(x[i], f);
+}
 extern "C" double newton(int n, double d, double S, double xb, double r, double A, double C)
 {
     DfCoef c{};
@@ -38,6 +46,8 @@ def cells(tmp_path_factory):
                         "-shared", "-I", CSRC, src, "-o", lib], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
     L = C.CDLL(lib)
+    L.sixths.restype = None
+    L.sixths.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int]
     L.newton.restype = C.c_double
     L.newton.argtypes = [C.c_int] + [C.c_double] * 6
     return L
@@ -85,3 +95,29 @@ def test_coarsest_newton_solves_screened_cells(cells, n, A):
         noise = (16 * 2.0 ** -53 * (abs(A) * (S + 6.0 * abs(d)) + local + abs(r)) + 8.8e-14 * local) / slope
         tol = 1e-11 * min(abs(float(ds)), float(ws)) + noise + 2.0 ** -52
         assert abs(float(got - ds)) <= tol, (w, w0, float(got - ds), tol)
+
+
+# the inner nDGP smoother's quotient by 6 / dx^2, dx = 2^level, over the whole
+# FP32 range: a division's results, infinities and NaN among them
+@pytest.mark.parametrize("level", range(10))
+def test_ndgp_quotient_is_a_division(cells, level):
+    rng = np.random.default_rng(level)
+    x = rng.integers(0, 1 << 32, 1 << 20, dtype=np.uint64).astype(np.uint32).view(np.float32)
+    x = np.concatenate([x, np.float32([0.0, -0.0, np.inf, -np.inf, np.nan, 3.4028235e38, -3.4028235e38, 1e38, 1e-45])])
+    got = np.empty_like(x)
+    cells.sixths(x.ctypes.data, got.ctypes.data, x.size, level)
+    six = np.float32(6.0) * np.float32(4.0 ** -level)
+    with np.errstate(all="ignore"):
+        ref = x / six
+        wide = x.astype(np.float64) / np.float64(six)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    # an overflow of the quotient rounds up or down in its last place
+    top = (np.abs(wide) < 2.0 ** 128 * (1 - 2.0 ** -22)) | np.isinf(x)
+    big = (np.abs(x) >= 2.0 ** -100) & top
+    assert np.array_equal(got[big], ref[big])
+    tiny = np.abs(x) < 2.0 ** -100
+    # the last rounding, and the remainder's, half the smallest denormal, over six
+    half = 0.5 * np.spacing(np.abs(ref[tiny])).astype(np.float64)
+    assert np.all(np.abs(got[tiny] - wide[tiny]) <= half + 2.0 ** -149 / np.float64(six))
+    edge = ~np.isnan(x) & ~top
+    assert np.all(np.isinf(got[edge]) | (np.abs(got[edge]) >= np.float32(3.4028e38)))
