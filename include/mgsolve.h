@@ -257,6 +257,10 @@ int mgs_synchronize(mgs_handle* h);
 /* launch the coarse levels of each V-cycle from a captured hipGraph (default
  * 1) or as individual kernels (0); results are identical either way */
 int mgs_use_graphs(mgs_handle* h, int32_t enable);
+/* run the small levels of each V-cycle (64^3 cells and below) in one launch per
+ * cycle or half cycle (default 1) or in one launch per operation (0); results
+ * are identical either way */
+int mgs_use_fused_levels(mgs_handle* h, int32_t enable);
 /* device pointer of the level-0 field in the internal colour-split layout
  * (for zero-copy consumers on the same device) */
 int mgs_device_field(mgs_handle* h, void** ptr, size_t* bytes);

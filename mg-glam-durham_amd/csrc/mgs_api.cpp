@@ -513,7 +513,7 @@ void drop_graphs(mgs_handle* h)
 // residual and field; the small levels in one launch
 static int vcycle_plain_from_restricted(mgs_handle* h, int l)
 {
-    if (l < h->lc && h->L[l].n <= h->tail_n && h->use_tail) {
+    if (l < h->lc && h->L[l].n <= h->tail_n && h->fuse_levels) {
         prof_begin(h, MGS_KC_COARSE, 16.0 * n3d(h->L[l].n) * 8.0);
         const bool ok = launch_plain_tail(h, l);
         prof_end(h);
@@ -598,7 +598,7 @@ static int cycle_from_restricted(mgs_handle* h, int l, const float** dH)
     LevelF& v = h->M[l];
     const DfCoef dc = df_coefs(h->p, l);
     *dH = v.d;
-    if (l < h->lc && v.n <= h->tail_n && h->use_tail) {
+    if (l < h->lc && v.n <= h->tail_n && h->fuse_levels) {
         TailLevelIn lv[16];
         const int nlev = h->lc - l + 1;
         for (int i = 0; i < nlev && i < 16; i++) {
@@ -610,7 +610,7 @@ static int cycle_from_restricted(mgs_handle* h, int l, const float** dH)
         prof_end(h);
         if (ok) return 0;
     }
-    if (l < h->lc && df_block_level(v.n) && h->sweeps1[0] == 2 && h->sweeps1[1] == 2) {
+    if (l < h->lc && df_block_level(v.n) && h->fuse_levels && h->sweeps1[0] == 2 && h->sweeps1[1] == 2) {
         LevelF& c = h->M[l + 1];
         prof_begin(h, MGS_KC_COARSE, (5.0 * n3d(v.n) + 3.0 * n3d(c.n)) * 4.0);
         launch_df_block_down(frn, v.rd, v.rres, v.xb, v.d, v.f, c.rres, c.rd, c.d, v.n, dc, h->s);
@@ -821,7 +821,7 @@ static int vcycle_inner_dgp(mgs_handle* h, int l, bool first = false);
 static int dgpm_from_restricted(mgs_handle* h, int l)
 {
     LevelF& c = h->M[l];
-    if (l < h->lc && c.n <= h->tail_n && h->use_tail) {
+    if (l < h->lc && c.n <= h->tail_n && h->fuse_levels) {
         prof_begin(h, MGS_KC_COARSE, 20.0 * n3d(c.n) * 4.0);
         const bool ok = launch_dgpm_tail(h, l);
         prof_end(h);
@@ -1110,8 +1110,6 @@ int init_handle(mgs_handle* h, const mgs_params* params, bool use_arena, unsigne
     // inner cycle's shape; the shipped library's numerics depend on no
     // environment variable
     if (!use_arena) {
-        const char* e = std::getenv("MGS_NO_TAIL");
-        h->use_tail = !(e && e[0] == '1');
         const char* tn = std::getenv("MGS_TAIL_N");
         const int tv = tn ? std::atoi(tn) : 0;
         if (tv == 8 || tv == 16 || tv == 32) h->tail_n = tv;
@@ -1611,6 +1609,15 @@ int mgs_use_graphs(mgs_handle* h, int32_t enable)
     HIPCHK(h, hipStreamSynchronize(h->s));
     drop_graphs(h);
     h->use_graphs = enable != 0;
+    return 0;
+}
+
+int mgs_use_fused_levels(mgs_handle* h, int32_t enable)
+{
+    if (!h) return MGS_E_ARG;
+    HIPCHK(h, hipStreamSynchronize(h->s));
+    drop_graphs(h);
+    h->fuse_levels = enable != 0;
     return 0;
 }
 

@@ -110,9 +110,9 @@ struct mgs_handle {
     // the host waits for the norm while the base restriction runs
     hipEvent_t ev_norm = nullptr;
     bool use_graphs = true;
-    // mixed f(R): small inner levels in one launch; tuning builds
-    // (-DMGS_TUNING) read MGS_NO_TAIL=1 to turn it off
-    bool use_tail = true;
+    // the small levels of a cycle in one launch (the tails) or one per half
+    // cycle (mixed f(R)'s blocks), not one per operation: mgs_use_fused_levels
+    bool fuse_levels = true;
     int tail_n = 16;  // the tail starts at the first level with n <= tail_n (tuning builds: MGS_TAIL_N 8, 16 or 32)
     // mixed f(R): level-0 pre/post sweeps of the inner cycle and the
     // automatic inner-cycle cap (tuning builds: MGS_INNER_SWEEPS "a,b" and

@@ -154,6 +154,7 @@ def load():
         "mgs_profile_get": ([H, i32, C.POINTER(C.c_int64), C.POINTER(C.c_double), C.POINTER(C.c_double)], C.c_int),
         "mgs_synchronize": ([H], C.c_int),
         "mgs_use_graphs": ([H, i32], C.c_int),
+        "mgs_use_fused_levels": ([H, i32], C.c_int),
         "mgs_device_field": ([H, C.POINTER(C.c_void_p), C.POINTER(C.c_size_t)], C.c_int),
         "mgs_server_create": ([C.POINTER(ServerOpts), C.POINTER(H)], C.c_int),
         "mgs_server_destroy": ([H], C.c_int),
@@ -425,6 +426,10 @@ class Solver:
 
     def use_graphs(self, enable=True):
         self._chk(self.L.mgs_use_graphs(self.h, int(bool(enable))), "mgs_use_graphs")
+
+    def use_fused_levels(self, enable=True):
+        """Small levels in one launch per cycle or half cycle, or one per operation (same results)."""
+        self._chk(self.L.mgs_use_fused_levels(self.h, int(bool(enable))), "mgs_use_fused_levels")
 
 
 def exported_symbols_declared_in_header(header_path):

@@ -1,6 +1,7 @@
-"""The one-launch forms of the small inner levels (the tail, the half-cycle
-blocks) against the server's operation-by-operation launches of the same
-cycle, bit for bit, on grids whose coarse levels meet their edges."""
+"""The small levels of a cycle on grids that meet the edges of their one-launch
+forms: the mixed solves against the server's, bit for bit (whose f(R) levels
+above 16^3 run one launch per operation, and whose smaller ones are the same
+tails), and the FP64 cycles against the oracle."""
 import numpy as np
 import pytest
 
