@@ -264,47 +264,6 @@ __device__ __forceinline__ double dgpm_outer_cell(const double* __restrict__ u, 
     return OP * OP;
 }
 
-// e_h += P(e_H - R e_h) for the 8 children of coarse cell (I, J, K) (no
-// guard for DGP)
-__device__ __forceinline__ void dgpm_correct_cell(const float* __restrict__ eH, const float* __restrict__ rd,
-                                                  float* __restrict__ ef, const Geo& gf, const Geo& gc, int I, int J,
-                                                  int K)
-{
-    const int nc = gc.n;
-    const float a = 1.0f / 64.0f, b = 3.0f * a, c9 = 9.0f * a, dd = 27.0f * a;
-    const float wt[8] = {a, b, b, c9, b, c9, c9, dd};
-    const int Xs[3] = {wrap_dec(I, nc), I, wrap_inc(I, nc)};
-    const int Ys[3] = {wrap_dec(J, nc), J, wrap_inc(J, nc)};
-    const int Zs[3] = {wrap_dec(K, nc), K, wrap_inc(K, nc)};
-    float ev[27];
-#pragma unroll
-    for (int z = 0; z < 3; z++)
-#pragma unroll
-        for (int y = 0; y < 3; y++)
-#pragma unroll
-            for (int x = 0; x < 3; x++) {
-                const size_t q = split_index(gc, Xs[x], Ys[y], Zs[z]);
-                ev[x + 3 * y + 9 * z] = eH[q] - rd[q];
-            }
-    float old[8];
-#pragma unroll
-    for (int sind = 0; sind < 8; sind++)
-        old[sind] = ef[split_index(gf, 2 * I + (sind & 1), 2 * J + ((sind >> 1) & 1), 2 * K + (sind >> 2))];
-#pragma unroll
-    for (int sind = 0; sind < 8; sind++) {
-        const int s1 = sind & 1, s2 = (sind >> 1) & 1, s3 = sind >> 2;
-        float P = 0.0f;
-#pragma unroll
-        for (int ind = 0; ind < 8; ind++) {
-            const int x = (ind & 1) ? 1 : (s1 ? 2 : 0);
-            const int y = (ind & 2) ? 1 : (s2 ? 2 : 0);
-            const int z = (ind & 4) ? 1 : (s3 ? 2 : 0);
-            P += wt[ind] * ev[x + 3 * y + 9 * z];
-        }
-        ef[split_index(gf, 2 * I + s1, 2 * J + s2, 2 * K + s3)] = old[sind] + P;
-    }
-}
-
 // coarsest level: sweeps of the inner smoother by one workgroup, the update
 // evaluated in FP64 (the level holds at most a few thousand cells)
 __device__ __forceinline__ void dgpm_coarsest_block(float* __restrict__ e, const float* __restrict__ pb,
@@ -821,11 +780,11 @@ __device__ __forceinline__ void dgpm_zsmooth_run(const float* __restrict__ e0, c
     }
 }
 
-// The same correction z-marching over coarse columns, as k_df_correct: planes
-// of e = e_H - R e_h in registers (x-neighbours from the adjacent lanes), all
-// 8 sons of a coarse cell, software-pipelined (plane K's sons computed, the
-// loads of plane K+1 issued, then plane K's sons stored).  Sums in
-// dgpm_correct_cell's order.
+// e_h += P(e_H - R e_h) (no guard for DGP), z-marching over coarse columns, as
+// k_df_correct: planes of e = e_H - R e_h in registers (x-neighbours from the
+// adjacent lanes), all 8 sons of a coarse cell, software-pipelined (plane K's
+// sons computed, the loads of plane K+1 issued, then plane K's sons stored).
+// A son's sum runs over its 8 contributors with x fastest, the coarse cell last.
 template <int S3, bool NT>
 __device__ __forceinline__ void dgpm_sons_load(const float* __restrict__ ef, const Geo& gf, int I, int J, int K,
                                                float* old)

@@ -301,7 +301,7 @@ __device__ void ptail_cycle(const PTailDesc<MD>& G, int i0, typename MD::T* lds)
         const PTailLevel<MD>&L = G.L[i], &C = G.L[i + 1];
         const PTailArrays<MD> l = ptail_level(G, i, lds), c = ptail_level(G, i + 1, lds);
         // u += P (u_H - R u), a thread per fine cell; weights and order of
-        // correct64_sons_apply / dgpm_correct_cell
+        // correct64_sons_apply / dgpm_sons_new
         for (int t = tid; t < 2 * (int)L.g.half; t += nthr) {
             int x, y, z;
             coarse_ijk(L.g, t, x, y, z);
