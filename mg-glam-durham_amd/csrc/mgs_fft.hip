@@ -227,8 +227,8 @@ __global__ __launch_bounds__(256) void k_lognormal(const double* __restrict__ g,
 // registers: every access is a unit-stride run (the pairs of the rows beside
 // it lie at the same m), and the outputs are written once, past the caches.
 // A stream of 8 bytes in and 16 out per cell; 256^3, all four outputs in
-// REAL*4: 115 us = 3.5 TB/s (one thread per cell with 64-bit divisions 187,
-// pairs without the march 139, with cached stores 156).
+// REAL*4: 97 us = 4.1 TB/s (one thread per cell with 64-bit divisions 187; when
+// the march took 115, pairs without it 139, with cached stores 156).
 template <typename T>
 __global__ __launch_bounds__(256) void k_fifth_force(const double* __restrict__ u, T* __restrict__ psi,
                                                      T* __restrict__ gx, T* __restrict__ gy, T* __restrict__ gz, Geo g,

@@ -1026,7 +1026,8 @@ __device__ __forceinline__ void restrict8_cell(const T* __restrict__ fine, T* __
 // a colour run in the first wave without barriers; index divisions by the
 // level's side, which made up most of the chain on the small levels, are
 // shifts (half_mjk).  From 16^3: 57 us and a launch of 3.9 for f before, now 41
-// for both, of which two thirds on the 16^3 level and 5 us on the coarsest.
+// for both in a 64^3 solve (45 at 128^3, 55 at 512^3, between longer launches), of
+// which two thirds on the 16^3 level and 5 us on the coarsest.
 // ---------------------------------------------------------------------------
 struct TailLevel {
     Geo g;

@@ -164,7 +164,8 @@ __device__ __forceinline__ unsigned long long run_record(unsigned rank, int bin,
 // 2.13 ms for 512^3 particles in lattice order, now 0.49 ms (1.6 GB of
 // positions read, 0.4 GB of records written).  A run whose bin finds no slot
 // within PM_PROBES (blocks of unordered particles) takes the global atomic
-// itself.
+// itself: 2.6 ms for 400^3 shuffled particles, as with one atomic per run (4.0
+// without the table, whose bins' atomics are issued together).
 constexpr int PM_SLOTS = 1024, PM_PROBES = 8;
 
 __global__ __launch_bounds__(PM_BLOCK) void k_bin_count(const float* __restrict__ xs, const float* __restrict__ ys,
@@ -380,10 +381,11 @@ __device__ __forceinline__ void pm_add8(unsigned long long* acc, int b, double D
 //
 // 512^3 cells, 512^3 particles (lattice displaced by 2 cells rms): this kernel
 // 1.35 ms (2.75 with a thread per run and position), the whole deposit with
-// its reading back 6.5 -> 2.85 ms.  Before, 16^3-cell tiles added into the
+// its reading back 6.5 -> 2.7 ms.  Before, 16^3-cell tiles added into the
 // grid in eight launches by parity class (2.65 ms) between a clearing and a
 // conversion pass (0.55 ms).  What is left is the gather of
-// positions in bin order and the LDS additions.
+// positions in bin order and the LDS additions; for shuffled particles the
+// gather alone (400^3: 4.4 ms, as before).
 constexpr int PM_SEGS = 21;  // own inner bin; own bins 1..7; 4 + 4 + 2 + 4 + 2 + 2 + 1 bins of the others
 constexpr int PM_DBLOCK = 512;
 

@@ -7,9 +7,10 @@
 // all participating requests (a prefix sum of their tile counts in a device
 // plan), so one launch smooths, restricts or corrects the same level of every
 // request at once, whatever their grid sizes and parameters.  The sequence
-// depends only on the deepest f(R) and nDGP hierarchies in the batch, so it
-// is captured once per pair of depths as a hipGraph and replayed; requests joining or leaving only
-// change the plan in device memory.
+// depends only on the deepest f(R) and nDGP hierarchies in the batch and on the
+// deepest levels from which one workgroup finishes a cycle (struct Depths), so
+// it is captured once per such four depths as a hipGraph and replayed; requests
+// joining or leaving only change the plan in device memory.
 //
 // Per request the arithmetic, the tiling and the reduction order are those of
 // the single-request solve (mgs_api.cpp, solve_mixed with one inner cycle),
@@ -215,9 +216,9 @@ __device__ __forceinline__ bool tile_xy(int width, unsigned rows, const Shape& z
     return x < width && row < rows;
 }
 
-// FP64 outer residual (and the inner problem's g, xb, d: f(R) after its
-// first colour-0 pass, nDGP d = 0) on level 0; one block partial per tile, as
-// k_both_colours / k_dgpm_outer
+// FP64 outer residual (and the inner problem's g, xb, d, after its first
+// colour-0 pass) on level 0; one block partial per tile, as k_both_colours /
+// k_dgpm_outer
 __global__ __launch_bounds__(256) void kb_outer_residual(const SlotDesc* __restrict__ S, const Plan* __restrict__ P)
 {
     const unsigned total = P->res_pre[P->nres];
