@@ -312,7 +312,7 @@ __device__ __forceinline__ void dgpm_coarsest_block(float* __restrict__ e, const
 // spills scalar registers into vector lanes.  Instructions per cell: FP32 pass
 // 239 -> 177, FP32 residual 238 -> 160, FP64 residual 162 -> 111.  At 512^3, by
 // where the arrays lie in memory (each process keeps its times): FP32 pass
-// 456-484 -> 399-445 us, in one process of twelve 524; FP32 residual 718-850 ->
+// 456-484 -> 399-445 us, in one process 524; FP32 residual 718-850 ->
 // 669-705, FP64 outer residual 880-921 -> 730-745 (5.1 TB/s), FP64 pass 632 ->
 // 460.  Side values of
 // the FP32 pass by vector loads: 467 where scalar ones take 444; of the FP32
