@@ -58,12 +58,16 @@ def test_other_cycles(model, cycle):
           _solve(mode=1, rel_tol=1e-6, max_cycles=3, cycle=cycle))
 
 
+# (the levels' arrays too, which a caller can read)
 @pytest.mark.gpu
 @pytest.mark.parametrize("model,n", [(M.MODEL_FR, 0), (M.MODEL_FR, 1), (M.MODEL_FR, 2), (M.MODEL_DGP, 1)])
-def test_fp64(model, n):
+@pytest.mark.parametrize("N", [32, 48])
+def test_fp64(N, model, n):
     def run(S):
         S.initialise()
         S.vcycle(0)
+        levels = [S.get_level(l, a).tobytes() for l in range(1, S.levels()[2] + 1)
+                  for a in (M.ARR_U, M.ARR_F, M.ARR_RES, M.ARR_RRES, M.ARR_RU, M.ARR_RHO)]
         S.fcycle(0)
-        return S.residual(0)
-    _both(M.Config(N=48, model=model, fr_n=n, branch=1, box=96.0, fr0=-1e-5), run)
+        return levels, S.residual(0)
+    _both(M.Config(N=N, model=model, fr_n=n, branch=1, box=2.0 * N, fr0=-1e-5), run)
